@@ -31,9 +31,9 @@ IP = C.POINTER(C.c_int)
 
 
 def build(ref: bool = True) -> None:
-    """Compile liboracle.so (and _ref/ref_harness when the reference tree exists)."""
+    """Compile liboracle.so (and _ref/ref_harness when the reference's sources are there)."""
     targets = ["all"]
-    if ref and os.path.isdir(REF_TREE):
+    if ref and os.path.exists(os.path.join(REF_TREE, "bounds", "src", "bound_abstract.cpp")):
         targets.append("ref")
     subprocess.run(["make", "-s", "-C", HERE] + targets, check=True)
 
