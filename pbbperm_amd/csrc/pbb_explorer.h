@@ -18,11 +18,6 @@ namespace pbb {
 // of explorers in one workgroup (whose release/acquire then need no L2
 // writeback or invalidate).
 template <int S = __HIP_MEMORY_SCOPE_AGENT>
-__device__ __forceinline__ int ld_acq(const int *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_ACQUIRE, S);
-}
-template <int S = __HIP_MEMORY_SCOPE_AGENT>
 __device__ __forceinline__ int ld_rlx(const int *p)
 {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, S);
@@ -48,13 +43,6 @@ __device__ __forceinline__ void st_rlx(int *p, int v)
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, S);
 }
 
-template <int S>
-__device__ __forceinline__ void fence_acq()
-{
-    if constexpr (S == __HIP_MEMORY_SCOPE_WORKGROUP) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    else __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-}
-
 // lane-0 read-modify-writes, result broadcast to the wavefront
 template <int S = __HIP_MEMORY_SCOPE_AGENT>
 __device__ __forceinline__ int w_add(int *p, int v)
@@ -64,27 +52,8 @@ __device__ __forceinline__ int w_add(int *p, int v)
     return rdlane(r, 0);
 }
 // Relaxed counters: on this multi-XCD device an agent-scope release writes
-// back the wave's L2 and an acquire invalidates it, so the idle-ring tickets
-// and the work counter, whose values carry no other data, take no fence.
-template <int S = __HIP_MEMORY_SCOPE_AGENT>
-__device__ __forceinline__ int w_add_rlx(int *p, int v)
-{
-    int r = 0;
-    if (lane_id() == 0) r = __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, S);
-    return rdlane(r, 0);
-}
-template <int S = __HIP_MEMORY_SCOPE_AGENT>
-__device__ __forceinline__ unsigned w_addu_rlx(unsigned *p, unsigned v)
-{
-    unsigned r = 0;
-    if (lane_id() == 0) r = __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, S);
-    return (unsigned)rdlane((int)r, 0);
-}
-template <int S = __HIP_MEMORY_SCOPE_AGENT>
-__device__ __forceinline__ unsigned long long ld_rlx64(const unsigned long long *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, S);
-}
+// back the wave's L2 and an acquire invalidates it, so the idle mask and the
+// work counter, whose values carry no other data, take no fence.
 template <int S = __HIP_MEMORY_SCOPE_AGENT>
 __device__ __forceinline__ void st_rlx64(unsigned long long *p, unsigned long long v)
 {
@@ -106,19 +75,6 @@ __device__ __forceinline__ bool w_cas(unsigned *p, unsigned expect, unsigned des
     if (lane_id() == 0) {
         unsigned e = expect;
         ok = __hip_atomic_compare_exchange_strong(p, &e, desired, __ATOMIC_ACQ_REL, __ATOMIC_RELAXED,
-                                                  S);
-    }
-    return rdlane(ok, 0) != 0;
-}
-// Relaxed claim: no agent-scope release/acquire, so a failed attempt costs
-// one atomic round trip and no L2 writeback or invalidate.
-template <int S = __HIP_MEMORY_SCOPE_AGENT>
-__device__ __forceinline__ bool w_cas_rlx(unsigned *p, unsigned expect, unsigned desired)
-{
-    int ok = 0;
-    if (lane_id() == 0) {
-        unsigned e = expect;
-        ok = __hip_atomic_compare_exchange_strong(p, &e, desired, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                   S);
     }
     return rdlane(ok, 0) != 0;
@@ -285,8 +241,10 @@ __device__ __forceinline__ InstRef engine_inst(const KArgs &a)
 {
     InstRef r;
     r.ctl = a.ctl;
-    r.ring = a.ring;
-    r.ring_cap = a.ring_cap;
+    r.idle = a.idle;
+    r.idle_words = a.idle_words;
+    r.member = nullptr;
+    r.occ = nullptr;
     r.ub0 = a.initial_ub;
     r.best = a.best;
     r.root_row = a.root_row;
@@ -324,6 +282,10 @@ struct Explorer {
     int pinfo[PCH];                   // this lane's Johnson machine pairs (REF 2)
     int local_best;
     unsigned dec, leaves, sb, jb;     // deltas since the last flush
+    unsigned mtag;                    // lane i: tag of word i of the last message consumed
+    int self;                         // this explorer's member index (bit self / words of word self % words)
+    int pollw;                        // next idle word to poll
+    int seen;                         // pool: the slot's member word as of the last poll
     unsigned nchk;                    // periodic checks so far (host-word phase)
     unsigned since;                   // nodes decomposed in this launch's own interval (ramp)
     bool end_dirty;                   // end moved since pos was last compared with it
@@ -342,6 +304,9 @@ struct Explorer {
         if constexpr (REF == 2) pair_lanes<PCH>(r.pair_ab, r.npairs, r.m, r.pairs_mode, pinfo);
         dec = leaves = sb = jb = 0;
         since = 0;
+        mtag = 0;
+        self = eid;
+        pollw = seen = 0;
         nchk = (unsigned)eid;  // staggers the host-word reads across explorers
         end_dirty = true;
         hist = jhist = 0;
@@ -930,7 +895,7 @@ struct Explorer {
         endv = lane < n ? (int)a.end[(size_t)e * 64 + lane] : 0;
         dirv = lane < n ? (int)a.dir[(size_t)e * 64 + lane] : 0;
         end_dirty = true;
-        since = a.ramp;  // a resumed or donated interval is shared at once
+        since = a.ramp;  // a resumed interval is shared at once
         __builtin_amdgcn_wave_barrier();
         rebuild_stacks();
     }
@@ -946,8 +911,85 @@ struct Explorer {
             a.end[(size_t)e * 64 + lane] = (int8_t)endv;
             a.dir[(size_t)e * 64 + lane] = (int8_t)dirv;
         }
-        if (lane == 0) a.line[e] = L;
-        if (lane == 0) st_rlx<SC>(a.state + e, st);
+        if (lane == 0) {
+            a.line[e] = L;
+            a.state[e] = st;
+            a.mtag[e] = mtag;
+        }
+    }
+
+    // an idle explorer leaves the launch
+    __device__ __forceinline__ void leave_idle()
+    {
+        if (lane == 0) {
+            a.state[e] = ST_IDLE;
+            a.mtag[e] = mtag;
+        }
+    }
+
+    // ------------------------------------------------------------ mailbox
+    // An interval is handed over as one message: 64 words of 64 bits, one per
+    // lane, written by one store instruction.  The low half of every word
+    // carries the message's tag (the previous one's plus 1, mod 64), so a
+    // thief that sees the new tag in all 64 words holds the whole message
+    // and neither side takes a fence: at agent scope a release writes back
+    // the XCD's L2 and an acquire invalidates it.  The high halves carry
+    // the front entry (lanes 0-19), the back entry (20-39) of the split
+    // line, so the thief replays no push.  Reading the former rows, interval
+    // vectors and line back from HBM and replaying the path took 18 us per
+    // hand-over (50x20, 98 k hand-overs).
+    static_assert(M <= 20, "the high halves of a message hold two vectors of 20 machines");
+
+    __device__ __forceinline__ unsigned long long *my_mail() const { return a.mbox + (size_t)e * 64 + lane; }
+    // the last message of this mailbox is consumed (or none was ever sent)
+    __device__ __forceinline__ void open_mail() { mtag = mail_tag((unsigned)ld_rlx<SC>(my_mail())); }
+    __device__ __forceinline__ unsigned long long peek_mail() const { return ld_rlx<SC>(my_mail()); }
+    __device__ __forceinline__ bool mail_here(unsigned long long w) const
+    {
+        return ballot(mail_tag((unsigned)w) == ((mtag + 1u) & MAIL_TAGS)) == ~0ull;
+    }
+
+    __device__ __forceinline__ void take_mail(unsigned long long word)
+    {
+        const unsigned w = (unsigned)word;
+        const int hi = (int)(unsigned)(word >> 32);
+        mtag = mail_tag(w);
+        const int job = (int)mail_job(w);
+        L = __ffsll((unsigned long long)ballot(job == (int)MAIL_NONE)) - 1;
+        rowv = mail_cell(w);
+        posv = mail_pos(w);
+        endv = mail_end(w);
+        dirv = mail_dir(w);
+        nb = __popcll(lanes_below(L) & ballot(dirv != 0));
+        nf = L - nb;
+        ftop = lane < M ? hi : 0;
+        if (lane < M) frow(nf)[lane] = hi;
+        if (lane >= 20 && lane < 20 + M) brow(nb)[lane - 20] = hi;
+        remv = lane < M ? lds.tot[lane] : 0;
+        for (int r = 0; r < L; r++) {
+            const int j = rdlane(job, r);
+            *(lane < n - r ? lds.mat + lds_mat_row(r, n) + lane : (int8_t *)(lds.sink + lane)) =
+                (int8_t)mail_path_cell(lane, rdlane(posv, r), j);
+            remv -= pmach(j);
+        }
+        end_dirty = true;
+        since = a.ramp;  // a donated interval is shared at once
+        __builtin_amdgcn_wave_barrier();
+    }
+
+    // the donor's side: rows 0..l of its path, the split row, the interval
+    // [.., cut] .. endE and the stack entries of line l
+    __device__ __forceinline__ void send_mail(int thief, unsigned tag, int l, int rowl, int cut, int endE)
+    {
+        int job = 0;
+        if (lane < l) job = flag_abs((int)lds.mat[lds_mat_row(lane, n) + posv]);
+        const int nbl = __popcll(lanes_below(l) & ballot(dirv != 0));
+        const int qf = lane < M ? lane : M - 1, qb = lane < 20 ? 0 : (lane < 20 + M ? lane - 20 : M - 1);
+        const int hi = lane < 20 ? frow(l - nbl)[qf] : brow(nbl)[qb];
+        const unsigned lo = mail_word(lane < n - l ? rowl : 0, lane < l ? posv : (lane == l ? cut : 0),
+                                      lane < n ? endE : 0, lane < l ? (unsigned)job : MAIL_NONE,
+                                      lane <= l ? dirv : 0, tag);
+        st_rlx64<SC>(a.mbox + (size_t)thief * 64 + lane, ((unsigned long long)(unsigned)hi << 32) | lo);
     }
 
     // fresh interval: row 0 = bounded root row, pos/end from HBM
@@ -993,14 +1035,6 @@ struct Explorer {
         if (nap < 16) nap <<= 1;
     }
 
-    __device__ __forceinline__ void fail(int code)
-    {
-        if (lane == 0) {
-            st_rlx<SC>(&run->err, code);
-            st_rlx<SC>(&run->stop, 1);
-        }
-    }
-
     // bbthread::shareWork + ivm::cuttingPosition (bbthread.cpp:39-72,
     // ivm.cpp:188-237): split at the first line l whose pos differs from end
     // (l <= L, l < n - margin, the size_d - margin rule of
@@ -1015,13 +1049,14 @@ struct Explorer {
     // work on: a small tree then runs depth-first in one explorer, finding
     // the incumbents the reference's order finds, and a large one fans out
     // after that many nodes (woken and resumed explorers share at once).
-    // h, t: idle-ring head/tail loaded before the node's work (prefetch).
-    // Returns whether idle explorers were waiting (the ring was not empty).
-    __device__ __forceinline__ bool try_donate(unsigned h, unsigned t)
+    // idle: the mask word loaded before the node's work (peek_idle).  Returns
+    // whether idle explorers were waiting in it.
+    __device__ __forceinline__ bool try_donate(unsigned long long idle)
     {
-        h = (unsigned)uni((int)h);
-        t = (unsigned)uni((int)t);
-        if (h == t) return false;
+        idle = uni64(idle);
+        const int word = pollw;
+        next_word();
+        if (!idle) return false;
         const int lim = min(L, n - 1 - a.steal_margin);  // last line a split may use
         if (lim < 0) return true;                         // margin >= n: never split
         uint64_t ne = lanes_below(n) & ballot(posv != endv);
@@ -1047,38 +1082,35 @@ struct Explorer {
             else if (lane >= l && lane < n) endE = n - 1 - lane;
         }
         int nexp = __popcll(expl);
-        // Every busy explorer that saw the ring non-empty races for ticket h.
-        // The claim orders nothing (the donor has published nothing yet, and
-        // the acquire load of the cell's sequence below orders the read of
-        // the thief's id), so it is relaxed: with thousands of contenders an
-        // acq_rel attempt, i.e. an L2 writeback + invalidate per loser,
-        // dominated the ramp-up of every solve.
-        if (!w_cas_rlx<SC>(&ir.ctl->idle_head, h, h + 1)) return true;
-        // claim the idle explorer registered at ticket h (bounded MPMC ring
-        // cell: the ticket and the explorer id share one word, so reading
-        // the id needs no acquire)
-        const unsigned slot = h & (unsigned)(ir.ring_cap - 1);
-        bool ok = false;
-        unsigned long long cell = 0ull;
-        for (int spin = 0; spin < PBB_SPIN_LIMIT; spin++) {
-            cell = uni64(ld_rlx64<SC>(ir.ring + slot));
-            if ((unsigned)(cell >> 32) == h + 1u) {
-                ok = true;
-                break;
-            }
-            __builtin_amdgcn_s_sleep(1);
+        // Claim one explorer of the word by clearing its bit; each donor starts
+        // its choice at another bit.  Relaxed: the claim orders nothing, the
+        // donor has published nothing yet.
+        const int rot = e & 63;
+        const int bit = (__ffsll((idle >> rot) | (idle << (-rot & 63))) - 1 + rot) & 63;
+        const int idx = bit * ir.idle_words + word;
+        int got = 0, thief = idx;
+        if (lane == 0) {
+            const unsigned long long old =
+                __hip_atomic_fetch_and(ir.idle + (size_t)word * IDLE_STRIDE, ~(1ull << bit), __ATOMIC_RELAXED, SC);
+            if (ir.member) thief = ld_rlx<SC>(ir.member + idx);
+            got = (int)((old >> bit) & 1ull);
         }
-        if (!ok) {
-            fail(PBB_DEV_ERR_RING);
-            return true;
+        if (!rdlane(got, 0)) return true;
+        thief = rdlane(thief, 0);
+        // The thief is idle and this donor's alone now, so its mailbox holds the
+        // last message it consumed: the next one's tag follows from it.  The
+        // thief counts as holding an interval before its message is sent (the
+        // count's old value has come back: used below), so its own release
+        // comes later in the count's order.
+        unsigned tag = 0u;
+        int held = 0;
+        if (lane == 0) {
+            held = __hip_atomic_fetch_add(&ir.ctl->work_count, 1, __ATOMIC_RELAXED, SC);
+            tag = mail_tag((unsigned)ld_rlx<SC>(a.mbox + (size_t)thief * 64));
         }
-        const int thief = (int)(unsigned)cell - 1;
-        // the cell waits for the ticket of the next lap
-        if (lane == 0) st_rlx64<SC>(ir.ring + slot, (unsigned long long)(h + (unsigned)ir.ring_cap) << 32);
-        if (thief < 0 || thief >= a.E) {
-            fail(PBB_DEV_ERR_RING);
-            return true;
-        }
+        held = rdlane(held, 0);
+        tag = ((unsigned)rdlane((int)tag, 0) + 1u) & MAIL_TAGS;
+        asm volatile("" : : "s"(held) : "memory");
         int keep = nexp / 2;
         int cut;
         if (keep == 0) {
@@ -1088,60 +1120,61 @@ struct Explorer {
             for (int i = 1; i < keep; i++) mm &= mm - 1;
             cut = __ffsll((unsigned long long)mm);  // index of the keep-th cell + 1
         }
-        int8_t *gm = a.mat + (size_t)thief * rows * 64;
-        for (int r = 0; r < l; r++)
-            if (lane < n - r) gm[r * 64 + lane] = lds.mat[lds_mat_row(r, n) + lane];
-        if (lane < n) gm[l * 64 + lane] = (int8_t)rowl;
-        if (lane < n) {
-            a.pos[(size_t)thief * 64 + lane] = (int8_t)(lane < l ? posv : (lane == l ? cut : 0));
-            a.end[(size_t)thief * 64 + lane] = (int8_t)endE;
-            a.dir[(size_t)thief * 64 + lane] = (int8_t)(lane <= l ? dirv : 0);
-        }
-        if (lane == 0) a.line[thief] = l;
+        send_mail(thief, tag, l, rowl, cut, endE);
         // the victim keeps [pos, cut-1] at line l and everything below
         endv = endE;
         if (lane == l) endv = cut - 1;
         if (lane > l && lane < n) endv = n - 1 - lane;
         end_dirty = true;
-        // The thief's count is added before the release below publishes its
-        // interval, so its own decrement (after its acquire) comes later in
-        // the counter's order: relaxed suffices.
-        w_add_rlx<SC>(&ir.ctl->work_count, 1);
-        if (lane == 0) st_rel<SC>(a.state + thief, ST_ACTIVE);
         return true;
     }
 
-    // enter the idle ring (cell sequence protocol of a bounded MPMC queue:
-    // ticket t owns cell t mod cap once the cell shows t; storing t + 1 with
-    // this explorer's id hands it to the consumer of ticket t).  All relaxed:
-    // the cell word carries everything the consumer reads.
+    // member index of this explorer in its instance (the engine's explorers
+    // are their own members).  The member word is complete before the first
+    // registration names it: the wait for the store is explicit, as a fence at
+    // agent scope would write the L2 back.
+    __device__ __forceinline__ void join(int idx)
+    {
+        self = idx;
+        if (ir.member) {
+            if (lane == 0) st_rlx<SC>(const_cast<int *>(ir.member) + idx, e);
+            asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+        }
+        pollw = ir.occ ? 0 : idx % ir.idle_words;
+    }
+
+    // the idle word of the next poll (a wavefront passes over all words in turn;
+    // a pool slot's over those its members fill so far)
+    __device__ __forceinline__ unsigned long long peek_idle()
+    {
+        if (ir.occ) seen = ld_rlx<SC>(ir.occ);
+        return ld_rlx<SC>(ir.idle + (size_t)pollw * IDLE_STRIDE);
+    }
+    __device__ __forceinline__ void next_word()
+    {
+        int words = ir.idle_words;
+        if (ir.occ) words = min(words, uni(seen) & POOL_MEMBERS);
+        pollw = pollw + 1 < words ? pollw + 1 : 0;
+    }
+
     __device__ __forceinline__ void register_idle()
     {
-        if (lane == 0) st_rlx<SC>(a.state + e, ST_IDLE);
-        unsigned t = w_addu_rlx<SC>(&ir.ctl->idle_tail, 1u);
-        const unsigned slot = t & (unsigned)(ir.ring_cap - 1);
-        bool ok = false;
-        for (int spin = 0; spin < PBB_SPIN_LIMIT; spin++) {
-            if ((unsigned)(uni64(ld_rlx64<SC>(ir.ring + slot)) >> 32) == t) {
-                ok = true;
-                break;
-            }
-            __builtin_amdgcn_s_sleep(1);
-        }
-        if (!ok) {
-            fail(PBB_DEV_ERR_RING);
-        } else if (lane == 0) {
-            st_rlx64<SC>(ir.ring + slot, ((unsigned long long)(t + 1u) << 32) | (unsigned)(e + 1));
-        }
+        if (lane == 0)
+            __hip_atomic_fetch_or(ir.idle + (size_t)(self % ir.idle_words) * IDLE_STRIDE,
+                                  1ull << (self / ir.idle_words), __ATOMIC_RELAXED, SC);
     }
 
     // give up an exhausted interval; returns true for the explorer whose
-    // release emptied the instance (all explorers idle: it is solved)
+    // release emptied the instance (all explorers idle: it is solved).  The
+    // registration may take effect before the release: a donor that claims this
+    // explorer counts it again before its message arrives, and itself holds an
+    // interval meanwhile.
     __device__ __forceinline__ bool go_idle()
     {
         register_idle();
-        int left = w_add_rlx<SC>(&ir.ctl->work_count, -1);
-        return left == 1;
+        int left = 0;
+        if (lane == 0) left = __hip_atomic_fetch_add(&ir.ctl->work_count, -1, __ATOMIC_RELAXED, SC);
+        return rdlane(left, 0) == 1;
     }
 
     __device__ __forceinline__ void flush_counters()

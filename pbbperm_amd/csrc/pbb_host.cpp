@@ -212,13 +212,15 @@ struct pbb_engine {
     pbb_config cfg;
     HostTables T;
     DevTables D;
-    int n, m, E, blocks, ring_cap;
+    int n, m, E, blocks;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // device buffers
     int8_t *mat = nullptr, *pos = nullptr, *end = nullptr, *dir = nullptr;
     int *line = nullptr, *state = nullptr;
-    unsigned long long *ring = nullptr;
+    unsigned *mtag = nullptr;
+    unsigned long long *mbox = nullptr;
+    unsigned long long *idle = nullptr;
     Ctl *ctl = nullptr;
     unsigned long long *best = nullptr;
     int *best_perm = nullptr, *root_row = nullptr, *root_dir = nullptr;
@@ -261,8 +263,10 @@ static KArgs make_args(pbb_engine *e)
     a.dir = e->dir;
     a.line = e->line;
     a.state = e->state;
-    a.ring = e->ring;
-    a.ring_cap = e->ring_cap;
+    a.mtag = e->mtag;
+    a.mbox = e->mbox;
+    a.idle = e->idle;
+    a.idle_words = idle_words_for(e->E);
     a.ctl = e->ctl;
     a.best = e->best;
     a.best_perm = e->best_perm;
@@ -314,8 +318,7 @@ extern "C" int pbb_destroy(pbb_engine *e)
     hipFree(e->end);
     hipFree(e->dir);
     hipFree(e->line);
-    hipFree(e->state);
-    hipFree(e->ring);
+    hipFree(e->mbox);
     hipFree(e->ctl);
     hipFree(e->best);
     hipFree(e->best_perm);
@@ -382,16 +385,19 @@ extern "C" int pbb_create(const int32_t *ptm, int n, int m, const pbb_config *cf
         while (w > 0 && team_lds_bytes(e->D.I, lb2, w) > 160 * 1024) w--;
         e->team_E = w;
     }
-    e->ring_cap = 1;
-    while (e->ring_cap < 2 * e->E) e->ring_cap <<= 1;
     size_t E = (size_t)e->E;
     HTRY(hipMalloc(&e->mat, E * n * 64));
     HTRY(hipMalloc(&e->pos, E * 64));
     HTRY(hipMalloc(&e->end, E * 64));
     HTRY(hipMalloc(&e->dir, E * 64));
     HTRY(hipMalloc(&e->line, E * 4));
-    HTRY(hipMalloc(&e->state, E * 4));
-    HTRY(hipMalloc(&e->ring, (size_t)e->ring_cap * 8));
+    // one allocation, cleared once: mailboxes, idle mask, state words, tags
+    const size_t idle_bytes = (size_t)idle_words_for(e->E) * IDLE_STRIDE * 8;
+    const size_t share_bytes = E * 64 * 8 + idle_bytes + E * 8;
+    HTRY(hipMalloc(&e->mbox, share_bytes));
+    e->idle = e->mbox + E * 64;
+    e->state = (int *)((char *)e->idle + idle_bytes);
+    e->mtag = (unsigned *)(e->state + E);
     HTRY(hipMalloc(&e->ctl, sizeof(Ctl)));
     HTRY(hipMalloc(&e->best, 8));
     HTRY(hipMalloc(&e->best_perm, E * 64 * 4));
@@ -405,7 +411,7 @@ extern "C" int pbb_create(const int32_t *ptm, int n, int m, const pbb_config *cf
     int dev = 0;
     HTRY(hipGetDevice(&dev));
     HTRY(hipDeviceGetAttribute(&e->wall_khz, hipDeviceAttributeWallClockRate, dev));
-    HTRY(hipMemsetAsync(e->state, 0, E * 4, e->stream));
+    HTRY(hipMemsetAsync(e->mbox, 0, share_bytes, e->stream));
     unsigned long long packed = ((unsigned long long)(unsigned)ub << 32) | 0xffffffffull;
     HTRY(copy_sync(e, e->best, &packed, 8, hipMemcpyHostToDevice));
 #undef HTRY
@@ -479,7 +485,7 @@ static int setup_pool(pbb_engine *e, const std::vector<int> &ids, const int *pos
             he[(size_t)id * 64 + i] = (int8_t)end[k * n + i];
         }
     }
-    // The idle ring starts empty: idle explorers register themselves when
+    // The idle mask starts empty: idle explorers register themselves when
     // their wavefront runs (pbb_run empties it again before every launch).
     Ctl c;
     memset(&c, 0, sizeof c);
@@ -538,8 +544,8 @@ extern "C" int pbb_init_intervals(pbb_engine *e, int nb, const int *ids, const i
     return setup_pool(e, idv, pos, end);
 }
 
-// One launch: empty the idle ring and clear the stop word (explorers idle at
-// the end of the previous launch register again when they run, so the ring
+// One launch: empty the idle mask and clear the stop word (explorers idle at
+// the end of the previous launch register again when they run, so the mask
 // never names a wavefront that is not resident), then the explorers, either
 // the device-wide grid or the one-workgroup team; the control block and the
 // incumbent word come back into pinned memory behind them, and the host
@@ -548,7 +554,10 @@ static int launch_once(pbb_engine *e, bool team, uint64_t node_budget, double ti
 {
     *e->host_flag = 0;
     KArgs a = make_args(e);
-    if (team) a.E = e->team_E;
+    if (team) {
+        a.E = e->team_E;
+        a.idle_words = idle_words_for(a.E);
+    }
     a.node_budget = node_budget ? e->dec_dev + node_budget : 0;
     a.deadline = time_budget_s > 0 ? (unsigned long long)(time_budget_s * e->wall_khz * 1000.0) : 0;
     HIPCHK(launch_prelaunch(a, e->stream));
@@ -563,7 +572,7 @@ static int launch_once(pbb_engine *e, bool team, uint64_t node_budget, double ti
     const Ctl &c = *e->ctl_h;
     e->done_host = c.done != 0;
     e->dec_dev = c.dec;
-    if (c.err) return fail(PBB_E_HIP, "device error %d in the explorer kernel", c.err);
+    if (!c.done) HIPCHK(launch_collect(a, e->stream));
     return take_incumbent(e, *e->best_h);
 }
 

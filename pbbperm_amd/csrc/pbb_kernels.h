@@ -11,20 +11,46 @@ namespace pbb {
 
 enum { ST_IDLE = 0, ST_ACTIVE = 1, ST_UNFOLD = 2 };
 
-enum { PBB_DEV_ERR_RING = 1 };
+// Idle explorers register in a bit mask: bit b of mask word w stands for the
+// explorer (or pool member) b * words + w.  Each word sits on its own 128-byte
+// line (IDLE_STRIDE words of 64 bits apart).  A donor polls one word at a time,
+// another at every poll, and claims an explorer by clearing its bit: one atomic
+// per attempt, on a line shared with 64 explorers.  One ring for all of them
+// (two ticket counters and a count) had every poll and every claim of the
+// device on one or two lines: 50 us per attempt at 4096 explorers on a thin
+// tree (50x20, 49.7 M nodes, 300 k hand-overs), 77 ms against 29 ms.
+#define IDLE_STRIDE 16
+__device__ __host__ inline int idle_words_for(int explorers) { return (explorers + 63) / 64; }
+
+// Message word of lane i (low 32 bits; the high 32 carry stack entries):
+// bits 0-5 the job of cell i of the split row l, 6 its pruned/visited flag,
+// 7-12 pos[i], 13-18 end[i], 19-24 the job chosen at line i (MAIL_NONE from
+// line l on), 25 dir[i], 26-31 the message's tag.  63 jobs fit: ids and
+// positions are at most 62.
+#define MAIL_NONE 63u
+#define MAIL_TAGS 63u
+__device__ __forceinline__ unsigned mail_word(int cell, int pos, int end, unsigned job, int dir, unsigned tag)
+{
+    const unsigned c = cell < 0 ? (unsigned)(-cell - 1) | 64u : (unsigned)cell;
+    return c | ((unsigned)pos << 7) | ((unsigned)end << 13) | (job << 19) | ((unsigned)dir << 25) | (tag << 26);
+}
+__device__ __forceinline__ int mail_cell(unsigned w) { return (w & 64u) ? -(int)(w & 63u) - 1 : (int)(w & 63u); }
+__device__ __forceinline__ int mail_pos(unsigned w) { return (int)((w >> 7) & 63u); }
+__device__ __forceinline__ int mail_end(unsigned w) { return (int)((w >> 13) & 63u); }
+__device__ __forceinline__ unsigned mail_job(unsigned w) { return (w >> 19) & 63u; }
+__device__ __forceinline__ int mail_dir(unsigned w) { return (int)((w >> 25) & 1u); }
+__device__ __forceinline__ unsigned mail_tag(unsigned w) { return w >> 26; }
+// Cell i of row r < l of a received interval, pos p, chosen job j.  Lines
+// above the split hold no work (their end is their pos): the cells before p
+// are dead, and those after it live, so that coming back up to the line ends
+// the interval at once by the interval-end test, as on the donor's own row.
+__device__ __forceinline__ int mail_path_cell(int i, int p, int j) { return i == p ? j : (i > p ? 0 : -1); }
 
 #define PBB_SPIN_LIMIT (1 << 24)
 
-// A busy explorer of a device-wide launch reads the idle ring every
+// A busy explorer of a device-wide launch reads a word of the idle mask every
 // PBB_POLL_EVERY decomposed nodes (power of two), whether or not explorers
-// wait in it.  Polling at every node while some waited (the earlier policy)
-// had every busy explorer of a small tree race for the same ring ticket at
-// every node: on a 5.0 M-node 19x10 LB2 tree with a frozen incumbent the
-// plain engine took 94 / 275 / 354 ms at 256 / 1024 / 3072 explorers; polling
-// every 4 / 8 / 16 nodes instead, 89 / 81 / 95, 88 / 52 / 61 and 89 / 47 / 53
-// ms; the 512-instance batch at 1024 explorers per instance 599-929 ms
-// before, 178-189 ms at 16; the 50x20 explorer 1984 M nodes/s before,
-// 2036 M at 16.
+// wait in it.
 #ifndef PBB_POLL_EVERY
 #define PBB_POLL_EVERY 16
 #endif
@@ -53,20 +79,15 @@ enum { PBB_DEV_ERR_RING = 1 };
 #define PBB_HOST_POLL_CHECKS 16
 #endif
 
-// Device-resident control block of one engine (or pool slot).  The ring
-// tickets and the work counter take atomics from every donor; the flags are
-// polled by idle explorers; each group sits on its own 128-byte line so the
-// polls do not queue behind the atomics.
+// Device-resident control block of one engine (or pool slot).  The count of
+// working explorers takes atomics at every hand-over and the flags are polled
+// by idle explorers, so each sits on its own 128-byte line.
 struct Ctl {
-    unsigned idle_head;        // ring tickets (dequeue side)
-    unsigned idle_tail;        // ring tickets (enqueue side)
-    int pad0[30];
     int work_count;            // explorers holding an interval
     int pad1[31];
-    int done;                  // set when work_count reaches 0
-    int stop;                  // budget / deadline / interrupt / error
-    int err;                   // device error code
-    int pad2[29];
+    int done;                  // set when no explorer holds an interval
+    int stop;                  // budget / deadline / interrupt
+    int pad2[30];
     unsigned long long dec;    // decomposed nodes
     unsigned long long leaves;
     unsigned long long sb;     // simple (LB1) bounds
@@ -75,12 +96,14 @@ struct Ctl {
     unsigned long long jhisto[65];  // refinement bounds per depth of the bounded node
 };
 
-// The instance one explorer works on: its control block, idle ring,
-// incumbent and bounded root row (one per engine, one per pool slot).
+// The instance one explorer works on: its control block, idle
+// mask, incumbent and bounded root row (one per engine, one per pool slot).
 struct InstRef {
     Ctl *ctl;
-    unsigned long long *ring;   // idle-ring cells: ticket << 32 | explorer + 1
-    int ring_cap;
+    unsigned long long *idle;   // idle mask words, IDLE_STRIDE apart
+    int idle_words;
+    const int *member;          // pool: explorer of each member of the slot (nullptr: member = explorer)
+    const int *occ;             // pool: members so far (nullptr: all words are in use)
     int ub0;                    // initial UB (branching thresholds when not singleNode)
     unsigned long long *best;   // cost << 32 | explorer
     const int *root_row;
@@ -102,10 +125,12 @@ struct KArgs {
     int8_t *dir;        // [E][64]
     int *line;          // [E]
     int *state;         // [E]
-    // idle ring (bounded MPMC cells; each one word, ticket << 32 | explorer + 1,
-    // so a cell moves with single relaxed atomics and no fence)
-    unsigned long long *ring;   // [ring_cap]
-    int ring_cap;               // power of two >= E
+    unsigned *mtag;     // [E] tag of the last message this explorer consumed
+    // mailboxes: a donor hands an interval to an idle explorer as one message
+    // of 64 self-tagged words (pack_mail, pbb_explorer.h)
+    unsigned long long *mbox;   // [E][64]
+    unsigned long long *idle;   // idle mask words, IDLE_STRIDE apart
+    int idle_words;
     Ctl *ctl;
     unsigned long long *best;   // cost << 32 | explorer
     int *best_perm;             // [E][64]
@@ -184,7 +209,7 @@ inline size_t team_lds_bytes(const DevInst &I, bool lb2, int waves)
            (size_t)waves * lds_wave_bytes(I.n, I.m, lb2);
 }
 // LDS size handed to the occupancy query of the persistent kernels.  Their
-// explorers wait on one another (the idle ring, work_count), so every
+// explorers wait on one another (hand-overs, the work count), so every
 // workgroup of the grid must be resident at once.  The query's count can be
 // one workgroup per CU too high when the workgroups fill the CU's LDS to
 // within a granule (12x20 with the Johnson table: 3 x 53904 B of 163840 B
@@ -201,7 +226,7 @@ inline size_t root_lds_bytes(const DevInst &I)
 // instance slot at a time: the first group to pop a slot from the request
 // queue admits it (tables, idle ring, root), later groups join running slots
 // whose explorers are all busy, up to a per-instance explorer cap; work moves
-// between the members of a slot through its idle ring exactly as in the
+// between the members of a slot through its idle mask exactly as in the
 // one-instance engine.  The last member to leave a solved slot writes its
 // result record.  Instances with fewer machines than the pool's M are padded
 // with zero-time machines, which changes none of the bounds or makespans.
@@ -247,10 +272,10 @@ struct PoolSlot {                 // device header of one instance slot
 
 // byte offsets inside one slot's arena (all 256-byte aligned)
 struct PoolLayout {
-    size_t hdr, ptm, ptmT, minA, minD, pair, key, jtab, ring, stride;
+    size_t hdr, ptm, ptmT, minA, minD, pair, key, jtab, idle, member, stride;
 };
 __device__ __host__ inline size_t pool_al(size_t x) { return (x + 255) & ~(size_t)255; }
-__device__ __host__ inline PoolLayout pool_layout(int nmax, int M, int pmax, int ring_cap)
+__device__ __host__ inline PoolLayout pool_layout(int nmax, int M, int pmax, int members)
 {
     const int mp = (M + 3) & ~3;
     PoolLayout L;
@@ -263,7 +288,8 @@ __device__ __host__ inline PoolLayout pool_layout(int nmax, int M, int pmax, int
     L.pair = o;     o += pool_al((size_t)(pmax > 0 ? pmax : 1) * 4);
     L.key = o;      o += pool_al((size_t)(pmax > 0 ? pmax : 1) * nmax * 4);
     L.jtab = o;     o += pool_al((size_t)(pmax > 0 ? pmax : 1) * nmax * 16);
-    L.ring = o;     o += pool_al((size_t)ring_cap * 8);
+    L.idle = o;     o += pool_al((size_t)idle_words_for(members) * IDLE_STRIDE * 8);
+    L.member = o;   o += pool_al((size_t)members * 4);
     L.stride = o;
     return L;
 }
@@ -276,7 +302,7 @@ struct PoolArgs {
     int epi;                      // explorer cap per instance
     int nmax;                     // largest n served
     int pmax;                     // pair-table capacity
-    int ring_cap;                 // idle-ring cells per slot (power of two >= epi)
+    int idle_words;               // idle mask words per slot (64 members each)
     int jt_lds;                   // Johnson tables staged in LDS
     int pairs_mode;               // JohnsonMode: pair list built at admission
     int qcap;                     // queue capacity (power of two)
@@ -285,7 +311,7 @@ struct PoolArgs {
     PoolRes *res;                 // [nslots]
     PoolQueue *q;
     unsigned *q_head;             // consumer ticket (device memory)
-    Ctl *run;                     // stop / error of the launch
+    Ctl *run;                     // stop word of the launch
     unsigned long long req_ticks; // per-request budget after admission (wall_clock64 ticks), 0 = none
     int ig_iters;                 // IG helper rounds per instance (0 = no helper wave)
 };
@@ -336,10 +362,13 @@ hipError_t explore_occupancy(const KArgs &a, int *blocks_per_cu);
 hipError_t launch_root(const KArgs &a, const RootPerm &root_perm, hipStream_t s);
 // engine set-up kernels (pbb_setup.hip, one translation unit): the whole
 // search space to explorer 0 and every other explorer idle, with the
-// control block cleared; the idle ring emptied and the stop word cleared
+// control block cleared; the idle mask emptied and the stop word cleared
 // before a launch
 hipError_t launch_setup_full(const KArgs &a, hipStream_t s);
 hipError_t launch_prelaunch(const KArgs &a, hipStream_t s);
+// after a launch that stopped early: messages that arrived at explorers which
+// had left already become intervals of the saved state
+hipError_t launch_collect(const KArgs &a, hipStream_t s);
 // which: 0 lb1 children, 1 lb1 node, 2 lb2 node, 3 makespan
 hipError_t launch_bounds(int which, const KArgs &a, int count, const int *perms, const int *l1,
                          const int *l2, int arg, int *o1, int *o2, hipStream_t s);

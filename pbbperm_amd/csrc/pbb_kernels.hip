@@ -9,7 +9,7 @@
 //                  with ivm.cpp navigation and ivm_bound.cpp bounding,
 //                  branching and pruning.  Work is balanced on the device: an
 //                  explorer whose interval is exhausted registers in an idle
-//                  ring; busy explorers split their interval as
+//                  mask; busy explorers split their interval as
 //                  bbthread::shareWork (multicore/src/bbthread.cpp:39-72) and
 //                  hand the upper part to an idle explorer.  No host round
 //                  trip until the run ends (all idle, node budget, deadline
@@ -42,6 +42,8 @@ __device__ __forceinline__ void explore_loop(const KArgs &a, const Lds &lds, int
 {
     Explorer<M, REF, SC> X(a, lds, e, engine_inst(a), a.ctl, a.I.n, a.I.mp);
     X.local_best = uni((int)(unsigned)(ld_rlx<SC>(a.best) >> 32));
+    X.open_mail();
+    X.join(e);
     // what the host or the previous launch left is visible at launch start
     int st = uni(ld_rlx<SC>(a.state + e));
     if (st == ST_UNFOLD) {
@@ -54,8 +56,8 @@ __device__ __forceinline__ void explore_loop(const KArgs &a, const Lds &lds, int
     } else if (st == ST_ACTIVE) {
         X.load_state();
     } else {
-        // An idle explorer enters the idle ring only once it runs (the host
-        // leaves the ring empty at every launch), so donors only ever hand
+        // An idle explorer enters the idle mask only once it runs (the host
+        // leaves the mask empty at every launch), so donors only ever hand
         // work to wavefronts that are resident: one still waiting for a CU
         // (another kernel or process on the device, an occupancy estimate
         // that was too high) holds no work that the others wait for.
@@ -72,20 +74,20 @@ __device__ __forceinline__ void explore_loop(const KArgs &a, const Lds &lds, int
             // longest, and the first to see it raises the device stop word
             int nap = 1;
             while (true) {
-                // relaxed poll (an acquire would invalidate the L2 at every
-                // pass); the fence pairs with the donor's release of the word
-                int s = uni(ld_rlx<SC>(a.state + e));
-                if (s == ST_ACTIVE) {
-                    fence_acq<SC>();
+                // one poll: the mailbox and the words a leave depends on, all
+                // in flight together
+                const unsigned long long mail = X.peek_mail(), bw = ld_rlx<SC>(a.best);
+                const int done = ld_rlx<SC>(&a.ctl->done), stop = ld_rlx<SC>(&a.ctl->stop);
+                if (X.mail_here(mail)) {
                     st = ST_ACTIVE;
-                    X.load_state();
+                    X.take_mail(mail);
                     // a donated interval is explored under the current incumbent,
                     // not the one this explorer saw before it went idle
-                    X.take_best(ld_rlx<SC>(a.best));
+                    X.take_best(bw);
                     break;
                 }
-                if (uni(ld_rlx<SC>(&a.ctl->done)) || uni(ld_rlx<SC>(&a.ctl->stop)) ||
-                    (X.t_end && wall_clock64() >= X.t_end)) {
+                if (uni(done) || uni(stop) || (X.t_end && wall_clock64() >= X.t_end)) {
+                    X.leave_idle();
                     X.flush_counters();
                     return;
                 }
@@ -96,20 +98,15 @@ __device__ __forceinline__ void explore_loop(const KArgs &a, const Lds &lds, int
                 else X.idle_pause(nap);
             }
         }
-        // idle-ring poll issued before the node's work so its latency is
+        // idle-mask poll issued before the node's work so its latency is
         // hidden; none while the ramp holds this explorer's work back.  In
         // the workgroup team (at most 16 explorers, workgroup-scope atomics)
         // a donor that saw explorers waiting polls again at the next node; at
-        // device scope every busy explorer racing for the same ring ticket at
-        // every node made the ring words a hot spot, so there it polls every
-        // PBB_POLL_EVERY nodes only.
+        // device scope it polls every PBB_POLL_EVERY nodes only.
         constexpr bool team = SC == __HIP_MEMORY_SCOPE_WORKGROUP;
         const bool poll = X.since >= a.ramp && ((team && hungry) || (iter & (PBB_POLL_EVERY - 1)) == 0u);
-        unsigned rh = 0, rt = 0;
-        if (poll) {
-            rh = ld_rlx<SC>(&a.ctl->idle_head);
-            rt = ld_rlx<SC>(&a.ctl->idle_tail);
-        }
+        unsigned long long idle = 0ull;
+        if (poll) idle = X.peek_idle();
         const bool refresh = (iter & (PBB_BEST_EVERY - 1)) == 0u;
         unsigned long long bw = ~0ull;
         if (refresh) bw = ld_rlx<SC>(a.best);
@@ -124,7 +121,7 @@ __device__ __forceinline__ void explore_loop(const KArgs &a, const Lds &lds, int
             X.flush_counters();
             return;
         }
-        if (poll) hungry = X.try_donate(rh, rt);
+        if (poll) hungry = X.try_donate(idle);
     }
 }
 

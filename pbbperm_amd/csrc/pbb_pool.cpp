@@ -42,7 +42,7 @@ int next_pow2(int x)
 struct pbb_pool {
     pbb_config cfg;
     pbb_pool_params prm;
-    int M = 0, nmax = 0, pmax = 0, ring_cap = 0, jt_lds = 0, W = 0, epi = 0, margin = 0;
+    int M = 0, nmax = 0, pmax = 0, epi_max = 0, jt_lds = 0, W = 0, epi = 0, margin = 0;
     int ig = 0;  // IG helper rounds per instance (0 = none)
     int groups = 0, E = 0, qcap = 0;
     size_t lds = 0;
@@ -54,6 +54,7 @@ struct pbb_pool {
     char *arena = nullptr;
     int8_t *mat = nullptr, *pos = nullptr, *end = nullptr, *dir = nullptr;
     int *line = nullptr, *state = nullptr, *best_perm = nullptr;
+    unsigned long long *mbox = nullptr;
     Ctl *run = nullptr;
     unsigned *q_head = nullptr;
     PoolReq *req_d = nullptr;
@@ -99,6 +100,7 @@ static KArgs pool_kargs(const pbb_pool *p, double budget_s)
     a.dir = p->dir;
     a.line = p->line;
     a.state = p->state;
+    a.mbox = p->mbox;
     a.best_perm = p->best_perm;
     a.ctl = p->run;
     a.host_flag = p->host_flag_d;
@@ -124,7 +126,7 @@ static PoolArgs pool_pargs(const pbb_pool *p, bool serve)
     q.epi = p->epi;
     q.nmax = p->nmax;
     q.pmax = p->pmax;
-    q.ring_cap = p->ring_cap;
+    q.idle_words = idle_words_for(p->epi);
     q.ig_iters = p->ig;
     q.jt_lds = p->jt_lds;
     q.pairs_mode = p->cfg.johnson_pairs;
@@ -171,6 +173,7 @@ extern "C" int pbb_pool_destroy(pbb_pool *p)
     hipFree(p->dir);
     hipFree(p->line);
     hipFree(p->state);
+    hipFree(p->mbox);
     hipFree(p->best_perm);
     hipFree(p->run);
     hipFree(p->q_head);
@@ -261,8 +264,8 @@ extern "C" int pbb_pool_create(const pbb_config *cfg, const pbb_pool_params *prm
     }
     p->E = p->groups * p->W;
     p->epi = std::min(p->epi, p->E);
-    p->ring_cap = next_pow2(std::max(64, 2 * p->epi));
-    p->lay = pool_layout(p->nmax, p->M, p->pmax, p->ring_cap);
+    p->epi_max = next_pow2(std::max(32, p->epi));
+    p->lay = pool_layout(p->nmax, p->M, p->pmax, p->epi_max);
     const size_t S = (size_t)prm->slots, E = (size_t)p->E;
     HTRY(hipMalloc(&p->arena, S * p->lay.stride));
     HTRY(hipMalloc(&p->mat, E * p->nmax * 64));
@@ -271,6 +274,7 @@ extern "C" int pbb_pool_create(const pbb_config *cfg, const pbb_pool_params *prm
     HTRY(hipMalloc(&p->dir, E * 64));
     HTRY(hipMalloc(&p->line, E * 4));
     HTRY(hipMalloc(&p->state, E * 4));
+    HTRY(hipMalloc(&p->mbox, E * 64 * 8));
     HTRY(hipMalloc(&p->best_perm, E * 64 * 4));
     HTRY(hipMalloc(&p->run, sizeof(Ctl)));
     HTRY(hipMalloc(&p->q_head, 64));
@@ -279,6 +283,7 @@ extern "C" int pbb_pool_create(const pbb_config *cfg, const pbb_pool_params *prm
     HTRY(hipMalloc(&p->q_d, queue_bytes(p->qcap)));
     HTRY(hipMemset(p->arena, 0, S * p->lay.stride));
     HTRY(hipMemset(p->state, 0, E * 4));
+    HTRY(hipMemset(p->mbox, 0, E * 64 * 8));
     HTRY(hipMemset(p->run, 0, sizeof(Ctl)));
     HTRY(hipHostMalloc((void **)&p->req_h, S * sizeof(PoolReq), hipHostMallocDefault));
     HTRY(hipHostMalloc((void **)&p->res_h, S * sizeof(PoolRes), hipHostMallocDefault));
@@ -320,9 +325,8 @@ extern "C" int pbb_pool_retune(pbb_pool *p, int explorers_per_instance, int stea
     if (explorers_per_instance < p->W || steal_margin < 0)
         return fail(PBB_E_ARG, "explorers_per_instance %d / steal_margin %d", explorers_per_instance, steal_margin);
     int epi = std::min(explorers_per_instance - explorers_per_instance % p->W, p->E);
-    if (2 * epi > p->ring_cap)
-        return fail(PBB_E_CAPACITY, "explorers_per_instance %d above the pool's idle-ring capacity %d", epi,
-                    p->ring_cap / 2);
+    if (epi > p->epi_max)
+        return fail(PBB_E_CAPACITY, "explorers_per_instance %d above the pool's member capacity %d", epi, p->epi_max);
     p->epi = epi;
     p->margin = steal_margin ? steal_margin : p->cfg.steal_margin;
     return PBB_OK;
@@ -358,14 +362,6 @@ static void to_result(const pbb_pool *p, const PoolRes &r, int n, int tag, unsig
     o->admit_ms = r.t_admit >= t0 ? (double)(r.t_admit - t0) * k : 0.0;
     o->done_ms = r.t_done >= t0 ? (double)(r.t_done - t0) * k : 0.0;
     for (int i = 0; i < PBB_MAX_JOBS; i++) o->perm[i] = (r.improved && i < n) ? r.perm[i] : -1;
-}
-
-static int check_run_error(pbb_pool *p)
-{
-    Ctl c;
-    HIPCHK(hipMemcpy(&c, p->run, sizeof c, hipMemcpyDeviceToHost));
-    if (c.err) return fail(PBB_E_HIP, "device error %d in the pool kernel", c.err);
-    return PBB_OK;
 }
 
 extern "C" int pbb_pool_solve(pbb_pool *p, int count, const int32_t *ptms, const int *n, const int *m,
@@ -429,8 +425,6 @@ extern "C" int pbb_pool_solve(pbb_pool *p, int count, const int32_t *ptms, const
     HIPCHK(hipEventElapsedTime(&ms, p->ev0, p->ev1));
     if (kernel_ms) *kernel_ms = ms;
     p->last_count = count;
-    int rc = check_run_error(p);
-    if (rc) return rc;
     unsigned long long t0 = ULLONG_MAX;
     for (int i = 0; i < count; i++)
         if (p->res_h[i].tag == i) t0 = std::min(t0, p->res_h[i].t_admit);
@@ -557,7 +551,7 @@ extern "C" int pbb_serve_stop(pbb_pool *p)
     __atomic_store_n(&p->sq->closed, 1, __ATOMIC_RELEASE);
     HIPCHK(hipStreamSynchronize(p->stream));
     p->serving = false;
-    return check_run_error(p);
+    return PBB_OK;
 }
 
 // Stop serving on several pools: close every queue first, then wait for

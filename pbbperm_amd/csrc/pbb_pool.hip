@@ -15,7 +15,7 @@
 //                    * helper: joins the running slot with the most busy
 //                      explorers net of idle ones (up to the per-instance
 //                      cap) and receives work
-//                      through the slot's idle ring, as explorers of the
+//                      through the slot's idle mask, as explorers of the
 //                      one-instance engine do.
 //                  The explorer whose release empties a slot records the
 //                  optimum; the last member to leave writes the result
@@ -83,8 +83,10 @@ __device__ __forceinline__ InstRef slot_ref(const PoolArgs &p, int s, PoolSlot *
     char *b = slot_base(p, s);
     InstRef r;
     r.ctl = &S->c;
-    r.ring = (unsigned long long *)(b + p.lay.ring);
-    r.ring_cap = p.ring_cap;
+    r.idle = (unsigned long long *)(b + p.lay.idle);
+    r.idle_words = p.idle_words;
+    r.member = (const int *)(b + p.lay.member);
+    r.occ = &S->occ;
     r.ub0 = ub;
     r.best = &S->best;
     r.root_row = S->root_row;
@@ -189,14 +191,14 @@ static __device__ __forceinline__ bool pool_admit(const PoolArgs &p, int s, bool
         for (int k = a + 1; k < c; k++) lag += ptm[k * n + j];
         jtab[pi * n + rank] = make_int4(j, ptm[a * n + j], ptm[c * n + j], lag);
     }
-    // control block, incumbent, idle ring
+    // control block, incumbent, idle mask
     int *ci = (int *)&S->c;
     const int wc = (int)(offsetof(Ctl, work_count) / 4);
     // explorer 0 holds the full interval; an IG helper wave holds one more unit
     const int held = p.ig_iters > 0 ? 2 : 1;
     for (int i = tid; i < (int)(sizeof(Ctl) / 4); i += nt) ci[i] = (i == wc) ? held : 0;
-    unsigned long long *rs = (unsigned long long *)(b + p.lay.ring);
-    for (int i = tid; i < p.ring_cap; i += nt) rs[i] = (unsigned long long)(unsigned)i << 32;
+    unsigned long long *im = (unsigned long long *)(b + p.lay.idle);
+    for (int i = tid; i < p.idle_words; i += nt) im[(size_t)i * IDLE_STRIDE] = 0ull;
     if (tid == 0) {
         S->best = ((unsigned long long)(unsigned)ub << 32) | 0xffffffffull;
         S->t_admit = wall_clock64();
@@ -217,8 +219,11 @@ static __device__ __forceinline__ bool pool_admit(const PoolArgs &p, int s, bool
 // -------------------------------------------------------- slot selection
 // Wave 0 of a free workgroup: a new instance from the queue first, else the
 // running slot with the largest surplus of busy over idle explorers (below
-// the per-instance cap), else wait.  Returns the role; *slot receives the slot id.
-static __device__ __forceinline__ int pool_pick(const PoolArgs &p, int W, unsigned long long t_end, const int *host_flag, int *slot)
+// the per-instance cap), else wait.  Returns the role; *slot receives the slot id
+// and *base the member index of the group's first wave (members stay until the
+// slot is done, so the indices are dense).
+static __device__ __forceinline__ int pool_pick(const PoolArgs &p, int W, unsigned long long t_end, const int *host_flag, int *slot,
+                                                 int *base)
 {
     const int lane = lane_id();
     // A waiting group passes here every microsecond or so, and hundreds may
@@ -245,6 +250,7 @@ static __device__ __forceinline__ int pool_pick(const PoolArgs &p, int W, unsign
                 // still being admitted, instead of leaving the launch
                 if (lane == 0)
                     __hip_atomic_store(&slot_hdr(p, *slot)->occ, W, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                *base = 0;
                 return ROLE_OWNER;
             }
             continue;
@@ -275,6 +281,7 @@ static __device__ __forceinline__ int pool_pick(const PoolArgs &p, int W, unsign
         if (best_slot >= 0) {
             if (w_cas((unsigned *)&slot_hdr(p, best_slot)->occ, (unsigned)best_occ, (unsigned)(best_occ + W))) {
                 *slot = best_slot;
+                *base = best_occ & POOL_MEMBERS;
                 return ROLE_HELPER;
             }
             continue;
@@ -404,7 +411,7 @@ template <int M, int REF>
 __global__ __launch_bounds__(256, PBB_POOL_MIN_WAVES(M)) void k_pool(KArgs a, PoolArgs p)
 {
     extern __shared__ __align__(16) char smem[];
-    __shared__ int s_pick[2];
+    __shared__ int s_pick[3];
     const int W = p.W;
     const int wave = threadIdx.x >> 6;
     const int e = blockIdx.x * W + wave;
@@ -421,15 +428,16 @@ __global__ __launch_bounds__(256, PBB_POOL_MIN_WAVES(M)) void k_pool(KArgs a, Po
     }
     for (;;) {
         if (wave == 0) {
-            int slot = -1;
-            const int role = pool_pick(p, W, t_end, a.host_flag, &slot);
+            int slot = -1, base = 0;
+            const int role = pool_pick(p, W, t_end, a.host_flag, &slot, &base);
             if (lane == 0) {
                 s_pick[0] = slot;
                 s_pick[1] = role;
+                s_pick[2] = base;
             }
         }
         __syncthreads();
-        const int slot = s_pick[0], role = s_pick[1];
+        const int slot = s_pick[0], role = s_pick[1], base = s_pick[2];
         if (role == ROLE_EXIT) break;
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         PoolSlot *S = slot_hdr(p, slot);
@@ -483,6 +491,8 @@ __global__ __launch_bounds__(256, PBB_POOL_MIN_WAVES(M)) void k_pool(KArgs a, Po
             Explorer<M, REF> X(a, lds, e, slot_ref(p, slot, S, m, npairs, ub), p.run, n, I.mp);
             X.t_end = slot_end;
             X.local_best = uni((int)(unsigned)(ld_rlx(&S->best) >> 32));
+            X.open_mail();
+            X.join(base + wave);
             int st = ST_IDLE;
             if (igw) {
                 if (X.go_idle()) pool_finish(X, a, S);
@@ -516,17 +526,15 @@ __global__ __launch_bounds__(256, PBB_POOL_MIN_WAVES(M)) void k_pool(KArgs a, Po
                     bool leave = false;
                     int nap = 1;
                     while (true) {
-                        const int sv = uni(ld_rlx(a.state + e));
-                        if (sv == ST_ACTIVE) {
-                            // pairs with the donor's release of the state word
-                            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+                        const unsigned long long mail = X.peek_mail(), bw = ld_rlx(&S->best);
+                        const int done = ld_rlx(&S->c.done), stop = ld_rlx(&p.run->stop);
+                        if (X.mail_here(mail)) {
                             st = ST_ACTIVE;
-                            X.load_state();
-                            X.take_best(ld_rlx(&S->best));
+                            X.take_mail(mail);
+                            X.take_best(bw);
                             break;
                         }
-                        if (uni(ld_rlx(&S->c.done)) || uni(ld_rlx(&p.run->stop)) ||
-                            (t_end && uni64(wall_clock64()) >= t_end)) {
+                        if (uni(done) || uni(stop) || (t_end && uni64(wall_clock64()) >= t_end)) {
                             leave = true;
                             break;
                         }
@@ -535,11 +543,8 @@ __global__ __launch_bounds__(256, PBB_POOL_MIN_WAVES(M)) void k_pool(KArgs a, Po
                     if (leave) break;
                 }
                 const bool poll = (iter & (PBB_POLL_EVERY - 1)) == 0u;
-                unsigned rh = 0, rt = 0;
-                if (poll) {
-                    rh = ld_rlx(&S->c.idle_head);
-                    rt = ld_rlx(&S->c.idle_tail);
-                }
+                unsigned long long idle = 0ull;
+                if (poll) idle = X.peek_idle();
                 const bool refresh = (iter & (PBB_BEST_EVERY - 1)) == 0u;
                 unsigned long long bw = ~0ull;
                 if (refresh) bw = ld_rlx(&S->best);
@@ -558,7 +563,7 @@ __global__ __launch_bounds__(256, PBB_POOL_MIN_WAVES(M)) void k_pool(KArgs a, Po
                         continue;
                     }
                 }
-                if (poll) X.try_donate(rh, rt);
+                if (poll) X.try_donate(idle);
             }
             X.flush_counters();
         }
@@ -588,7 +593,6 @@ __global__ void k_pool_init(PoolArgs p, int count)
     if (t == 0) {
         *p.q_head = 0u;
         p.run->stop = 0;
-        p.run->err = 0;
         if (count > 0) {
             p.q->tail = count;
             p.q->closed = 1;

@@ -38,16 +38,37 @@ __global__ __launch_bounds__(256) void k_setup_full(KArgs a)
     }
 }
 
-// before every explorer launch: the idle ring empty (cell i waits for ticket
-// i and names no explorer, both ticket counters 0) and the stop word clear
+// before every explorer launch: the idle mask empty and the stop word clear
 __global__ __launch_bounds__(256) void k_prelaunch(KArgs a)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < a.ring_cap) a.ring[t] = (unsigned long long)(unsigned)t << 32;
-    if (t == 0) {
-        a.ctl->idle_head = 0u;
-        a.ctl->idle_tail = 0u;
-        a.ctl->stop = 0;
+    if (t < a.idle_words) a.idle[(size_t)t * IDLE_STRIDE] = 0ull;
+    if (t == 0) a.ctl->stop = 0;
+}
+
+// One wavefront per explorer: a message newer than the one its explorer last
+// consumed was handed over while the launch stopped (the donor had claimed the
+// explorer, which then left on the stop word).  It becomes the explorer's saved
+// interval, as the explorer would have saved it.
+__global__ __launch_bounds__(64) void k_collect(KArgs a)
+{
+    const int e = blockIdx.x, lane = threadIdx.x, n = a.I.n;
+    const unsigned w = (unsigned)a.mbox[(size_t)e * 64 + lane];
+    if (a.state[e] != ST_IDLE || mail_tag(w) == a.mtag[e]) return;  // uniform: one tag per message
+    const int l = __ffsll((unsigned long long)__ballot(mail_job(w) == MAIL_NONE)) - 1;
+    int8_t *gm = a.mat + (size_t)e * a.rows * 64;
+    for (int r = 0; r < l; r++) {
+        const unsigned wr = (unsigned)__shfl((int)w, r, 64);
+        gm[r * 64 + lane] = (int8_t)mail_path_cell(lane, mail_pos(wr), (int)mail_job(wr));
+    }
+    gm[l * 64 + lane] = (int8_t)mail_cell(w);
+    a.pos[(size_t)e * 64 + lane] = (int8_t)mail_pos(w);
+    a.end[(size_t)e * 64 + lane] = (int8_t)mail_end(w);
+    a.dir[(size_t)e * 64 + lane] = (int8_t)mail_dir(w);
+    if (lane == 0) {
+        a.line[e] = l;
+        a.state[e] = ST_ACTIVE;
+        a.mtag[e] = mail_tag(w);
     }
 }
 
@@ -61,7 +82,13 @@ hipError_t launch_setup_full(const KArgs &a, hipStream_t s)
 
 hipError_t launch_prelaunch(const KArgs &a, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_prelaunch, dim3((a.ring_cap + 255) / 256), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(k_prelaunch, dim3((a.idle_words + 255) / 256), dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_collect(const KArgs &a, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_collect, dim3(a.E), dim3(64), 0, s, a);
     return hipGetLastError();
 }
 
