@@ -97,7 +97,10 @@ struct DevInst {
     const int *min_dep;   // [m] bound_fsp_weak.cpp:253-267
     int npairs;
     const int *pair_ab;   // [npairs] a | b << 8, (i<j) lexicographic (bound_fsp_strong.cpp:282-297)
-    const int4 *jtab;     // [npairs][n] {job, p_a, p_b, lag} in Johnson order
+    // [n][npairs]: the i-th job of every pair's Johnson order, packed words
+    // (jpacked) or pairs of words
+    const void *jtab;
+    int jpacked;
 };
 
 // ---------------------------------------------------------------------------
@@ -180,61 +183,106 @@ __device__ __forceinline__ void pair_lanes(const int *pair_ab, int npairs, int m
     }
 }
 
+// Entry of a Johnson table: job, p_a - p_b and w = p_a + lag, all the bound's
+// recurrence needs (lb2_pairs).  Packed in one word when no processing time
+// exceeds JPACK_MAX (job in bits 0-5, w in 6-20: at most 19 x 1023; p_a - p_b
+// in 21-31), else two words {w, (p_a - p_b) << 6 | job} (times of at most
+// 10^6, as the entry points check).
+#define JPACK_MAX 1023
+__device__ __host__ inline unsigned jpack_word(int job, int pa, int pb, int lag)
+{
+    return (unsigned)job | ((unsigned)(pa + lag) << 6) | ((unsigned)(pa - pb) << 21);
+}
+__device__ __host__ inline int2 jpack_pair(int job, int pa, int pb, int lag)
+{
+    return int2{pa + lag, (int)(((unsigned)(pa - pb) << 6) | (unsigned)job)};
+}
+
+// -1 when the job in the low bits of e is unscheduled, else 0
+template <bool N32>
+__device__ __forceinline__ int job_mask(int e, uint64_t unsched)
+{
+    if constexpr (N32) return __builtin_amdgcn_sbfe((int)(unsigned)unsched, (unsigned)e, 1u);  // offset: bits 0-4 of e
+    else return __builtin_amdgcn_sbfe((int)(unsigned)(unsched >> (e & 63)), 0u, 1u);
+}
+
 // Johnson LB2 of one partial schedule over the machine pairs of pinfo
 // (bound_fsp_strong.cpp:50-100, :102-162 without early exit, as
-// bornes_calculer calls them, :540-560): fs / bs are its front and back completion
-// times (LDS, indexed by machine), unsched the bit set of its unscheduled
-// jobs, jtab the per-pair Johnson order {job, p_a, p_b, lag} of all n jobs.
-// Each lane runs its pair's two-machine recurrence over the unscheduled jobs
-// in that order; the loop body is predicated, so a lane never branches on a
-// job, and jtab is read with one 16-byte load per job (ds_read_b128 when the
-// caller passes the LDS copy: a pointer that may be either would make every
-// access a flat load).  N32: n <= 32, the membership test is one bit
-// extract of the low word.
-template <int PCH, bool N32>
-__device__ __forceinline__ int lb2_pairs(const int (&pinfo)[PCH], const int4 *jtab, int n, const int *fs,
-                                         const int *bs, uint64_t unsched)
+// bornes_calculer calls them, :540-560).  fs: its front completion times;
+// gs: back completion times plus remaining work (both LDS, by machine);
+// unsched: the bit set of its unscheduled jobs, not empty.
+//
+// The reference's recurrence over the unscheduled jobs in Johnson order,
+//   t0 += p_a;  t1 = max(t1, t0 + lag) + p_b,
+// is t1 = S_b + max(t1_0, max_j (D_j + p_aj + lag_j)) with S_b the sum of all
+// p_b and D_j = t0_0 + sum of p_a - p_b over the unscheduled jobs before j, and
+// t0 ends at t0_0 + S_a.  So a step is one table word, masked to zero for a
+// scheduled job, an add to D and a max, instead of a chain of six dependent
+// operations with two selects.  A scheduled job's D + 0 enters the max too:
+// never above the true value, since the next unscheduled job's term is at
+// least D, and after the last one D + S_b = t0_0 + S_a <= t1.
+//
+// Lane = pair, all chunks of 64 pairs in one pass (independent chains), the
+// table job-major so that the lanes of a step read consecutive words.  The
+// former layout (a row of 16-byte entries per pair) had 64 lanes read 64
+// cache lines per step from global memory (20 machines), or one LDS bank group
+// (n a multiple of 8).  30x20: 42 us per node of 1.4 bounds before.
+// Each use of it names one table, in LDS or in global memory: a pointer that
+// may be either makes every access a flat load.
+template <int PCH, bool N32, bool PACKED>
+__device__ __forceinline__ int lb2_pairs(const int (&pinfo)[PCH], const void *jtab, int n, int npairs,
+                                         const int *fs, const int *gs, uint64_t unsched)
 {
-    const unsigned unsched32 = (unsigned)unsched;
     const int lane = lane_id();
-    int best = 0;
+    int D[PCH], best[PCH], col[PCH];
+#pragma unroll
+    for (int c = 0; c < PCH; c++) {
+        col[c] = min(c * PBB_WAVE + lane, npairs - 1);
+        const int ab = pinfo[c] < 0 ? 0 : pinfo[c];
+        D[c] = fs[ab & 0xff];
+        best[c] = fs[ab >> 8];
+    }
+#pragma unroll 4
+    for (int i = 0; i < n; i++) {
+#pragma unroll
+        for (int c = 0; c < PCH; c++) {
+            if constexpr (PACKED) {
+                int e = (int)((const unsigned *)jtab)[i * npairs + col[c]];
+                e &= job_mask<N32>(e, unsched);
+                best[c] = max(best[c], D[c] + (int)__builtin_amdgcn_ubfe((unsigned)e, 6u, 15u));
+                D[c] += e >> 21;
+            } else {
+                const int2 e = ((const int2 *)jtab)[i * npairs + col[c]];
+                const int m = job_mask<N32>(e.y, unsched);
+                best[c] = max(best[c], D[c] + (e.x & m));
+                D[c] += (e.y & m) >> 6;
+            }
+        }
+    }
+    int r = 0;
 #pragma unroll
     for (int c = 0; c < PCH; c++) {
         const int info = pinfo[c];
         if (info >= 0) {
             const int a = info & 0xff, b = info >> 8;
-            int t0 = fs[a], t1 = fs[b];
-            const int4 *row = jtab + (size_t)(c * PBB_WAVE + lane) * n;
-#pragma unroll 4
-            for (int i = 0; i < n; i++) {
-                const int4 e = row[i];
-                bool use;
-                if constexpr (N32)
-                    use = (unsched32 >> e.x) & 1u;
-                else
-                    use = (unsched >> e.x) & 1ull;
-                const int u0 = t0 + e.y;
-                const int u1 = max(t1, u0 + e.w) + e.z;
-                t0 = use ? u0 : t0;
-                t1 = use ? u1 : t1;
-            }
-            best = max(best, max(t1 + bs[b], t0 + bs[a]));
+            r = max(r, max(best[c] + gs[b], fs[a] + gs[a]));
         }
     }
-    return wave_max(best);
+    return wave_max(r);
 }
 
-// lb2_pairs with the table in LDS (jl) or in global memory, for any n
+// lb2_pairs with the packed table staged in LDS, or the packed or the wide one
+// in global memory
 template <int PCH>
-__device__ __forceinline__ int lb2_pairs_any(const int (&pinfo)[PCH], bool jl, const int4 *jtabL,
-                                             const int4 *jtabG, int n, const int *fs, const int *bs,
-                                             uint64_t unsched)
+__device__ __forceinline__ int lb2_pairs_any(const int (&pinfo)[PCH], bool staged, const unsigned *jtabL,
+                                             const void *jtabG, bool packed, int n, int npairs, const int *fs,
+                                             const int *gs, uint64_t unsched)
 {
-    if (n <= 32)
-        return jl ? lb2_pairs<PCH, true>(pinfo, jtabL, n, fs, bs, unsched)
-                  : lb2_pairs<PCH, true>(pinfo, jtabG, n, fs, bs, unsched);
-    return jl ? lb2_pairs<PCH, false>(pinfo, jtabL, n, fs, bs, unsched)
-              : lb2_pairs<PCH, false>(pinfo, jtabG, n, fs, bs, unsched);
+    if (staged)
+        return n <= 32 ? lb2_pairs<PCH, true, true>(pinfo, jtabL, n, npairs, fs, gs, unsched)
+                       : lb2_pairs<PCH, false, true>(pinfo, jtabL, n, npairs, fs, gs, unsched);
+    return packed ? lb2_pairs<PCH, false, true>(pinfo, jtabG, n, npairs, fs, gs, unsched)
+                  : lb2_pairs<PCH, false, false>(pinfo, jtabG, n, npairs, fs, gs, unsched);
 }
 
 }  // namespace pbb

@@ -124,9 +124,9 @@ struct Lds {
     int *pmR;       // the same rows, machines reversed: pmR[q] = pm[m-1-q]
     int ps;         // row stride of pm (PM_STRIDE)
     int *minA, *minD, *tot;
-    int4 *jtabL;    // Johnson table staged in LDS (valid when jtl)
-    const int4 *jtabG;  // the same table in global memory
-    bool jtl;
+    unsigned *jtabL;    // packed Johnson table staged in LDS (valid when jtl)
+    const void *jtabG;  // the table in global memory
+    bool jtl, jpacked;
     int8_t *mat;    // this wave's IVM matrix, row l at mat + lds_mat_row(l, n)
     int *stk;       // this wave's stacks: F entry s at row s, B entry s at row n-s ((n+1) x m)
     int2 *U;        // this wave's LB1 operand block [2][m]
@@ -148,8 +148,9 @@ __device__ __forceinline__ Lds lds_setup(const DevInst &I, char *smem, bool load
     L.tot = L.minD + mp;
     size_t off = ((size_t)2 * m * PM_STRIDE + 3 * (size_t)mp) * 4;
     off = (off + 15) & ~(size_t)15;
-    load_jtab = load_jtab && jtab_in_lds(n, I.npairs);
-    L.jtabL = (int4 *)(smem + off);
+    load_jtab = load_jtab && jtab_staged(I);
+    L.jtabL = (unsigned *)(smem + off);
+    L.jpacked = I.jpacked != 0;
     L.jtabG = I.jtab;
     L.jtl = load_jtab;
     char *wbase = smem + lds_table_bytes(n, m, I.npairs, load_jtab) +
@@ -173,7 +174,7 @@ __device__ __forceinline__ Lds lds_setup(const DevInst &I, char *smem, bool load
         L.tot[i] = s;
     }
     if (load_jtab)
-        for (int i = threadIdx.x; i < I.npairs * n; i += blockDim.x) L.jtabL[i] = I.jtab[i];
+        for (int i = threadIdx.x; i < I.npairs * n; i += blockDim.x) L.jtabL[i] = ((const unsigned *)I.jtab)[i];
     __syncthreads();
     return L;
 }
@@ -277,6 +278,7 @@ struct Explorer {
     int L;                            // current line
     int rowv, posv, endv, dirv, remv; // lane vectors (remv: lane q = remaining work on machine q)
     int nf, nb;
+    uint64_t free_jobs;               // unscheduled jobs of the current path (REF 2)
     int ftop;                         // lane q < M: top front entry f_q (frow(nf)), else 0
     static constexpr int PCH = (M * (M - 1) / 2 + PBB_WAVE - 1) / PBB_WAVE;  // pair chunks (M >= 2)
     int pinfo[PCH];                   // this lane's Johnson machine pairs (REF 2)
@@ -301,6 +303,7 @@ struct Explorer {
         rowv = posv = endv = dirv = remv = 0;
         nf = nb = 0;
         ftop = 0;
+        free_jobs = 0ull;
         if constexpr (REF == 2) pair_lanes<PCH>(r.pair_ab, r.npairs, r.m, r.pairs_mode, pinfo);
         dec = leaves = sb = jb = 0;
         since = 0;
@@ -345,6 +348,7 @@ struct Explorer {
             brow(0)[lane] = lds.minD[lane];
         }
         remv = lane < M ? lds.tot[lane] : 0;
+        if constexpr (REF == 2) free_jobs = lanes_below(n);
         __builtin_amdgcn_wave_barrier();
     }
 
@@ -370,6 +374,7 @@ struct Explorer {
             nb++;
         }
         remv -= pk;
+        if constexpr (REF == 2) free_jobs &= ~(1ull << j);
         __builtin_amdgcn_wave_barrier();
     }
 
@@ -382,6 +387,7 @@ struct Explorer {
             nb--;
         }
         remv += pmach(j);
+        if constexpr (REF == 2) free_jobs |= 1ull << j;
     }
 
     // ivm::beforeEnd (ivm.cpp:152-160): lexicographic pos <= end
@@ -579,18 +585,6 @@ struct Explorer {
     }
 
     // ---------------------------------------------------------- refinement
-    __device__ __forceinline__ uint64_t row_jobs(bool valid, int job) const
-    {
-        uint64_t bits = valid ? (1ull << job) : 0ull;
-        unsigned lo = (unsigned)bits, hi = (unsigned)(bits >> 32);
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            lo |= (unsigned)__shfl_xor((int)lo, o, PBB_WAVE);
-            hi |= (unsigned)__shfl_xor((int)hi, o, PBB_WAVE);
-        }
-        return ((uint64_t)(unsigned)uni((int)hi) << 32) | (unsigned)uni((int)lo);
-    }
-
     // The refinement bounds below work on one child per lane (lane = row
     // cell), both directions, with the child's chains computed per lane
     // (the refinement modes serve instances of up to 30 jobs; LB1 above is
@@ -643,40 +637,43 @@ struct Explorer {
     // (bound_fsp_strong::bornes_calculer with the child's partial schedule).
     // The child's front (d = 0) or back (d = 1) completion times come from
     // one lane-parallel chain scan (lane = machine, as a stack push) and go
-    // to the wave's LDS scratch, where the pair lanes read them.
-    __device__ __forceinline__ int lb2_child(int c, int d, uint64_t rowmask, int k)
+    // to the wave's LDS scratch, where the pair lanes read them: fs the front
+    // times, gs the back times plus the child's remaining work.
+    __device__ __forceinline__ int lb2_child(int c, int d, int k)
     {
         const int cj = flag_abs(rdlane(rowv, c));
-        int *fs = lds.scr, *bs = lds.scr + 32;
+        int *fs = lds.scr, *gs = lds.scr + 32;
+        const int pc = pmach(cj);
         if (d == 0) {
-            const int f = ftop;
-            const int cf = chain_scan(f, pmach(cj));
+            const int cf = chain_scan(ftop, pc);
             if (lane < M) {
                 fs[lane] = cf;
-                bs[lane] = brow(nb)[lane];
+                gs[lane] = brow(nb)[lane] + remv - pc;
             }
         } else {
             // back chain over machines M-1..0: lane q handles machine M-1-q
             const int base = lane < M ? brow(nb)[M - 1 - lane] : 0;
             const int pr = lane < M ? lds.pmR[lane * PM_STRIDE + cj] : 0;
+            const int rr = shfl(remv, lane < M ? M - 1 - lane : lane) - pr;
             const int cb = chain_scan(base, pr);
             if (lane < M) {
                 fs[lane] = ftop;
-                bs[M - 1 - lane] = cb;
+                gs[M - 1 - lane] = cb + rr;
             }
         }
         __builtin_amdgcn_wave_barrier();
         int r;
         if (k <= 2) {
-            // l2 - l1 <= 2: makespan of the completed permutation (bound_fsp_strong.cpp:543-546)
-            const int other = flag_abs(rdlane(rowv, 1 - c));
+            // l2 - l1 <= 2: makespan of the completed permutation (bound_fsp_strong.cpp:543-546);
+            // the other job is all the remaining work
+            const int po = pmach(flag_abs(rdlane(rowv, 1 - c)));
             const int fq = lane < M ? fs[lane] : 0;
-            const int bq = lane < M ? bs[lane] : 0;
-            const int cc = chain_scan(fq, pmach(other));
-            r = wave_max(lane < M ? cc + bq : 0);
+            const int gq = lane < M ? gs[lane] : 0;
+            const int cc = chain_scan(fq, po);
+            r = wave_max(lane < M ? cc + gq - po : 0);
         } else {
-            const uint64_t unsched = rowmask & ~(1ull << cj);
-            r = lb2_pairs_any<PCH>(pinfo, lds.jtl, lds.jtabL, lds.jtabG, n, fs, bs, unsched);
+            r = lb2_pairs_any<PCH>(pinfo, lds.jtl, lds.jtabL, lds.jtabG, lds.jpacked, n, ir.npairs, fs, gs,
+                                   free_jobs & ~(1ull << cj));
         }
         __builtin_amdgcn_wave_barrier();
         return r;
@@ -697,13 +694,12 @@ struct Explorer {
             int v = lb1p_child(d, job, chF, chB);
             return todo ? v : 0;
         }
-        uint64_t rowmask = row_jobs(valid, job);
         int cs = 0;
         uint64_t m = tmask;
         while (m) {
             int c = __ffsll((unsigned long long)m) - 1;
             m &= m - 1;
-            int v = lb2_child(c, d, rowmask, k);
+            int v = lb2_child(c, d, k);
             if (lane == c) cs = v;
         }
         return cs;
@@ -722,11 +718,10 @@ struct Explorer {
             csB = valid ? lb1p_child(1, job, chF, chB) : 0;
             return;
         }
-        uint64_t rowmask = row_jobs(valid, job);
         csF = csB = 0;
         for (int c = 0; c < k; c++) {
-            int v0 = lb2_child(c, 0, rowmask, k);
-            int v1 = lb2_child(c, 1, rowmask, k);
+            int v0 = lb2_child(c, 0, k);
+            int v1 = lb2_child(c, 1, k);
             if (lane == c) {
                 csF = v0;
                 csB = v1;
@@ -966,8 +961,10 @@ struct Explorer {
         if (lane < M) frow(nf)[lane] = hi;
         if (lane >= 20 && lane < 20 + M) brow(nb)[lane - 20] = hi;
         remv = lane < M ? lds.tot[lane] : 0;
+        if constexpr (REF == 2) free_jobs = lanes_below(n);
         for (int r = 0; r < L; r++) {
             const int j = rdlane(job, r);
+            if constexpr (REF == 2) free_jobs &= ~(1ull << j);
             *(lane < n - r ? lds.mat + lds_mat_row(r, n) + lane : (int8_t *)(lds.sink + lane)) =
                 (int8_t)mail_path_cell(lane, rdlane(posv, r), j);
             remv -= pmach(j);

@@ -81,11 +81,25 @@ void pbb::build_tables(const int32_t *ptm, int n, int m, HostTables &T)
                 T.jtab[(size_t)p * n + i] = int4{j, ptm[a * n + j], ptm[b * n + j], lag[j]};
             }
         }
+    T.jpacked = *std::max_element(T.ptm.begin(), T.ptm.end()) <= JPACK_MAX;
+    T.jdev.resize(T.jtab.size() * (T.jpacked ? 1 : 2));
+    for (int q = 0; q < T.npairs; q++)
+        for (int i = 0; i < n; i++) {
+            const int4 e = T.jtab[(size_t)q * n + i];
+            const size_t at = (size_t)i * T.npairs + q;
+            if (T.jpacked) {
+                T.jdev[at] = jpack_word(e.x, e.y, e.z, e.w);
+            } else {
+                const int2 v = jpack_pair(e.x, e.y, e.z, e.w);
+                T.jdev[2 * at] = (unsigned)v.x;
+                T.jdev[2 * at + 1] = (unsigned)v.y;
+            }
+        }
 }
 
 struct DevTables {
     int *ptm = nullptr, *ptmT = nullptr, *min_arr = nullptr, *min_dep = nullptr, *pair_ab = nullptr;
-    int4 *jtab = nullptr;
+    void *jtab = nullptr;
     DevInst I{};
 };
 
@@ -96,14 +110,14 @@ static int upload_tables(const HostTables &T, DevTables &D)
     HIPCHK(hipMalloc(&D.min_arr, T.m * 4));
     HIPCHK(hipMalloc(&D.min_dep, T.m * 4));
     HIPCHK(hipMalloc(&D.pair_ab, std::max(1, T.npairs) * 4));
-    HIPCHK(hipMalloc(&D.jtab, std::max<size_t>(1, T.jtab.size()) * sizeof(int4)));
+    HIPCHK(hipMalloc(&D.jtab, std::max<size_t>(1, T.jtab.size()) * 8));  // either form
     HIPCHK(hipMemcpy(D.ptm, T.ptm.data(), T.ptm.size() * 4, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(D.ptmT, T.ptmT.data(), T.ptmT.size() * 4, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(D.min_arr, T.min_arr.data(), T.m * 4, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(D.min_dep, T.min_dep.data(), T.m * 4, hipMemcpyHostToDevice));
     if (T.npairs) {
         HIPCHK(hipMemcpy(D.pair_ab, T.pair_ab.data(), T.npairs * 4, hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(D.jtab, T.jtab.data(), T.jtab.size() * sizeof(int4), hipMemcpyHostToDevice));
+        HIPCHK(hipMemcpy(D.jtab, T.jdev.data(), T.jdev.size() * 4, hipMemcpyHostToDevice));
     }
     D.I.n = T.n;
     D.I.m = T.m;
@@ -115,6 +129,7 @@ static int upload_tables(const HostTables &T, DevTables &D)
     D.I.npairs = T.npairs;
     D.I.pair_ab = D.pair_ab;
     D.I.jtab = D.jtab;
+    D.I.jpacked = T.jpacked ? 1 : 0;
     return PBB_OK;
 }
 
@@ -299,6 +314,7 @@ static hipError_t copy_sync(pbb_engine *e, void *dst, const void *src, size_t by
 static int capacity(pbb_engine *e, int *explorers)
 {
     KArgs a = make_args(e);
+    a.I.jpacked = 1;  // the larger footprint: a retargeted engine keeps its explorers
     int bpc = 0;
     HIPCHK(explore_occupancy(a, &bpc));
     if (bpc < 1) return fail(PBB_E_CAPACITY, "explorer kernel does not fit one workgroup per CU (LDS)");
@@ -382,7 +398,9 @@ extern "C" int pbb_create(const int32_t *ptm, int n, int m, const pbb_config *cf
         const int ref = cfg->bound_mode == 0 ? 0 : (cfg->refine == 1 ? 2 : 1);
         int w = std::min(e->E, team_waves_max(ref));
         if (cfg->team_waves > 0) w = std::min(w, cfg->team_waves);
-        while (w > 0 && team_lds_bytes(e->D.I, lb2, w) > 160 * 1024) w--;
+        DevInst I = e->D.I;
+        I.jpacked = 1;
+        while (w > 0 && team_lds_bytes(I, lb2, w) > 160 * 1024) w--;
         e->team_E = w;
     }
     size_t E = (size_t)e->E;
@@ -785,7 +803,8 @@ static int engine_retarget(pbb_engine *e, const int32_t *ptm, int ub, const int 
     HIPCHK(copy_sync(e, e->D.min_dep, T.min_dep.data(), T.m * 4, hipMemcpyHostToDevice));
     if (T.npairs) {
         HIPCHK(copy_sync(e, e->D.pair_ab, T.pair_ab.data(), T.npairs * 4, hipMemcpyHostToDevice));
-        HIPCHK(copy_sync(e, e->D.jtab, T.jtab.data(), T.jtab.size() * sizeof(int4), hipMemcpyHostToDevice));
+        HIPCHK(copy_sync(e, e->D.jtab, T.jdev.data(), T.jdev.size() * 4, hipMemcpyHostToDevice));
+        e->D.I.jpacked = T.jpacked ? 1 : 0;
     }
     e->inc_cost = ub;
     e->initial_ub = ub;

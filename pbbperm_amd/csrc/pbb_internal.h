@@ -20,6 +20,9 @@ struct HostTables {
     int n, m, mp, npairs;
     std::vector<int> ptm, ptmT, min_arr, min_dep, pair_ab;
     std::vector<int4> jtab;
+    // the device's form of it, job-major (pbb_device.h): packed words or pairs of words
+    bool jpacked;
+    std::vector<unsigned> jdev;
 };
 void build_tables(const int32_t *ptm, int n, int m, HostTables &T);
 int check_device();

@@ -158,7 +158,8 @@ struct RootPerm {
 // fixed odd row stride (lanes reading one job on different machines, or
 // different jobs on one machine, hit distinct banks, and every per-machine
 // offset is a compile-time immediate), min_arr, min_dep, per-machine totals,
-// and the Johnson table npairs*n int4 when LB2 is used and it fits.  Per
+// and the packed Johnson table (n*npairs words) when LB2 is used and it is
+// staged.  Per
 // wavefront: the IVM matrix (row l holds its n-l cells, rows packed), the
 // front/back stack ((n+1) x m ints), the LB1 operand block (2 x m int2) and,
 // for the LB2 variant, 64 ints of scratch, then a 64 x int2 sink for the
@@ -170,7 +171,7 @@ __device__ __host__ inline size_t lds_table_bytes(int n, int m, int npairs, bool
     const int mp = (m + 3) & ~3;
     size_t off = ((size_t)2 * m * PM_STRIDE + 3 * (size_t)mp) * 4;
     off = (off + 15) & ~(size_t)15;
-    if (lb2) off += (size_t)npairs * n * 16;
+    if (lb2) off += ((size_t)npairs * n * 4 + 15) & ~(size_t)15;
     return off;
 }
 // offset of IVM row l (rows 0..l-1 hold n, n-1, ..., n-l+1 cells)
@@ -186,9 +187,13 @@ __device__ __host__ inline size_t lds_wave_bytes(int n, int m, bool scratch)
 {
     return lds_mat_bytes(n) + lds_stack_bytes(n, m) + (size_t)m * 16 + (scratch ? 64 * 4 : 0) + 64 * 8;
 }
-// The Johnson table is staged in LDS when it is at most 64 KB (m <= 10 at
-// n <= 50, m = 20 at n <= 21); larger tables are read from global memory.
-__device__ __host__ inline bool jtab_in_lds(int n, int npairs) { return (size_t)npairs * n * 16 <= 64 * 1024; }
+// The packed Johnson table is staged in LDS when it is at most 24 KB (20
+// machines up to 32 jobs, 13 at any n): the workgroups of the LB2 explorers
+// then stay within a third (engine) and half (20-machine pool) of the CU's LDS,
+// as their registers allow.  Larger ones, and tables of large processing
+// times, are read from global memory (consecutive words per step).
+__device__ __host__ inline bool jtab_in_lds(int n, int npairs) { return (size_t)npairs * n * 4 <= 24 * 1024; }
+__device__ __host__ inline bool jtab_staged(const DevInst &I) { return I.jpacked && jtab_in_lds(I.n, I.npairs); }
 // Explorers (wavefronts) per workgroup of the one-instance engine; they share
 // the workgroup's tables.
 #ifndef PBB_EXPLORE_WAVES
@@ -196,7 +201,7 @@ __device__ __host__ inline bool jtab_in_lds(int n, int npairs) { return (size_t)
 #endif
 inline size_t explore_lds_bytes(const DevInst &I, bool lb2)
 {
-    return lds_table_bytes(I.n, I.m, I.npairs, lb2 && jtab_in_lds(I.n, I.npairs)) +
+    return lds_table_bytes(I.n, I.m, I.npairs, lb2 && jtab_staged(I)) +
            PBB_EXPLORE_WAVES * lds_wave_bytes(I.n, I.m, lb2);
 }
 // The team launch (one workgroup) holds at most 16 explorers with LB1 only
@@ -205,7 +210,7 @@ inline size_t explore_lds_bytes(const DevInst &I, bool lb2)
 __device__ __host__ constexpr int team_waves_max(int ref) { return ref == 0 ? 16 : 8; }
 inline size_t team_lds_bytes(const DevInst &I, bool lb2, int waves)
 {
-    return lds_table_bytes(I.n, I.m, I.npairs, lb2 && jtab_in_lds(I.n, I.npairs)) +
+    return lds_table_bytes(I.n, I.m, I.npairs, lb2 && jtab_staged(I)) +
            (size_t)waves * lds_wave_bytes(I.n, I.m, lb2);
 }
 // LDS size handed to the occupancy query of the persistent kernels.  Their
@@ -265,7 +270,7 @@ struct PoolSlot {                 // device header of one instance slot
     unsigned long long best;      // cost << 32 | explorer
     unsigned long long t_admit;
     int occ;                      // POOL_RUNNING | POOL_DONE | member explorers
-    int n, m, ub, tag, npairs, root_dir, best_cost, improved, status, pad[2];
+    int n, m, ub, tag, npairs, root_dir, best_cost, improved, status, jpacked, pad[1];
     int root_row[PBB_POOL_ROW];
     int perm[PBB_POOL_ROW];
 };
@@ -287,7 +292,7 @@ __device__ __host__ inline PoolLayout pool_layout(int nmax, int M, int pmax, int
     L.minD = o;     o += pool_al((size_t)mp * 4);
     L.pair = o;     o += pool_al((size_t)(pmax > 0 ? pmax : 1) * 4);
     L.key = o;      o += pool_al((size_t)(pmax > 0 ? pmax : 1) * nmax * 4);
-    L.jtab = o;     o += pool_al((size_t)(pmax > 0 ? pmax : 1) * nmax * 16);
+    L.jtab = o;     o += pool_al((size_t)(pmax > 0 ? pmax : 1) * nmax * 8);
     L.idle = o;     o += pool_al((size_t)idle_words_for(members) * IDLE_STRIDE * 8);
     L.member = o;   o += pool_al((size_t)members * 4);
     L.stride = o;
@@ -303,7 +308,7 @@ struct PoolArgs {
     int nmax;                     // largest n served
     int pmax;                     // pair-table capacity
     int idle_words;               // idle mask words per slot (64 members each)
-    int jt_lds;                   // Johnson tables staged in LDS
+    int jt_lds;                   // packed Johnson tables staged in LDS
     int pairs_mode;               // JohnsonMode: pair list built at admission
     int qcap;                     // queue capacity (power of two)
     int sys;                      // req/res/q live in host-mapped memory

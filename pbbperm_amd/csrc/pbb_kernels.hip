@@ -286,16 +286,16 @@ __global__ __launch_bounds__(256) void k_bounds(KArgs a, int which, int count, c
         if (lane == 0) o1[s] = lb;
     } else {
         // bound_fsp_strong::bornes_calculer (bound_fsp_strong.cpp:540-560)
-        uint64_t um = X.row_jobs(valid, job);
-        int *fs = lds.scr, *bs = lds.scr + 32;
+        int *fs = lds.scr, *gs = lds.scr + 32;
         if (lane < M) {
             fs[lane] = X.frow(X.nf)[lane];
-            bs[lane] = X.brow(X.nb)[lane];
+            gs[lane] = X.brow(X.nb)[lane] + X.remv;
         }
         __builtin_amdgcn_wave_barrier();
         int pinfo[Explorer<M, 2>::PCH];
         pair_lanes<Explorer<M, 2>::PCH>(a.I.pair_ab, a.I.npairs, a.I.m, arg, pinfo);
-        int v = lb2_pairs_any<Explorer<M, 2>::PCH>(pinfo, lds.jtl, lds.jtabL, lds.jtabG, a.I.n, fs, bs, um);
+        int v = lb2_pairs_any<Explorer<M, 2>::PCH>(pinfo, lds.jtl, lds.jtabL, lds.jtabG, lds.jpacked, a.I.n,
+                                                   a.I.npairs, fs, gs, X.free_jobs);
         if (lane == 0) o1[s] = v;
     }
 }
@@ -379,7 +379,7 @@ template <int M>
 hipError_t launch_bounds_m(int which, const KArgs &a, int count, const int *perms, const int *l1,
                            const int *l2, int arg, int *o1, int *o2, hipStream_t s)
 {
-    const bool lb2 = which == 2 && jtab_in_lds(a.I.n, a.I.npairs);
+    const bool lb2 = which == 2 && jtab_staged(a.I);
     const size_t lds = lds_table_bytes(a.I.n, a.I.m, a.I.npairs, lb2) + 4 * lds_wave_bytes(a.I.n, a.I.m, true);
     if (const hipError_t err =
             hipFuncSetAttribute((const void *)k_bounds<M>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))

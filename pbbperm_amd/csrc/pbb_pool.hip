@@ -61,7 +61,7 @@ __device__ __forceinline__ PoolSlot *slot_hdr(const PoolArgs &p, int s)
 }
 
 template <int M>
-__device__ __forceinline__ DevInst slot_inst(const PoolArgs &p, int s, int n, int npairs)
+__device__ __forceinline__ DevInst slot_inst(const PoolArgs &p, int s, int n, int npairs, int jpacked)
 {
     char *b = slot_base(p, s);
     DevInst I;
@@ -74,7 +74,8 @@ __device__ __forceinline__ DevInst slot_inst(const PoolArgs &p, int s, int n, in
     I.min_dep = (const int *)(b + p.lay.minD);
     I.npairs = npairs;
     I.pair_ab = (const int *)(b + p.lay.pair);
-    I.jtab = (const int4 *)(b + p.lay.jtab);
+    I.jtab = b + p.lay.jtab;
+    I.jpacked = jpacked;
     return I;
 }
 
@@ -117,17 +118,19 @@ static __device__ __forceinline__ bool pool_admit(const PoolArgs &p, int s, bool
     int *minD = (int *)(b + p.lay.minD);
     int *pair = (int *)(b + p.lay.pair);
     int *key = (int *)(b + p.lay.key);
-    int4 *jtab = (int4 *)(b + p.lay.jtab);
-    int npairs = 0;
+    char *jtab = b + p.lay.jtab;
+    int npairs = 0, big = 0;
     if (lb2 && ok) npairs = p.pairs_mode == 0 ? m * (m - 1) / 2 : m - 1;
     if (ok) {
         for (int i = tid; i < M * n; i += nt) {
             int q = i / n, j = i - q * n;
-            ptm[i] = q < m ? sys_ld_rlx(&R->ptm[q * n + j]) : 0;
+            const int v = q < m ? sys_ld_rlx(&R->ptm[q * n + j]) : 0;
+            ptm[i] = v;
+            big |= v > JPACK_MAX ? 1 : 0;
         }
     }
     __threadfence_block();
-    __syncthreads();
+    const bool jpacked = __syncthreads_or(big) == 0;
     if (ok) {
         for (int i = tid; i < n * mp; i += nt) {
             int j = i / mp, q = i - j * mp;
@@ -189,7 +192,9 @@ static __device__ __forceinline__ bool pool_admit(const PoolArgs &p, int s, bool
         int ab = pair[pi], a = ab & 0xff, c = ab >> 8;
         int lag = 0;
         for (int k = a + 1; k < c; k++) lag += ptm[k * n + j];
-        jtab[pi * n + rank] = make_int4(j, ptm[a * n + j], ptm[c * n + j], lag);
+        const int at = rank * npairs + pi;
+        if (jpacked) ((unsigned *)jtab)[at] = jpack_word(j, ptm[a * n + j], ptm[c * n + j], lag);
+        else ((int2 *)jtab)[at] = jpack_pair(j, ptm[a * n + j], ptm[c * n + j], lag);
     }
     // control block, incumbent, idle mask
     int *ci = (int *)&S->c;
@@ -207,6 +212,7 @@ static __device__ __forceinline__ bool pool_admit(const PoolArgs &p, int s, bool
         S->ub = ub;
         S->tag = tag;
         S->npairs = npairs;
+        S->jpacked = jpacked ? 1 : 0;
         S->best_cost = ub;
         S->improved = 0;
         S->status = ok ? RES_PENDING : RES_INVALID;
@@ -451,7 +457,7 @@ __global__ __launch_bounds__(256, PBB_POOL_MIN_WAVES(M)) void k_pool(KArgs a, Po
                                       __HIP_MEMORY_SCOPE_AGENT);
         } else {
             const int n = uni(ld_rlx(&S->n)), m = uni(ld_rlx(&S->m)), npairs = uni(ld_rlx(&S->npairs));
-            const DevInst I = slot_inst<M>(p, slot, n, npairs);
+            const DevInst I = slot_inst<M>(p, slot, n, npairs, uni(ld_rlx(&S->jpacked)));
             const Lds lds = lds_setup(I, smem, p.jt_lds != 0, REF == 2);
             if (role == ROLE_OWNER) {
                 // a request without an incumbent gets NEH's (ub < 0)
