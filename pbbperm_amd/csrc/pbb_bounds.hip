@@ -1,0 +1,353 @@
+// pbb_bounds.hip -- batched bound_abstract calls over device buffers: LB1 of
+// all children (bound_fsp_weak::boundChildren, bound_fsp_weak.cpp:193-221), LB1'
+// (bornes_calculer, :288-311), Johnson LB2 (bound_fsp_strong.cpp:540-560) and the
+// makespan (evalSolution) of explicit partial schedules (perm, l1, l2): front
+// perm[0..l1], back perm[l2..n-1], the middle unscheduled.
+//
+// A workgroup takes tiles of T schedules, its tables staged once:
+//   1. chains: one lane per schedule and side, its completion times in
+//      registers, so that a job costs 3 instructions per machine for 64 chains
+//      (a wavefront per schedule, lane = machine, pays a prefix scan of 25
+//      dependent instructions per job for one).  Lengths run over 0..n and a
+//      wavefront runs as long as its longest chain, so the tile's 2T chains are
+//      first sorted by length (a counting sort of 64 bins);
+//   2. operands: per schedule and machine the front and back times with the
+//      remaining work folded in, in LDS;
+//   3. the bound: children one lane per child, both directions, over the tile's
+//      children laid end to end (a wavefront per schedule leaves the lanes past
+//      its k children idle, 12 of 64 in use at 50 jobs over all depths); LB2 one
+//      wavefront per schedule, lane = machine pair; the others a lane each.
+// What bounds it: the children are LDS reads (two 8-byte operands and a time per
+// child and machine) and VALU in about equal parts.
+//
+// Translation units: compiled once per machine count M (-DPBB_M=<m>).
+#include "pbb_device.h"
+#include "pbb_kernels.h"
+
+namespace pbb {
+
+enum { B_CHILDREN = 0, B_LB1 = 1, B_LB2 = 2, B_MAKESPAN = 3 };
+
+// jobs of a tile's schedules, one byte each; the odd word stride keeps lanes
+// that read one position of different schedules on distinct banks
+#define BJ_STRIDE 68
+#define B_THREADS 256
+
+struct BoundTile {
+    int2 *U;                 // [T][2M + 1]: front operands, then back operands (machines reversed)
+    uint8_t *jobs;           // [T][BJ_STRIDE]
+    uint64_t *mid;           // [T] unscheduled jobs
+    int *start;              // [T + 1] first child of every schedule among the tile's
+    short *l1, *l2;          // [T]; a malformed schedule has l1 = -2
+    unsigned short *order;   // [2T] chains by decreasing length: schedule << 1 | side
+    int *hist;               // [64] chains per length, then the next place of each
+};
+
+template <int M>
+__device__ __host__ inline size_t bound_tile_bytes(int T)
+{
+    size_t b = (size_t)T * (2 * M + 1) * 8 + (size_t)T * 8 + (size_t)T * BJ_STRIDE;
+    b += (size_t)(T + 1) * 4 + 64 * 4 + (size_t)T * 2 * 4;
+    return (b + 15) & ~(size_t)15;
+}
+
+template <int M>
+__device__ __host__ inline size_t bound_table_bytes(const DevInst &I, bool jtab)
+{
+    size_t b = ((size_t)2 * M * PM_STRIDE + 3 * M) * 4;
+    b = (b + 15) & ~(size_t)15;
+    if (jtab) b += ((size_t)I.npairs * I.n * 4 + 15) & ~(size_t)15;
+    return b;
+}
+
+template <int M, int WHICH>
+__global__ __launch_bounds__(B_THREADS) void k_bounds(DevInst I, int count, int T, const int *perms, const int *l1s,
+                                                      const int *l2s, int arg, int *o1, int *o2)
+{
+    extern __shared__ __align__(16) char smem[];
+    const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
+    const int n = I.n;
+    constexpr int US = 2 * M + 1;
+    const bool jtab = WHICH == B_LB2 && I.jpacked;
+
+    int *pm = (int *)smem, *pmR = pm + M * PM_STRIDE;
+    int *minA = pmR + M * PM_STRIDE, *minD = minA + M, *tot = minD + M;
+    unsigned *jtabL = (unsigned *)(smem + bound_table_bytes<M>(I, false));
+    BoundTile S;
+    S.U = (int2 *)(smem + bound_table_bytes<M>(I, jtab));
+    S.mid = (uint64_t *)(S.U + (size_t)T * US);
+    S.start = (int *)(S.mid + T);
+    S.hist = S.start + T + 1;
+    S.l1 = (short *)(S.hist + 64);
+    S.l2 = S.l1 + T;
+    S.order = (unsigned short *)(S.l2 + T);
+    S.jobs = (uint8_t *)(S.order + 2 * T);
+
+    for (int i = tid; i < n * M; i += B_THREADS) {
+        const int q = i / n, j = i - q * n, v = I.ptm[i];
+        pm[q * PM_STRIDE + j] = v;
+        pmR[(M - 1 - q) * PM_STRIDE + j] = v;
+    }
+    if (tid < M) {
+        minA[tid] = I.min_arr[tid];
+        minD[tid] = I.min_dep[tid];
+    }
+    if (jtab)
+        for (int i = tid; i < I.npairs * n; i += B_THREADS) jtabL[i] = ((const unsigned *)I.jtab)[i];
+    __syncthreads();
+    if (tid < M) {
+        int s = 0;
+        for (int j = 0; j < n; j++) s += pm[tid * PM_STRIDE + j];
+        tot[tid] = s;
+    }
+    constexpr int PCH = (M * (M - 1) / 2 + PBB_WAVE - 1) / PBB_WAVE;
+    int pinfo[PCH];
+    if constexpr (WHICH == B_LB2) pair_lanes<PCH>(I.pair_ab, I.npairs, I.m, arg, pinfo);
+
+    for (long long s0 = (long long)blockIdx.x * T; s0 < count; s0 += (long long)gridDim.x * T) {
+        const int ns = (int)min((long long)T, count - s0);
+        __syncthreads();  // the tables; the last tile's readers are done
+        if (tid < 64) S.hist[tid] = 0;
+        // ids outside 0..n-1 become 63, which is none of them (n <= 63)
+        const int *src = perms + s0 * n;
+        for (int s = wave; s < ns; s += B_THREADS / 64) {
+            const int v = lane < n ? src[(size_t)s * n + lane] : 63;
+            S.jobs[s * BJ_STRIDE + lane] = (uint8_t)((unsigned)v < (unsigned)n ? v : 63);
+        }
+        __syncthreads();
+        // inputs must be permutations of 0..n-1 with -1 <= l1 < l2 <= n;
+        // anything else yields -1 outputs instead of out-of-range table reads
+        for (int s = tid; s < ns; s += B_THREADS) {
+            // the makespan is a chain of all jobs
+            int l1 = n - 1, l2 = n;
+            if constexpr (WHICH != B_MAKESPAN) {
+                l1 = l1s[s0 + s];
+                l2 = l2s[s0 + s];
+            }
+            const uint8_t *js = S.jobs + s * BJ_STRIDE;
+            uint64_t seen = 0ull, mid = 0ull;
+            for (int i = 0; i < n; i++) {
+                const uint64_t bit = 1ull << js[i];
+                seen |= bit;
+                mid |= (i > l1 && i < l2) ? bit : 0ull;
+            }
+            const bool bad = seen != lanes_below(n) || (WHICH != B_MAKESPAN && (l1 < -1 || l2 > n || l1 >= l2));
+            S.mid[s] = bad ? 0ull : mid;
+            S.l1[s] = (short)(bad ? -2 : l1);
+            S.l2[s] = (short)(bad ? n : l2);
+            if constexpr (WHICH != B_MAKESPAN) {
+                atomicAdd(&S.hist[bad ? 0 : l1 + 1], 1);
+                atomicAdd(&S.hist[bad ? 0 : n - l2], 1);
+            } else {
+                S.order[s] = (unsigned short)(2 * s);
+                S.order[ns + s] = (unsigned short)(2 * s + 1);
+            }
+        }
+        __syncthreads();
+        if constexpr (WHICH != B_MAKESPAN) {
+            // places by decreasing length: chains longer than this lane's bin
+            // come before it (lane 0 = the longest)
+            if (wave == 0) {
+                const int c = S.hist[63 - lane];
+                int x = c;
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int y = __shfl_up(x, o, 64);
+                    x += lane >= o ? y : 0;
+                }
+                S.hist[63 - lane] = x - c;
+            }
+            if (WHICH == B_CHILDREN && wave == 1) {
+                int base = 0;
+                for (int b = 0; b < ns; b += 64) {
+                    const int k = b + lane < ns ? __popcll(S.mid[b + lane]) : 0;
+                    int x = k;
+#pragma unroll
+                    for (int o = 1; o < 64; o <<= 1) {
+                        const int y = __shfl_up(x, o, 64);
+                        x += lane >= o ? y : 0;
+                    }
+                    if (b + lane < ns) S.start[b + lane] = base + x - k;
+                    base += __shfl(x, 63, 64);
+                }
+                if (lane == 0) S.start[ns] = base;
+            }
+            __syncthreads();
+            for (int s = tid; s < ns; s += B_THREADS) {
+                const int lf = S.l1[s] < -1 ? 0 : S.l1[s] + 1;
+                S.order[atomicAdd(&S.hist[lf], 1)] = (unsigned short)(2 * s);
+                S.order[atomicAdd(&S.hist[n - S.l2[s]], 1)] = (unsigned short)(2 * s + 1);
+            }
+            __syncthreads();
+        }
+        // chains: front over machines 0..M-1 from min_arr, back over machines
+        // M-1..0 from min_dep (as starting from zero, bound_fsp_weak.cpp:61-110)
+        for (int c = tid; c < 2 * ns; c += B_THREADS) {
+            const int s = S.order[c] >> 1, side = S.order[c] & 1;
+            const int len = side ? n - S.l2[s] : (S.l1[s] < -1 ? 0 : S.l1[s] + 1);
+            const uint8_t *js = S.jobs + s * BJ_STRIDE + (side ? n - 1 : 0);
+            const int *tab = side ? pmR : pm;
+            const int step = side ? -1 : 1;
+            int f[M], w[M];
+#pragma unroll
+            for (int q = 0; q < M; q++) {
+                f[q] = side ? minD[M - 1 - q] : minA[q];
+                w[q] = 0;
+            }
+            for (int i = 0; i < len; i++, js += step) {
+                const int *p = tab + *js;
+                int t = 0;
+#pragma unroll
+                for (int q = 0; q < M; q++) {
+                    const int v = p[q * PM_STRIDE];
+                    t = max(t, f[q]) + v;  // times are not negative: t = 0 before the first machine
+                    f[q] = t;
+                    w[q] += v;
+                }
+            }
+            int2 *u = S.U + (size_t)s * US + side * M;
+#pragma unroll
+            for (int q = 0; q < M; q++) u[q] = make_int2(f[q], w[q]);
+        }
+        __syncthreads();
+        // (f, work in front), (b, work behind) -> (f, r + b), (b, f + r)
+        for (int i = tid; i < ns * M; i += B_THREADS) {
+            const int s = i / M, q = i - s * M;
+            int2 *u = S.U + (size_t)s * US;
+            const int2 x = u[q], y = u[M + M - 1 - q];
+            const int r = tot[q] - x.y - y.y;
+            u[q].y = r + y.x;
+            u[M + M - 1 - q].y = x.x + r;
+        }
+        if constexpr (WHICH == B_CHILDREN) {
+            // jobs that are no children get 0, malformed schedules -1
+            int *r1 = o1 + s0 * n, *r2 = arg ? o2 + s0 * n : nullptr;
+            for (int s = wave; s < ns; s += B_THREADS / 64) {
+                const int v = S.l1[s] < -1 ? -1 : 0;
+                if (lane < n) {
+                    r1[(size_t)s * n + lane] = v;
+                    if (arg) r2[(size_t)s * n + lane] = v;
+                }
+            }
+            __syncthreads();
+            const int kids = S.start[ns];
+            for (int c = tid; c < kids; c += B_THREADS) {
+                // the schedule of child c: the last one that starts at or before it
+                int s = 0, hi = ns;
+                while (hi - s > 1) {
+                    const int h = (s + hi) >> 1;
+                    if (S.start[h] <= c) s = h;
+                    else hi = h;
+                }
+                const int job = S.jobs[s * BJ_STRIDE + S.l1[s] + 1 + (c - S.start[s])];
+                const int2 *u = S.U + (size_t)s * US;
+                int p[M];
+#pragma unroll
+                for (int q = 0; q < M; q++) p[q] = pm[q * PM_STRIDE + job];
+                int t = 0, lb = 0;
+#pragma unroll
+                for (int q = 0; q < M; q++) {
+                    const int2 x = u[q];
+                    t = max(t, x.x);
+                    lb = max(lb, t + x.y);
+                    t += p[q];
+                }
+                r1[(size_t)s * n + job] = lb;
+                if (arg) {
+                    t = lb = 0;
+#pragma unroll
+                    for (int q = 0; q < M; q++) {
+                        const int2 x = u[M + q];
+                        t = max(t, x.x);
+                        lb = max(lb, t + x.y);
+                        t += p[M - 1 - q];
+                    }
+                    r2[(size_t)s * n + job] = lb;
+                }
+            }
+        } else {
+            __syncthreads();
+            // a lane per schedule: LB1' and, where at most one job (LB2) or
+            // none is left, the makespan of the completed permutation
+            // (bound_fsp_strong.cpp:543-546)
+            for (int s = tid; s < ns; s += B_THREADS) {
+                const int2 *u = S.U + (size_t)s * US;
+                const int k = __popcll(S.mid[s]);
+                int v = 0, t = 0;
+                if (S.l1[s] < -1) {
+                    v = -1;
+                } else if (WHICH == B_LB1 && k > 0) {
+                    // t = max over machines up to q of f + r
+#pragma unroll
+                    for (int q = 0; q < M; q++) {
+                        const int2 y = u[M + M - 1 - q];
+                        t = max(t, y.y);
+                        v = max(v, t + y.x);
+                    }
+                } else {
+                    const int *p = pm + (k ? __ffsll((unsigned long long)S.mid[s]) - 1 : 0);
+#pragma unroll
+                    for (int q = 0; q < M; q++) {
+                        const int pq = k ? p[q * PM_STRIDE] : 0;
+                        const int x = u[q].x;
+                        t = k ? max(t, x) + pq : x;
+                        v = max(v, t + u[M + M - 1 - q].x);
+                    }
+                }
+                if (WHICH != B_LB2 || k <= 1) o1[s0 + s] = v;
+            }
+            if constexpr (WHICH == B_LB2) {
+                for (int s = wave; s < ns; s += B_THREADS / 64) {
+                    const uint64_t mid = uni64(S.mid[s]);
+                    if (__popcll(mid) <= 1) continue;
+                    const int *fs = (const int *)(S.U + (size_t)s * US);
+                    const int v = lb2_pairs_any<PCH, 2>(pinfo, jtab, jtabL, I.jtab, false, n, I.npairs, fs, fs + 1, mid);
+                    if (lane == 0) o1[s0 + s] = v;
+                }
+            }
+        }
+    }
+}
+
+// Tile size: up to 128 schedules, as many as leave room for three workgroups
+// per CU beside the tables (two with a Johnson table); a small batch is spread
+// over the CUs in smaller tiles, 16 schedules at least.
+template <int M, int WHICH>
+static hipError_t launch(const DevInst &I, int count, const int *perms, const int *l1, const int *l2, int arg, int *o1,
+                         int *o2, hipStream_t s)
+{
+    const size_t tab = bound_table_bytes<M>(I, WHICH == B_LB2 && I.jpacked);
+    const size_t room = 160 * 1024 / (WHICH == B_LB2 ? 2 : 3) - 2048;
+    int T = WHICH == B_LB2 ? 32 : 128;
+    while (T > 16 && tab + bound_tile_bytes<M>(T) > room) T -= 16;
+    while (T > 16 && (count + T - 1) / T < 512) T -= 16;
+    const size_t lds = tab + bound_tile_bytes<M>(T);
+    if (const hipError_t err = hipFuncSetAttribute((const void *)k_bounds<M, WHICH>,
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
+        return err;
+    const int tiles = (count + T - 1) / T;
+    const int resident = 256 * (int)(160 * 1024 / lds < 8 ? 160 * 1024 / lds : 8);
+    const int grid = tiles < resident ? tiles : resident;
+    hipLaunchKernelGGL((k_bounds<M, WHICH>), dim3(grid), dim3(B_THREADS), lds, s, I, count, T, perms, l1, l2, arg, o1,
+                       o2);
+    return hipGetLastError();
+}
+
+template <int M>
+hipError_t launch_bounds_m(int which, const DevInst &I, int count, const int *perms, const int *l1, const int *l2,
+                           int arg, int *o1, int *o2, hipStream_t s)
+{
+    switch (which) {
+    case B_CHILDREN: return launch<M, B_CHILDREN>(I, count, perms, l1, l2, arg, o1, o2, s);
+    case B_LB1: return launch<M, B_LB1>(I, count, perms, l1, l2, arg, o1, o2, s);
+    case B_LB2: return launch<M, B_LB2>(I, count, perms, l1, l2, arg, o1, o2, s);
+    default: return launch<M, B_MAKESPAN>(I, count, perms, l1, l2, arg, o1, o2, s);
+    }
+}
+
+#ifdef PBB_M
+template hipError_t launch_bounds_m<PBB_M>(int, const DevInst &, int, const int *, const int *, const int *, int, int *,
+                                          int *, hipStream_t);
+#endif
+
+}  // namespace pbb

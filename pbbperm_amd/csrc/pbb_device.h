@@ -209,7 +209,8 @@ __device__ __forceinline__ int job_mask(int e, uint64_t unsched)
 // Johnson LB2 of one partial schedule over the machine pairs of pinfo
 // (bound_fsp_strong.cpp:50-100, :102-162 without early exit, as
 // bornes_calculer calls them, :540-560).  fs: its front completion times;
-// gs: back completion times plus remaining work (both LDS, by machine);
+// gs: back completion times plus remaining work (both LDS, by machine, ST words
+// apart);
 // unsched: the bit set of its unscheduled jobs, not empty.
 //
 // The reference's recurrence over the unscheduled jobs in Johnson order,
@@ -229,7 +230,7 @@ __device__ __forceinline__ int job_mask(int e, uint64_t unsched)
 // (n a multiple of 8).  30x20: 42 us per node of 1.4 bounds before.
 // Each use of it names one table, in LDS or in global memory: a pointer that
 // may be either makes every access a flat load.
-template <int PCH, bool N32, bool PACKED>
+template <int PCH, bool N32, bool PACKED, int ST>
 __device__ __forceinline__ int lb2_pairs(const int (&pinfo)[PCH], const void *jtab, int n, int npairs,
                                          const int *fs, const int *gs, uint64_t unsched)
 {
@@ -239,8 +240,8 @@ __device__ __forceinline__ int lb2_pairs(const int (&pinfo)[PCH], const void *jt
     for (int c = 0; c < PCH; c++) {
         col[c] = min(c * PBB_WAVE + lane, npairs - 1);
         const int ab = pinfo[c] < 0 ? 0 : pinfo[c];
-        D[c] = fs[ab & 0xff];
-        best[c] = fs[ab >> 8];
+        D[c] = fs[(ab & 0xff) * ST];
+        best[c] = fs[(ab >> 8) * ST];
     }
 #pragma unroll 4
     for (int i = 0; i < n; i++) {
@@ -265,7 +266,7 @@ __device__ __forceinline__ int lb2_pairs(const int (&pinfo)[PCH], const void *jt
         const int info = pinfo[c];
         if (info >= 0) {
             const int a = info & 0xff, b = info >> 8;
-            r = max(r, max(best[c] + gs[b], fs[a] + gs[a]));
+            r = max(r, max(best[c] + gs[b * ST], fs[a * ST] + gs[a * ST]));
         }
     }
     return wave_max(r);
@@ -273,16 +274,16 @@ __device__ __forceinline__ int lb2_pairs(const int (&pinfo)[PCH], const void *jt
 
 // lb2_pairs with the packed table staged in LDS, or the packed or the wide one
 // in global memory
-template <int PCH>
+template <int PCH, int ST = 1>
 __device__ __forceinline__ int lb2_pairs_any(const int (&pinfo)[PCH], bool staged, const unsigned *jtabL,
                                              const void *jtabG, bool packed, int n, int npairs, const int *fs,
                                              const int *gs, uint64_t unsched)
 {
     if (staged)
-        return n <= 32 ? lb2_pairs<PCH, true, true>(pinfo, jtabL, n, npairs, fs, gs, unsched)
-                       : lb2_pairs<PCH, false, true>(pinfo, jtabL, n, npairs, fs, gs, unsched);
-    return packed ? lb2_pairs<PCH, false, true>(pinfo, jtabG, n, npairs, fs, gs, unsched)
-                  : lb2_pairs<PCH, false, false>(pinfo, jtabG, n, npairs, fs, gs, unsched);
+        return n <= 32 ? lb2_pairs<PCH, true, true, ST>(pinfo, jtabL, n, npairs, fs, gs, unsched)
+                       : lb2_pairs<PCH, false, true, ST>(pinfo, jtabL, n, npairs, fs, gs, unsched);
+    return packed ? lb2_pairs<PCH, false, true, ST>(pinfo, jtabG, n, npairs, fs, gs, unsched)
+                  : lb2_pairs<PCH, false, false, ST>(pinfo, jtabG, n, npairs, fs, gs, unsched);
 }
 
 }  // namespace pbb

@@ -191,10 +191,7 @@ static int bounds_call(pbb_bounds *b, int which, int count, const int *perms, co
     if (which != 3 && (!l1 || !l2)) return fail(PBB_E_ARG, "null l1/l2");
     if (which == 0 && arg && !o2) return fail(PBB_E_ARG, "null ce with both=1");
     if (count == 0) return PBB_OK;
-    KArgs a{};
-    a.I = b->D.I;
-    a.rows = b->D.I.n;
-    HIPCHK(launch_bounds(which, a, count, perms, l1, l2, arg, o1, o2, (hipStream_t)stream));
+    HIPCHK(launch_bounds(which, b->D.I, count, perms, l1, l2, arg, o1, o2, (hipStream_t)stream));
     return PBB_OK;
 }
 

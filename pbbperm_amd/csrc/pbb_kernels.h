@@ -331,8 +331,10 @@ template <int M> hipError_t launch_explore_m(const KArgs &a, int blocks, hipStre
 template <int M> hipError_t launch_team_m(const KArgs &a, hipStream_t s);
 template <int M> hipError_t occupancy_m(const KArgs &a, int *blocks_per_cu);
 template <int M> hipError_t launch_root_m(const KArgs &a, const RootPerm &root_perm, hipStream_t s);
+
+// batched bounds (pbb_bounds.hip, one translation unit per M)
 template <int M>
-hipError_t launch_bounds_m(int which, const KArgs &a, int count, const int *perms, const int *l1,
+hipError_t launch_bounds_m(int which, const DevInst &I, int count, const int *perms, const int *l1,
                            const int *l2, int arg, int *o1, int *o2, hipStream_t s);
 
 // pool kernels (pbb_pool.hip, one translation unit per M)
@@ -375,7 +377,7 @@ hipError_t launch_prelaunch(const KArgs &a, hipStream_t s);
 // had left already become intervals of the saved state
 hipError_t launch_collect(const KArgs &a, hipStream_t s);
 // which: 0 lb1 children, 1 lb1 node, 2 lb2 node, 3 makespan
-hipError_t launch_bounds(int which, const KArgs &a, int count, const int *perms, const int *l1,
+hipError_t launch_bounds(int which, const DevInst &I, int count, const int *perms, const int *l1,
                          const int *l2, int arg, int *o1, int *o2, hipStream_t s);
 // init_count > 0: batch launch, the queue holds slots 0..init_count-1
 hipError_t launch_pool(int M, const KArgs &a, const PoolArgs &p, int groups, int init_count, hipStream_t s);

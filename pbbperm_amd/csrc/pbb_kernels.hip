@@ -17,9 +17,6 @@
 //                  compile time: 0 LB1 only (boundingMode 0), 1 LB1 + LB1'
 //                  refinement (modes 1/2 as shipped), 2 LB1 + Johnson LB2.
 //   k_bound_root<M> LB1 root bounding, ivm_bound::boundRoot (ivm_bound.cpp:273-330).
-//   k_bounds<M>    batched bound_abstract calls over device buffers, one
-//                  partial schedule per wavefront, on the explorer's own
-//                  routines (LB1 children, LB1', LB2, makespan).
 //
 // Translation units: this file is compiled once per machine count M
 // (-DPBB_M=<m>) so the 19 instantiations build in parallel.
@@ -166,140 +163,6 @@ __global__ __launch_bounds__(64) void k_bound_root(KArgs a, RootPerm root_perm)
     if (X.lane == 0) a.root_dir_out[0] = d0;
 }
 
-// ------------------------------------------------- batched bound_abstract
-// Load an explicit partial schedule (perm, l1, l2) into an explorer's
-// stacks: F <- perm[0..l1] (scheduleFront), B <- perm[l2..n-1] in reverse
-// (scheduleBack), remain <- the middle.  Then the explorer's own routines
-// produce the bounds.  Requires (l1+1) + (n-l2) < n.
-template <int M>
-__device__ __forceinline__ void load_partial(Explorer<M, 2> &X, const int *perm, int l1, int l2)
-{
-    X.reset_stacks();
-    for (int i = 0; i <= l1; i++) X.push_job(uni(perm[i]), 0);
-    for (int i = X.n - 1; i >= l2; i--) X.push_job(uni(perm[i]), 1);
-}
-
-// makespan of perm with perm[mid] the only job between the stacks
-// (front = perm[0..mid-1], back = perm[mid+1..n-1])
-template <int M>
-__device__ __forceinline__ int makespan_mid(Explorer<M, 2> &X, const int *perm, int mid)
-{
-    load_partial<M>(X, perm, mid - 1, mid + 1);
-    return X.makespan_with(uni(perm[mid]));
-}
-
-template <int M>
-__global__ __launch_bounds__(256) void k_bounds(KArgs a, int which, int count, const int *perms,
-                                                const int *l1s, const int *l2s, int arg, int *o1, int *o2)
-{
-    extern __shared__ __align__(16) char smem[];
-    Lds lds = lds_setup(a.I, smem, which == 2, true);
-    const int w = threadIdx.x >> 6;
-    const int s = blockIdx.x * 4 + w;
-    if (s >= count) return;
-    Explorer<M, 2> X(a, lds, 0, engine_inst(a), a.ctl, a.I.n, a.I.mp);
-    const int n = X.n, lane = X.lane;
-    const int *perm = perms + (size_t)s * n;
-    // inputs must be permutations of 0..n-1 with -1 <= l1 < l2 <= n;
-    // anything else yields -1 outputs instead of out-of-range table reads
-    const int pv = lane < n ? perm[lane] : 0;
-    bool bad = ballot(lane < n && (pv < 0 || pv >= n)) != 0ull;
-    int l1 = -1, l2 = n;
-    if (which != 3) {
-        l1 = uni(l1s[s]);
-        l2 = uni(l2s[s]);
-        bad = bad || l1 < -1 || l2 > n || l1 >= l2;
-    }
-    if (!bad) {
-        if (lane < n) lds.scr[lane] = 0;
-        __builtin_amdgcn_wave_barrier();
-        if (lane < n) atomicAdd(&lds.scr[pv], 1);
-        __builtin_amdgcn_wave_barrier();
-        bad = ballot(lane < n && lds.scr[lane] != 1) != 0ull;  // repeated job ids
-        __builtin_amdgcn_wave_barrier();
-    }
-    if (bad) {
-        if (which == 0) {
-            if (lane < n) o1[(size_t)s * n + lane] = -1;
-            if (arg && lane < n) o2[(size_t)s * n + lane] = -1;
-        } else if (lane == 0) {
-            o1[s] = -1;
-        }
-        return;
-    }
-    if (which == 3) {
-        // bound_fsp_weak::evalSolution
-        int v = makespan_mid<M>(X, perm, n - 1);
-        if (lane == 0) o1[s] = v;
-        return;
-    }
-    const int k = l2 - l1 - 1;
-    if (which == 0 && k == 0) {
-        if (lane < n) {
-            o1[(size_t)s * n + lane] = 0;
-            if (arg) o2[(size_t)s * n + lane] = 0;
-        }
-        return;
-    }
-    if ((which == 1 && k == 0) || (which == 2 && k <= 1)) {
-        // nothing (LB1') or at most one job (LB2, bound_fsp_strong.cpp:543-546)
-        // unscheduled: both reduce to the makespan of the completed permutation
-        int v = makespan_mid<M>(X, perm, k == 1 ? l1 + 1 : (l1 >= 0 ? l1 : 0));
-        if (lane == 0) o1[s] = v;
-        return;
-    }
-    load_partial<M>(X, perm, l1, l2);
-    const bool valid = lane < k;
-    const int job = valid ? perm[l1 + 1 + lane] : 0;
-    if (which == 0) {
-        // bound_fsp_weak::boundChildren (bound_fsp_weak.cpp:193-221)
-        X.rowv = job;
-        X.L = n - k;
-        int cb, ce;
-        X.lb1_children(k, cb, ce);
-        int *inv = lds.scr;
-        if (lane < n) inv[pv] = lane;
-        __builtin_amdgcn_wave_barrier();
-        int ci = lane < n ? inv[lane] - (l1 + 1) : -1;
-        bool child = ci >= 0 && ci < k;
-        int vF = shfl(cb, child ? ci : 0);
-        int vB = shfl(ce, child ? ci : 0);
-        if (lane < n) {
-            o1[(size_t)s * n + lane] = child ? vF : 0;
-            if (arg) o2[(size_t)s * n + lane] = child ? vB : 0;
-        }
-    } else if (which == 1) {
-        // bound_fsp_weak::bornes_calculer (bound_fsp_weak.cpp:288-311)
-        int t0 = 0, lb = 0;
-#pragma unroll
-        for (int q = 0; q < M; q++) {
-            int f = X.fval(q), b = X.bval(q), r = X.rval(q);
-            if (q == 0) {
-                t0 = f + r;
-                lb = t0 + b;
-            } else {
-                int t1 = max(f + r, t0);
-                lb = max(lb, t1 + b);
-                t0 = t1;
-            }
-        }
-        if (lane == 0) o1[s] = lb;
-    } else {
-        // bound_fsp_strong::bornes_calculer (bound_fsp_strong.cpp:540-560)
-        int *fs = lds.scr, *gs = lds.scr + 32;
-        if (lane < M) {
-            fs[lane] = X.frow(X.nf)[lane];
-            gs[lane] = X.brow(X.nb)[lane] + X.remv;
-        }
-        __builtin_amdgcn_wave_barrier();
-        int pinfo[Explorer<M, 2>::PCH];
-        pair_lanes<Explorer<M, 2>::PCH>(a.I.pair_ab, a.I.npairs, a.I.m, arg, pinfo);
-        int v = lb2_pairs_any<Explorer<M, 2>::PCH>(pinfo, lds.jtl, lds.jtabL, lds.jtabG, lds.jpacked, a.I.n,
-                                                   a.I.npairs, fs, gs, X.free_jobs);
-        if (lane == 0) o1[s] = v;
-    }
-}
-
 // ---------------------------------------------------------- host launchers
 template <int M>
 static const void *explore_kernel(const KArgs &a)
@@ -375,27 +238,11 @@ hipError_t launch_root_m(const KArgs &a, const RootPerm &root_perm, hipStream_t 
     return hipGetLastError();
 }
 
-template <int M>
-hipError_t launch_bounds_m(int which, const KArgs &a, int count, const int *perms, const int *l1,
-                           const int *l2, int arg, int *o1, int *o2, hipStream_t s)
-{
-    const bool lb2 = which == 2 && jtab_staged(a.I);
-    const size_t lds = lds_table_bytes(a.I.n, a.I.m, a.I.npairs, lb2) + 4 * lds_wave_bytes(a.I.n, a.I.m, true);
-    if (const hipError_t err =
-            hipFuncSetAttribute((const void *)k_bounds<M>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
-        return err;
-    hipLaunchKernelGGL(k_bounds<M>, dim3((count + 3) / 4), dim3(256), lds, s, a, which, count, perms, l1, l2,
-                       arg, o1, o2);
-    return hipGetLastError();
-}
-
 #ifdef PBB_M
 template hipError_t launch_explore_m<PBB_M>(const KArgs &, int, hipStream_t);
 template hipError_t launch_team_m<PBB_M>(const KArgs &, hipStream_t);
 template hipError_t occupancy_m<PBB_M>(const KArgs &, int *);
 template hipError_t launch_root_m<PBB_M>(const KArgs &, const RootPerm &, hipStream_t);
-template hipError_t launch_bounds_m<PBB_M>(int, const KArgs &, int, const int *, const int *, const int *,
-                                          int, int *, int *, hipStream_t);
 #endif
 
 }  // namespace pbb
