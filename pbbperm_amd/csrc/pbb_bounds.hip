@@ -32,6 +32,20 @@ enum { B_CHILDREN = 0, B_LB1 = 1, B_LB2 = 2, B_MAKESPAN = 3 };
 // that read one position of different schedules on distinct banks
 #define BJ_STRIDE 68
 #define B_THREADS 256
+// most schedules per tile
+__host__ __device__ constexpr int b_tile(int which) { return which == B_LB2 ? 32 : 128; }
+
+// inclusive prefix sum over the 64 lanes
+__device__ __forceinline__ int wave_scan(int x)
+{
+    const int lane = lane_id();
+#pragma unroll
+    for (int o = 1; o < PBB_WAVE; o <<= 1) {
+        const int y = shfl(x, lane >= o ? lane - o : lane);
+        x += lane >= o ? y : 0;
+    }
+    return x;
+}
 
 struct BoundTile {
     int2 *U;                 // [T][2M + 1]: front operands, then back operands (machines reversed)
@@ -65,7 +79,7 @@ __global__ __launch_bounds__(B_THREADS) void k_bounds(DevInst I, int count, int 
                                                       const int *l2s, int arg, int *o1, int *o2)
 {
     extern __shared__ __align__(16) char smem[];
-    const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
+    const int tid = threadIdx.x, lane = lane_id(), wave = uni(tid >> 6);
     const int n = I.n;
     constexpr int US = 2 * M + 1;
     const bool jtab = WHICH == B_LB2 && I.jpacked;
@@ -83,10 +97,36 @@ __global__ __launch_bounds__(B_THREADS) void k_bounds(DevInst I, int count, int 
     S.order = (unsigned short *)(S.l2 + T);
     S.jobs = (uint8_t *)(S.order + 2 * T);
 
-    for (int i = tid; i < n * M; i += B_THREADS) {
-        const int q = i / n, j = i - q * n, v = I.ptm[i];
-        pm[q * PM_STRIDE + j] = v;
-        pmR[(M - 1 - q) * PM_STRIDE + j] = v;
+    // The next tile's schedules are loaded while this one is worked on, a row
+    // per wavefront and register: a load per row and a wait for each took most
+    // of the time (50x20: 700 us per million schedules, 473 this way).
+    // Ids outside 0..n-1 become 63, which is none of them (n <= 63).
+    constexpr int ROWS = b_tile(WHICH) / (B_THREADS / 64);
+    int rows[ROWS], pl1 = 0, pl2 = 0;
+    const auto prefetch = [&](long long s0) {
+        const int ns = (int)max(0ll, min((long long)T, count - s0));
+        const int *src = perms + s0 * n;
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            const int t = wave + r * (B_THREADS / 64);
+            if (t < ns) rows[r] = src[(size_t)t * n + min(lane, n - 1)];
+        }
+        if (WHICH != B_MAKESPAN && tid < ns) {
+            pl1 = l1s[s0 + tid];
+            pl2 = l2s[s0 + tid];
+        }
+    };
+    prefetch((long long)blockIdx.x * T);
+
+#pragma unroll
+    for (int r = 0; r < (M + 3) / 4; r++) {
+        const int q = wave + 4 * r;
+        if (q < M) {
+            const int v = I.ptm[q * n + min(lane, n - 1)];
+            if (lane < n) pm[q * PM_STRIDE + lane] = pmR[(M - 1 - q) * PM_STRIDE + lane] = v;
+            const int sum = wave_sum(lane < n ? v : 0);
+            if (lane == 0) tot[q] = sum;
+        }
     }
     if (tid < M) {
         minA[tid] = I.min_arr[tid];
@@ -94,92 +134,85 @@ __global__ __launch_bounds__(B_THREADS) void k_bounds(DevInst I, int count, int 
     }
     if (jtab)
         for (int i = tid; i < I.npairs * n; i += B_THREADS) jtabL[i] = ((const unsigned *)I.jtab)[i];
-    __syncthreads();
-    if (tid < M) {
-        int s = 0;
-        for (int j = 0; j < n; j++) s += pm[tid * PM_STRIDE + j];
-        tot[tid] = s;
-    }
     constexpr int PCH = (M * (M - 1) / 2 + PBB_WAVE - 1) / PBB_WAVE;
     int pinfo[PCH];
     if constexpr (WHICH == B_LB2) pair_lanes<PCH>(I.pair_ab, I.npairs, I.m, arg, pinfo);
+    // the chains of a tile of up to 32 schedules are one wavefront's: no order
+    const bool sorted = WHICH != B_MAKESPAN && T > 32;
 
     for (long long s0 = (long long)blockIdx.x * T; s0 < count; s0 += (long long)gridDim.x * T) {
         const int ns = (int)min((long long)T, count - s0);
-        __syncthreads();  // the tables; the last tile's readers are done
+        __syncthreads();  // the last tile's readers are done
         if (tid < 64) S.hist[tid] = 0;
-        // ids outside 0..n-1 become 63, which is none of them (n <= 63)
-        const int *src = perms + s0 * n;
-        for (int s = wave; s < ns; s += B_THREADS / 64) {
-            const int v = lane < n ? src[(size_t)s * n + lane] : 63;
-            S.jobs[s * BJ_STRIDE + lane] = (uint8_t)((unsigned)v < (unsigned)n ? v : 63);
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            const int t = wave + r * (B_THREADS / 64);
+            if (t < ns) S.jobs[t * BJ_STRIDE + lane] = (uint8_t)(lane < n && (unsigned)rows[r] < (unsigned)n ? rows[r] : 63);
         }
+        int l1 = n - 1, l2 = n;  // the makespan is a chain of all jobs
+        if constexpr (WHICH != B_MAKESPAN) {
+            l1 = pl1;
+            l2 = pl2;
+        }
+        prefetch(s0 + (long long)gridDim.x * T);
         __syncthreads();
         // inputs must be permutations of 0..n-1 with -1 <= l1 < l2 <= n;
         // anything else yields -1 outputs instead of out-of-range table reads
-        for (int s = tid; s < ns; s += B_THREADS) {
-            // the makespan is a chain of all jobs
-            int l1 = n - 1, l2 = n;
-            if constexpr (WHICH != B_MAKESPAN) {
-                l1 = l1s[s0 + s];
-                l2 = l2s[s0 + s];
+        if (tid < ns) {
+            const uint32_t *js = (const uint32_t *)(S.jobs + tid * BJ_STRIDE);
+            uint64_t seen = 0ull;
+            for (int i = 0; i < n; i += 4) {
+                const uint32_t w = js[i >> 2];  // past the jobs: 63
+                seen |= (1ull << (w & 63u)) | (1ull << ((w >> 8) & 63u)) | (1ull << ((w >> 16) & 63u)) |
+                        (1ull << (w >> 24));
             }
-            const uint8_t *js = S.jobs + s * BJ_STRIDE;
-            uint64_t seen = 0ull, mid = 0ull;
-            for (int i = 0; i < n; i++) {
-                const uint64_t bit = 1ull << js[i];
-                seen |= bit;
-                mid |= (i > l1 && i < l2) ? bit : 0ull;
+            const bool bad = (seen & ~(1ull << 63)) != lanes_below(n) || l1 < -1 || l2 > n || l1 >= l2;
+            if constexpr (WHICH == B_LB1 || WHICH == B_LB2) {
+                uint64_t mid = 0ull;
+                if (!bad)
+                    for (int i = l1 + 1; i < l2; i++) mid |= 1ull << S.jobs[tid * BJ_STRIDE + i];
+                S.mid[tid] = mid;
             }
-            const bool bad = seen != lanes_below(n) || (WHICH != B_MAKESPAN && (l1 < -1 || l2 > n || l1 >= l2));
-            S.mid[s] = bad ? 0ull : mid;
-            S.l1[s] = (short)(bad ? -2 : l1);
-            S.l2[s] = (short)(bad ? n : l2);
-            if constexpr (WHICH != B_MAKESPAN) {
+            if (bad) {
+                l1 = -2;
+                l2 = n;
+            }
+            S.l1[tid] = (short)l1;
+            S.l2[tid] = (short)l2;
+            if (sorted) {
                 atomicAdd(&S.hist[bad ? 0 : l1 + 1], 1);
-                atomicAdd(&S.hist[bad ? 0 : n - l2], 1);
+                atomicAdd(&S.hist[n - l2], 1);
             } else {
-                S.order[s] = (unsigned short)(2 * s);
-                S.order[ns + s] = (unsigned short)(2 * s + 1);
+                S.order[tid] = (unsigned short)(2 * tid);
+                S.order[ns + tid] = (unsigned short)(2 * tid + 1);
             }
         }
         __syncthreads();
-        if constexpr (WHICH != B_MAKESPAN) {
-            // places by decreasing length: chains longer than this lane's bin
-            // come before it (lane 0 = the longest)
-            if (wave == 0) {
-                const int c = S.hist[63 - lane];
-                int x = c;
-#pragma unroll
-                for (int o = 1; o < 64; o <<= 1) {
-                    const int y = __shfl_up(x, o, 64);
-                    x += lane >= o ? y : 0;
-                }
-                S.hist[63 - lane] = x - c;
-            }
-            if (WHICH == B_CHILDREN && wave == 1) {
-                int base = 0;
-                for (int b = 0; b < ns; b += 64) {
-                    const int k = b + lane < ns ? __popcll(S.mid[b + lane]) : 0;
-                    int x = k;
-#pragma unroll
-                    for (int o = 1; o < 64; o <<= 1) {
-                        const int y = __shfl_up(x, o, 64);
-                        x += lane >= o ? y : 0;
-                    }
-                    if (b + lane < ns) S.start[b + lane] = base + x - k;
-                    base += __shfl(x, 63, 64);
-                }
-                if (lane == 0) S.start[ns] = base;
-            }
-            __syncthreads();
-            for (int s = tid; s < ns; s += B_THREADS) {
-                const int lf = S.l1[s] < -1 ? 0 : S.l1[s] + 1;
-                S.order[atomicAdd(&S.hist[lf], 1)] = (unsigned short)(2 * s);
-                S.order[atomicAdd(&S.hist[n - S.l2[s]], 1)] = (unsigned short)(2 * s + 1);
-            }
-            __syncthreads();
+        // places by decreasing length: chains longer than this lane's bin come
+        // before it (lane 0 = the longest)
+        if (sorted && wave == 0) {
+            const int c = S.hist[63 - lane];
+            S.hist[63 - lane] = wave_scan(c) - c;
         }
+        if (WHICH == B_CHILDREN && wave == 1) {
+            int base = 0;
+            for (int b = 0; b < ns; b += 64) {
+                const int t = b + lane;
+                const int k = t < ns && S.l1[t] >= -1 ? S.l2[t] - S.l1[t] - 1 : 0;
+                const int x = wave_scan(k);
+                if (t < ns) S.start[t] = base + x - k;
+                base += rdlane(x, 63);
+            }
+            if (lane == 0) S.start[ns] = base;
+        }
+        if (sorted) {
+            __syncthreads();
+            if (tid < ns) {
+                S.order[atomicAdd(&S.hist[l1 < -1 ? 0 : l1 + 1], 1)] = (unsigned short)(2 * tid);
+                S.order[atomicAdd(&S.hist[n - l2], 1)] = (unsigned short)(2 * tid + 1);
+            }
+        }
+        __syncthreads();
         // chains: front over machines 0..M-1 from min_arr, back over machines
         // M-1..0 from min_dep (as starting from zero, bound_fsp_weak.cpp:61-110)
         for (int c = tid; c < 2 * ns; c += B_THREADS) {
@@ -188,21 +221,31 @@ __global__ __launch_bounds__(B_THREADS) void k_bounds(DevInst I, int count, int 
             const uint8_t *js = S.jobs + s * BJ_STRIDE + (side ? n - 1 : 0);
             const int *tab = side ? pmR : pm;
             const int step = side ? -1 : 1;
-            int f[M], w[M];
+            int f[M], w[M], v[M];
 #pragma unroll
             for (int q = 0; q < M; q++) {
                 f[q] = side ? minD[M - 1 - q] : minA[q];
                 w[q] = 0;
             }
-            for (int i = 0; i < len; i++, js += step) {
-                const int *p = tab + *js;
+            // the next job's times are read before this one's are used (one
+            // past the chain: any byte, kept inside the table and unused)
+            int next = js[step] & 63;
+            {
+                const int *p = tab + js[0];
+#pragma unroll
+                for (int q = 0; q < M; q++) v[q] = p[q * PM_STRIDE];
+            }
+            for (int i = 0; i < len; i++) {
+                const int *p = tab + next;
+                js += step;
+                next = js[step] & 63;
                 int t = 0;
 #pragma unroll
                 for (int q = 0; q < M; q++) {
-                    const int v = p[q * PM_STRIDE];
-                    t = max(t, f[q]) + v;  // times are not negative: t = 0 before the first machine
+                    t = max(t, f[q]) + v[q];  // times are not negative: t = 0 before the first machine
                     f[q] = t;
-                    w[q] += v;
+                    w[q] += v[q];
+                    v[q] = p[q * PM_STRIDE];
                 }
             }
             int2 *u = S.U + (size_t)s * US + side * M;
@@ -272,7 +315,7 @@ __global__ __launch_bounds__(B_THREADS) void k_bounds(DevInst I, int count, int 
             // (bound_fsp_strong.cpp:543-546)
             for (int s = tid; s < ns; s += B_THREADS) {
                 const int2 *u = S.U + (size_t)s * US;
-                const int k = __popcll(S.mid[s]);
+                const int k = WHICH == B_MAKESPAN ? 0 : __popcll(S.mid[s]);
                 int v = 0, t = 0;
                 if (S.l1[s] < -1) {
                     v = -1;
@@ -318,7 +361,7 @@ static hipError_t launch(const DevInst &I, int count, const int *perms, const in
 {
     const size_t tab = bound_table_bytes<M>(I, WHICH == B_LB2 && I.jpacked);
     const size_t room = 160 * 1024 / (WHICH == B_LB2 ? 2 : 3) - 2048;
-    int T = WHICH == B_LB2 ? 32 : 128;
+    int T = b_tile(WHICH);
     while (T > 16 && tab + bound_tile_bytes<M>(T) > room) T -= 16;
     while (T > 16 && (count + T - 1) / T < 512) T -= 16;
     const size_t lds = tab + bound_tile_bytes<M>(T);
