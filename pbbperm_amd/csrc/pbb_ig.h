@@ -6,12 +6,18 @@
 //
 // A chain's sequences are lane vectors (lane = position).  Every move is
 // evaluated with the heads and tails of the current sequence
-// (fastInsertRemove's computeHeads / computeTails), computed by a systolic
-// pass over the lanes: at step t lane j advances position j to machine t - j
-// (heads) taking its left neighbour's value of the step before through DPP,
-// and likewise from the right for the tails, so one pass costs n + M - 1
-// steps.  The makespans of inserting a job before every position, or of
-// removing every position, then take M steps with one lane per position.
+// (fastInsertRemove's computeHeads / computeTails), one machine per step: over
+// the positions, a machine's heads are a prefix sum and a prefix max in lane
+// order (the form of chain_scan with positions for machines), and its tails the
+// same from the other end.  Up to 32 jobs both run in one pass, heads in
+// lanes 0-31 and tails in lanes 32-63.  The makespans of inserting a job before
+// every position, or of removing every position, then take M steps with one
+// lane per position.
+//
+// A chain is one wavefront on its SIMD, so what bounds it is the latency of
+// these passes.  The former systolic pass (lane j on machine t - j at step
+// t) took n + M - 1 steps with an LDS read and two stores each: 16 instances of
+// up to 30x20, 64 chains of 20 rounds, IG_BEFORE ms against IG_AFTER ms.
 //
 // The reference seeds its generators from std::random_device and accepts
 // worse solutions through a float exp; a chain here draws from its own
@@ -55,12 +61,16 @@ __device__ __forceinline__ int ig_visit(int n, int i)
     return (i & 1) ? start - 1 - (i >> 1) : start + (i >> 1);
 }
 
-// inclusive prefix sum over all 64 lanes
+// inclusive prefix sum / max over all 64 lanes
 __device__ __forceinline__ int scan_add64(int x)
 {
     x = scan_add32(x);
-    const int lo = rdlane(x, 31);
-    return lane_id() >= 32 ? x + lo : x;
+    return x + __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);
+}
+__device__ __forceinline__ int scan_max64(int x)
+{
+    x = scan_max32(x);
+    return max(x, __builtin_amdgcn_update_dpp((int)0x80000000, x, 0x143, 0xC, 0xF, false));
 }
 
 // lane i takes lane i+1 (lane 63: 0) / lane i-1 (lane 0: 0)
@@ -84,52 +94,66 @@ template <int M>
 struct IgWave {
     const int *pm;   // [M][PM_STRIDE] machine-major times (zero rows beyond the instance's m)
     const int *spt;  // [64] total time of each job
-    int *hd, *tl;    // [M][64] heads / tails of the current sequence
+    int *hd, *tl;    // [M][64] heads (up to 32 jobs: heads and tails) / tails of the current sequence
     int *scr;        // 64 ints of scratch
     int n, lane;
 
-    // computeHeads + computeTails (fastinsertremove.cpp:75-116) of the
-    // sequence in v, positions 0..len-1; returns its makespan
-    __device__ __forceinline__ int heads_tails(int v, int len) const
+    // One side of computeHeads / computeTails (fastinsertremove.cpp:75-116): lane
+    // vectors of the positions in scan order, `in` where the lane has one (the
+    // others come before all positions, or after them, and are zero), p the
+    // lane's job on the first machine of the side.  Stores every machine's
+    // values to out[s * 64 + lane]; returns the last machine's.
+    template <bool WIDE>
+    __device__ __forceinline__ int side(bool in, const int *p, int step, int *out) const
     {
-        const bool in = lane < len;
-        const int job = in ? v : 0;
-        int h = 0, q = 0;
-        const int steps = len + M - 1;
-        for (int t = 0; t < steps; t++) {
-            const int k = t - lane;                       // heads: machine of this position
-            const int kt = M - 1 - (t - (len - 1 - lane));  // tails: machine of this position
-            const int left = from_left(h);
-            const int right = from_right(q);
-            const bool dh = in && k >= 0 && k < M;
-            const bool dt = in && kt >= 0 && kt < M;
-            const int ph = dh ? pm[k * PM_STRIDE + job] : 0;
-            const int pt = dt ? pm[kt * PM_STRIDE + job] : 0;
-            if (dh) {
-                h = max(h, left) + ph;
-                hd[k * 64 + lane] = h;
-            }
-            if (dt) {
-                q = max(q, right) + pt;
-                tl[kt * 64 + lane] = q;
-            }
+        int h = 0;
+#pragma unroll
+        for (int s = 0; s < M; s++) {
+            const int t = in ? p[0] : 0;
+            p += step;
+            const int P = WIDE ? scan_add64(t) : scan_add32(t);
+            const int b = h - (P - t);
+            h = P + (WIDE ? scan_max64(b) : scan_max32(b));
+            out[s * 64 + lane] = h;
         }
-        __builtin_amdgcn_wave_barrier();
-        return uni(hd[(M - 1) * 64 + len - 1]);
+        return h;
     }
 
-    // insertMakespans (fastinsertremove.cpp:196-214): lane i <= len, the
+    // computeHeads + computeTails of the sequence in v, positions 0..len-1;
+    // returns its makespan.  Heads of position j on machine k at
+    // hd[k * 64 + j], tails at tails()[(M - 1 - k) * 64 + 63 - j] (zero at j = len
+    // < n).
+    __device__ __forceinline__ int heads_tails(int v, int len) const
+    {
+        __builtin_amdgcn_wave_barrier();
+        const bool up = lane >= 32;
+        const int rpos = 63 - lane, rjob = shfl(v, rpos);
+        constexpr int last = (M - 1) * PM_STRIDE;
+        int h;
+        if (n <= 32) {
+            const bool in = (up ? rpos : lane) < len;
+            const int job = in ? (up ? rjob : v) : 0;
+            h = side<false>(in, pm + (up ? last : 0) + job, up ? -PM_STRIDE : PM_STRIDE, hd);
+        } else {
+            h = side<true>(lane < len, pm + (lane < len ? v : 0), PM_STRIDE, hd);
+            side<true>(rpos < len, pm + last + (rpos < len ? rjob : 0), -PM_STRIDE, tl);
+        }
+        __builtin_amdgcn_wave_barrier();
+        return rdlane(h, len - 1);
+    }
+    __device__ __forceinline__ const int *tails() const { return n <= 32 ? hd : tl; }
+
+    // insertMakespans (fastinsertremove.cpp:196-214): lane i <= len < n, the
     // makespan with job inserted before position i (zero tail at the end)
     __device__ __forceinline__ int insert_eval(int len, int job) const
     {
-        const int i = lane;
+        const int *h = hd + (lane > 0 ? lane - 1 : 0), *t = tails() + 63 - lane;
+        const int first = lane > 0 ? -1 : 0;
         int e = 0, mk = 0;
 #pragma unroll
         for (int k = 0; k < M; k++) {
-            const int hp = (i > 0 && i <= len) ? hd[k * 64 + i - 1] : 0;
-            const int tv = i < len ? tl[k * 64 + i] : 0;
-            e = max(e, hp) + pm[k * PM_STRIDE + job];
-            mk = max(mk, e + tv);
+            e = max(e, h[k * 64] & first) + pm[k * PM_STRIDE + job];
+            mk = max(mk, e + t[(M - 1 - k) * 64]);
         }
         return mk;
     }
@@ -138,14 +162,11 @@ struct IgWave {
     // makespan without position i
     __device__ __forceinline__ int remove_eval(int len) const
     {
-        const int i = lane;
+        const int *h = hd + (lane > 0 ? lane - 1 : 0), *t = tails() + 62 - (lane < 63 ? lane : 62);
+        const int first = lane > 0 ? -1 : 0, end = lane + 1 < len ? -1 : 0;
         int mk = 0;
 #pragma unroll
-        for (int k = 0; k < M; k++) {
-            const int hp = (i > 0 && i < len) ? hd[k * 64 + i - 1] : 0;
-            const int tv = (i + 1 < len) ? tl[k * 64 + i + 1] : 0;
-            mk = max(mk, hp + tv);
-        }
+        for (int k = 0; k < M; k++) mk = max(mk, (h[k * 64] & first) + (t[(M - 1 - k) * 64] & end));
         return mk;
     }
 
@@ -188,7 +209,10 @@ struct IgWave {
             if (free_) {
                 const uint32_t s = (uint32_t)spt[job];
                 if (s > 0) {
-                    const uint64_t q = ((uint64_t)(uint32_t)(old - rm) << 8) / s;
+                    // a 64-bit division is a hundred instructions: only where
+                    // the makespan asks for one
+                    const uint32_t gain = (uint32_t)(old - rm);
+                    const uint64_t q = old < (1 << 24) ? (uint64_t)((gain << 8) / s) : ((uint64_t)gain << 8) / s;
                     w = (uint32_t)(q * q);
                 }
             }
@@ -249,6 +273,7 @@ __device__ __forceinline__ int ig_chain(const IgWave<M> &G, uint64_t &rng, const
                                         int *best_seq, const Stop &stop, const Publish &publish)
 {
     const int n = G.n, lane = G.lane;
+    rng = uni64(rng);  // one stream per wavefront: its arithmetic is scalar
     // NEH start (runIG calls runNEH on its subproblem, IG.cpp:357)
     int curcost = neh_wave<M>(G.pm, PM_STRIDE, n, G.scr);
     int cur = lane < n ? G.scr[lane] : 0;

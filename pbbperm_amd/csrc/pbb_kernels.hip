@@ -123,7 +123,7 @@ __device__ __forceinline__ void explore_loop(const KArgs &a, const Lds &lds, int
 }
 
 template <int M, int REF>
-__global__ __launch_bounds__(64 * PBB_EXPLORE_WAVES, REF == 0 ? PBB_EXPLORE_MIN_WAVES : 1) void k_explore(KArgs a)
+__global__ __launch_bounds__(64 * PBB_EXPLORE_WAVES, REF == 0 ? PBB_EXPLORE_MIN_WAVES : 3) void k_explore(KArgs a)
 {
     extern __shared__ __align__(16) char smem[];
     Lds lds = lds_setup(a.I, smem, REF == 2, REF == 2);

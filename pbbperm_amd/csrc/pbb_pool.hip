@@ -410,7 +410,7 @@ __device__ __forceinline__ void pool_ig_helper(const Lds &lds, int n, int e, con
 // budget): 3 up to 10 machines (168 VGPRs: the 10-machine LB2 pool would
 // otherwise take 169-176 and drop to 2 waves per SIMD), free above.
 #ifndef PBB_POOL_MIN_WAVES
-#define PBB_POOL_MIN_WAVES(M) ((M) <= 10 ? 3 : 1)
+#define PBB_POOL_MIN_WAVES(M) ((M) <= 10 ? 3 : 2)
 #endif
 
 template <int M, int REF>
