@@ -1203,7 +1203,8 @@ struct Explorer {
     {
         if (a.node_budget) {
             unsigned long long before = w_add64<SC>(&ir.ctl->dec, (unsigned long long)dec);
-            if (before + dec >= a.node_budget && lane == 0) st_rlx<SC>(&run->stop, 1);
+            const unsigned long long most = local_best < a.initial_ub ? a.node_budget : a.quiet_budget;
+            if (before + dec >= most && lane == 0) st_rlx<SC>(&run->stop, 1);
             dec = 0;
         }
         if (dec >= (1u << 28) || sb >= (1u << 28) || jb >= (1u << 28)) flush_counters();  // 32-bit deltas

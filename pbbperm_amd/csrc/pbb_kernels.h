@@ -50,9 +50,20 @@ __device__ __forceinline__ int mail_path_cell(int i, int p, int j) { return i ==
 
 // A busy explorer of a device-wide launch reads a word of the idle mask every
 // PBB_POLL_EVERY decomposed nodes (power of two), whether or not explorers
-// wait in it.
+// wait in it; with Johnson LB2, whose node takes several times an LB1 node's
+// time, it reads the next word at the next node while it sees explorers
+// waiting.  A poll costs a busy device, a long interval between them a thin
+// tree, whose fan-out takes that long per doubling.  Every 16 / 8 / 4 / 1 nodes:
+// 50x20 LB1 (49.7 M nodes) 29.3 / 29.0 / 30.5 / 45.8 ms, 20x20 LB1 (0.83 M) 4.3 /
+// 3.5 / 3.7 / 4.6 ms; again while explorers wait, 20x20 4.1-4.5 ms.  30x20 LB2
+// without the team phase: every 16 / 8 nodes 9.3 / 5.9 ms, again while explorers
+// wait 3.0 ms.
 #ifndef PBB_POLL_EVERY
-#define PBB_POLL_EVERY 16
+#define PBB_POLL_EVERY 8
+#endif
+// The pool's explorers poll every PBB_POOL_POLL_EVERY nodes.
+#ifndef PBB_POOL_POLL_EVERY
+#define PBB_POOL_POLL_EVERY 16
 #endif
 
 // A busy explorer reloads the shared incumbent every PBB_BEST_EVERY decomposed
@@ -127,7 +138,7 @@ struct KArgs {
     int *state;         // [E]
     unsigned *mtag;     // [E] tag of the last message this explorer consumed
     // mailboxes: a donor hands an interval to an idle explorer as one message
-    // of 64 self-tagged words (pack_mail, pbb_explorer.h)
+    // of 64 self-tagged words (mail_word)
     unsigned long long *mbox;   // [E][64]
     unsigned long long *idle;   // idle mask words, IDLE_STRIDE apart
     int idle_words;
@@ -140,6 +151,7 @@ struct KArgs {
     int *root_dir_out;
     // run control
     unsigned long long node_budget;   // 0 = none
+    unsigned long long quiet_budget;  // the same while the incumbent has not moved from initial_ub
     unsigned long long deadline;      // wall_clock64 ticks, 0 = none
     const int *host_flag;             // host-mapped interrupt flag (may be NULL)
     // configuration

@@ -98,10 +98,10 @@ __device__ __forceinline__ void explore_loop(const KArgs &a, const Lds &lds, int
         // idle-mask poll issued before the node's work so its latency is
         // hidden; none while the ramp holds this explorer's work back.  In
         // the workgroup team (at most 16 explorers, workgroup-scope atomics)
-        // a donor that saw explorers waiting polls again at the next node; at
-        // device scope it polls every PBB_POLL_EVERY nodes only.
-        constexpr bool team = SC == __HIP_MEMORY_SCOPE_WORKGROUP;
-        const bool poll = X.since >= a.ramp && ((team && hungry) || (iter & (PBB_POLL_EVERY - 1)) == 0u);
+        // and with LB2 a donor that saw explorers waiting polls again at the
+        // next node (PBB_POLL_EVERY).
+        constexpr bool eager = SC == __HIP_MEMORY_SCOPE_WORKGROUP || REF == 2;
+        const bool poll = X.since >= a.ramp && ((eager && hungry) || (iter & (PBB_POLL_EVERY - 1)) == 0u);
         unsigned long long idle = 0ull;
         if (poll) idle = X.peek_idle();
         const bool refresh = (iter & (PBB_BEST_EVERY - 1)) == 0u;

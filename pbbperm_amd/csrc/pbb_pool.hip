@@ -548,7 +548,7 @@ __global__ __launch_bounds__(256, PBB_POOL_MIN_WAVES(M)) void k_pool(KArgs a, Po
                     }
                     if (leave) break;
                 }
-                const bool poll = (iter & (PBB_POLL_EVERY - 1)) == 0u;
+                const bool poll = (iter & (PBB_POOL_POLL_EVERY - 1)) == 0u;
                 unsigned long long idle = 0ull;
                 if (poll) idle = X.peek_idle();
                 const bool refresh = (iter & (PBB_BEST_EVERY - 1)) == 0u;
