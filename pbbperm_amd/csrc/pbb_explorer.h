@@ -127,6 +127,8 @@ struct Lds {
     unsigned *jtabL;    // packed Johnson table staged in LDS (valid when jtl)
     const void *jtabG;  // the table in global memory
     bool jtl, jpacked;
+    int nch;        // chunks of 64 pairs (jtwalk)
+    bool jtwalk;    // jtabL holds lb2_walk's words (up to 32 jobs)
     int8_t *mat;    // this wave's IVM matrix, row l at mat + lds_mat_row(l, n)
     int *stk;       // this wave's stacks: F entry s at row s, B entry s at row n-s ((n+1) x m)
     int2 *U;        // this wave's LB1 operand block [2][m]
@@ -153,6 +155,8 @@ __device__ __forceinline__ Lds lds_setup(const DevInst &I, char *smem, bool load
     L.jpacked = I.jpacked != 0;
     L.jtabG = I.jtab;
     L.jtl = load_jtab;
+    L.nch = jtab_chunks(I.npairs);
+    L.jtwalk = load_jtab && n <= 32;
     char *wbase = smem + lds_table_bytes(n, m, I.npairs, load_jtab) +
                   (size_t)(threadIdx.x >> 6) * lds_wave_bytes(n, m, scratch);
     L.mat = (int8_t *)wbase;
@@ -173,8 +177,21 @@ __device__ __forceinline__ Lds lds_setup(const DevInst &I, char *smem, bool load
             for (int j = 0; j < n; j++) s += I.ptm[i * n + j];
         L.tot[i] = s;
     }
-    if (load_jtab)
+    if (L.jtwalk) {
+        // a thread per column; the columns past the last pair repeat it
+        const unsigned *src = (const unsigned *)I.jtab;
+        const int width = 64 * L.nch;
+        for (int c = threadIdx.x; c < width; c += blockDim.x) {
+            const int p = min(c, I.npairs - 1);
+#pragma unroll 4
+            for (int i = 0; i < n; i++) L.jtabL[i * width + c] = jwalk_word(src[i * I.npairs + p]);
+#pragma unroll 4
+            for (int i = 0; i < n; i++)
+                atomicOr(&L.jtabL[(int)(src[i * I.npairs + p] & 63u) * width + c], (unsigned)i << 16);
+        }
+    } else if (load_jtab) {
         for (int i = threadIdx.x; i < I.npairs * n; i += blockDim.x) L.jtabL[i] = ((const unsigned *)I.jtab)[i];
+    }
     __syncthreads();
     return L;
 }
@@ -282,6 +299,7 @@ struct Explorer {
     int ftop;                         // lane q < M: top front entry f_q (frow(nf)), else 0
     static constexpr int PCH = (M * (M - 1) / 2 + PBB_WAVE - 1) / PBB_WAVE;  // pair chunks (M >= 2)
     int pinfo[PCH];                   // this lane's Johnson machine pairs (REF 2)
+    unsigned places[PCH];             // unscheduled jobs by their places in the pairs' orders (REF 2, lds.jtwalk)
     int local_best;
     unsigned dec, leaves, sb, jb;     // deltas since the last flush
     unsigned mtag;                    // lane i: tag of word i of the last message consumed
@@ -304,6 +322,8 @@ struct Explorer {
         nf = nb = 0;
         ftop = 0;
         free_jobs = 0ull;
+#pragma unroll
+        for (int c = 0; c < PCH; c++) places[c] = 0u;
         if constexpr (REF == 2) pair_lanes<PCH>(r.pair_ab, r.npairs, r.m, r.pairs_mode, pinfo);
         dec = leaves = sb = jb = 0;
         since = 0;
@@ -339,6 +359,31 @@ struct Explorer {
         return lane < M ? v : 0;
     }
 
+    // job j's bit in the place masks: one LDS word per chunk, kept up along the
+    // path (rebuilt for every node, it costs what the shorter walk saves)
+    __device__ __forceinline__ unsigned place_bit(int c, int j) const
+    {
+        return 1u << jwalk_place(lds.jtabL[(j * lds.nch + c) * 64 + lane]);
+    }
+    template <bool ADD>
+    __device__ __forceinline__ void mark_places(int j)
+    {
+        if (!lds.jtwalk) return;
+#pragma unroll
+        for (int c = 0; c < PCH; c++)
+            if (c == 0 || c < lds.nch) {
+                const unsigned b = place_bit(c, j);
+                places[c] = ADD ? places[c] | b : places[c] & ~b;
+            }
+    }
+    // all jobs unscheduled
+    __device__ __forceinline__ void all_free()
+    {
+        free_jobs = lanes_below(n);
+#pragma unroll
+        for (int c = 0; c < PCH; c++) places[c] = (unsigned)free_jobs;
+    }
+
     __device__ __forceinline__ void reset_stacks()
     {
         nf = nb = 0;
@@ -348,7 +393,7 @@ struct Explorer {
             brow(0)[lane] = lds.minD[lane];
         }
         remv = lane < M ? lds.tot[lane] : 0;
-        if constexpr (REF == 2) free_jobs = lanes_below(n);
+        if constexpr (REF == 2) all_free();
         __builtin_amdgcn_wave_barrier();
     }
 
@@ -374,7 +419,10 @@ struct Explorer {
             nb++;
         }
         remv -= pk;
-        if constexpr (REF == 2) free_jobs &= ~(1ull << j);
+        if constexpr (REF == 2) {
+            free_jobs &= ~(1ull << j);
+            mark_places<false>(j);
+        }
         __builtin_amdgcn_wave_barrier();
     }
 
@@ -387,7 +435,10 @@ struct Explorer {
             nb--;
         }
         remv += pmach(j);
-        if constexpr (REF == 2) free_jobs |= 1ull << j;
+        if constexpr (REF == 2) {
+            free_jobs |= 1ull << j;
+            mark_places<true>(j);
+        }
     }
 
     // ivm::beforeEnd (ivm.cpp:152-160): lexicographic pos <= end
@@ -633,50 +684,98 @@ struct Explorer {
         return lb;
     }
 
-    // Johnson LB2 of child c (uniform), direction d
-    // (bound_fsp_strong::bornes_calculer with the child's partial schedule).
-    // The child's front (d = 0) or back (d = 1) completion times come from
-    // one lane-parallel chain scan (lane = machine, as a stack push) and go
-    // to the wave's LDS scratch, where the pair lanes read them: fs the front
-    // times, gs the back times plus the child's remaining work.
-    __device__ __forceinline__ int lb2_child(int c, int d, int k)
+    // Johnson LB2 of children c0 and c1 (uniform; K = 1: of c0 alone), direction d
+    // (bound_fsp_strong::bornes_calculer with the child's partial schedule), to v0
+    // and v1.  Half of the wavefront each: the child's front (d = 0) or back
+    // (d = 1) completion times come from one lane-parallel chain scan (lane =
+    // machine, as a stack push) and go to the wave's LDS, where the pair lanes
+    // read them: fs the front times, gs the back times plus the child's
+    // remaining work (in the sink, where nothing is read).  Then both children
+    // go through the pair lanes together.  Up to 10 machines and 20 jobs the scan,
+    // the LDS round trip and the reduction are more of a child's time than its
+    // walk, and all are latency.
+    template <int K>
+    __device__ __forceinline__ void lb2_children(int d, int c0, int c1, int k, int &v0, int &v1)
     {
-        const int cj = flag_abs(rdlane(rowv, c));
-        int *fs = lds.scr, *gs = lds.scr + 32;
-        const int pc = pmach(cj);
+        const int q = lane & 31, qq = min(q, M - 1);
+        const bool up = lane >= 32, in = q < M;
+        const int j0 = flag_abs(rdlane(rowv, c0)), j1 = K == 2 ? flag_abs(rdlane(rowv, c1)) : j0;
+        const int job = up ? j1 : j0;
+        int *fs = lds.scr, *gs = (int *)lds.sink;
+        const int ft = bcast_low_half(ftop), rem = bcast_low_half(remv);
+        int f;  // the child's front time on machine q
         if (d == 0) {
-            const int cf = chain_scan(ftop, pc);
-            if (lane < M) {
-                fs[lane] = cf;
-                gs[lane] = brow(nb)[lane] + remv - pc;
-            }
+            const int v = lds.pm[qq * PM_STRIDE + job], pc = in ? v : 0;
+            f = chain_scan(ft, pc);
+            fs[lane] = f;
+            gs[lane] = brow(nb)[qq] + rem - pc;
         } else {
             // back chain over machines M-1..0: lane q handles machine M-1-q
-            const int base = lane < M ? brow(nb)[M - 1 - lane] : 0;
-            const int pr = lane < M ? lds.pmR[lane * PM_STRIDE + cj] : 0;
-            const int rr = shfl(remv, lane < M ? M - 1 - lane : lane) - pr;
-            const int cb = chain_scan(base, pr);
-            if (lane < M) {
-                fs[lane] = ftop;
-                gs[M - 1 - lane] = cb + rr;
-            }
+            const int b = brow(nb)[M - 1 - qq], v = lds.pmR[qq * PM_STRIDE + job];
+            const int pr = in ? v : 0;
+            const int rr = shfl(rem, M - 1 - qq) - pr;
+            const int cb = chain_scan(in ? b : 0, pr);
+            f = ft;
+            fs[lane] = f;
+            gs[(up ? 32 : 0) + (in ? M - 1 - q : q)] = cb + rr;
         }
         __builtin_amdgcn_wave_barrier();
-        int r;
+        int r[2];
         if (k <= 2) {
             // l2 - l1 <= 2: makespan of the completed permutation (bound_fsp_strong.cpp:543-546);
             // the other job is all the remaining work
-            const int po = pmach(flag_abs(rdlane(rowv, 1 - c)));
-            const int fq = lane < M ? fs[lane] : 0;
-            const int gq = lane < M ? gs[lane] : 0;
-            const int cc = chain_scan(fq, po);
-            r = wave_max(lane < M ? cc + gq - po : 0);
+            const int o0 = flag_abs(rdlane(rowv, 1 - c0)), o1 = K == 2 ? flag_abs(rdlane(rowv, 1 - c1)) : o0;
+            const int v = lds.pm[qq * PM_STRIDE + (up ? o1 : o0)], po = in ? v : 0;
+            const int cc = chain_scan(f, po) + gs[lane] - po;
+            // both halves' values where the reduction below expects them
+            r[0] = up ? 0 : (in ? cc : 0);
+            r[1] = up ? (in ? cc : 0) : 0;
+        } else if (lds.jtwalk) {
+            if (PCH == 1 || lds.nch == 1) walk_children<K, 1>(k - 1, j0, j1, r);
+            else if (PCH == 2 || lds.nch == 2) walk_children<K, PCH < 2 ? PCH : 2>(k - 1, j0, j1, r);
+            else walk_children<K, PCH>(k - 1, j0, j1, r);
         } else {
-            r = lb2_pairs_any<PCH>(pinfo, lds.jtl, lds.jtabL, lds.jtabG, lds.jpacked, n, ir.npairs, fs, gs,
-                                   free_jobs & ~(1ull << cj));
+#pragma unroll
+            for (int i = 0; i < K; i++)
+                r[i] = lb2_pairs_any<PCH>(pinfo, lds.jtl, lds.jtabL, lds.jtabG, lds.jpacked, n, ir.npairs, fs + 32 * i,
+                                          gs + 32 * i, free_jobs & ~(1ull << (i ? j1 : j0)));
         }
+        if (K == 1) r[1] = r[0];
+        const auto h = __builtin_amdgcn_permlane32_swap(r[0], r[1], false, false);
+        const int x = scan_max32(max((int)h[0], (int)h[1]));  // lanes 31 and 63: a child's greatest
+        v0 = rdlane(x, 31);
+        v1 = rdlane(x, 63);
         __builtin_amdgcn_wave_barrier();
-        return r;
+    }
+
+    template <int K, int NCH>
+    __device__ __forceinline__ void walk_children(int cnt, int j0, int j1, int (&r)[2]) const
+    {
+        const int *fs = lds.scr, *gs = (const int *)lds.sink;
+        unsigned pl[K][NCH];
+        int D[K][NCH], best[K][NCH], end[K][NCH];
+#pragma unroll
+        for (int c = 0; c < NCH; c++) {
+            const int info = pinfo[c] < 0 ? 0 : pinfo[c], a = info & 0xff, b = info >> 8;
+#pragma unroll
+            for (int i = 0; i < K; i++) {
+                pl[i][c] = places[c] & ~(1u << jwalk_place(lds.jtabL[((i ? j1 : j0) * NCH + c) * 64 + lane]));
+                D[i][c] = fs[32 * i + a];
+                best[i][c] = fs[32 * i + b];
+                end[i][c] = D[i][c] + gs[32 * i + a];
+            }
+        }
+        lb2_walk<K, NCH>(lds.jtabL, cnt, pl, D, best);
+#pragma unroll
+        for (int i = 0; i < K; i++) {
+            r[i] = 0;
+#pragma unroll
+            for (int c = 0; c < NCH; c++) {
+                const int b = pinfo[c] < 0 ? 0 : pinfo[c] >> 8;
+                const int v = max(best[i][c] + gs[32 * i + b], end[i][c]);
+                r[i] = max(r[i], pinfo[c] < 0 ? 0 : v);
+            }
+        }
     }
 
     // mixed mode (computeStrongBounds, ivm_bound.cpp:141-195): refine the
@@ -697,10 +796,18 @@ struct Explorer {
         int cs = 0;
         uint64_t m = tmask;
         while (m) {
-            int c = __ffsll((unsigned long long)m) - 1;
+            const int c0 = __ffsll((unsigned long long)m) - 1;
             m &= m - 1;
-            int v = lb2_child(c, d, k);
-            if (lane == c) cs = v;
+            int v0, v1;
+            if (m) {
+                const int c1 = __ffsll((unsigned long long)m) - 1;
+                m &= m - 1;
+                lb2_children<2>(d, c0, c1, k, v0, v1);
+                cs = lane == c1 ? v1 : cs;
+            } else {
+                lb2_children<1>(d, c0, c0, k, v0, v1);
+            }
+            cs = lane == c0 ? v0 : cs;
         }
         return cs;
     }
@@ -719,12 +826,14 @@ struct Explorer {
             return;
         }
         csF = csB = 0;
-        for (int c = 0; c < k; c++) {
-            int v0 = lb2_child(c, 0, k);
-            int v1 = lb2_child(c, 1, k);
-            if (lane == c) {
-                csF = v0;
-                csB = v1;
+        for (int c = 0; c < k; c += 2) {
+            const int c1 = min(c + 1, k - 1);
+#pragma unroll
+            for (int d = 0; d < 2; d++) {
+                int v0, v1;
+                lb2_children<2>(d, c, c1, k, v0, v1);
+                int &cs = d ? csB : csF;
+                cs = lane == c ? v0 : (lane == c1 ? v1 : cs);
             }
         }
     }
@@ -961,10 +1070,13 @@ struct Explorer {
         if (lane < M) frow(nf)[lane] = hi;
         if (lane >= 20 && lane < 20 + M) brow(nb)[lane - 20] = hi;
         remv = lane < M ? lds.tot[lane] : 0;
-        if constexpr (REF == 2) free_jobs = lanes_below(n);
+        if constexpr (REF == 2) all_free();
         for (int r = 0; r < L; r++) {
             const int j = rdlane(job, r);
-            if constexpr (REF == 2) free_jobs &= ~(1ull << j);
+            if constexpr (REF == 2) {
+                free_jobs &= ~(1ull << j);
+                mark_places<false>(j);
+            }
             *(lane < n - r ? lds.mat + lds_mat_row(r, n) + lane : (int8_t *)(lds.sink + lane)) =
                 (int8_t)mail_path_cell(lane, rdlane(posv, r), j);
             remv -= pmach(j);

@@ -170,20 +170,29 @@ struct RootPerm {
 // fixed odd row stride (lanes reading one job on different machines, or
 // different jobs on one machine, hit distinct banks, and every per-machine
 // offset is a compile-time immediate), min_arr, min_dep, per-machine totals,
-// and the packed Johnson table (n*npairs words) when LB2 is used and it is
-// staged.  Per
+// and the packed Johnson table when LB2 is used and it is staged.  Per
 // wavefront: the IVM matrix (row l holds its n-l cells, rows packed), the
 // front/back stack ((n+1) x m ints), the LB1 operand block (2 x m int2) and,
 // for the LB2 variant, 64 ints of scratch, then a 64 x int2 sink for the
 // lanes past a row in stores that would otherwise need an exec mask.
 #define PM_STRIDE 65
 __device__ __host__ inline int lds_pm_stride(int) { return PM_STRIDE; }
+// Words of the staged Johnson table: up to 32 jobs rows of a multiple of 64
+// pairs (lb2_walk), above that rows of npairs; not less for a smaller instance
+// in a pool's larger layout.
+__device__ __host__ inline int jtab_chunks(int npairs) { return (npairs + 63) / 64; }
+__device__ __host__ inline size_t jtab_lds_words(int n, int npairs)
+{
+    const size_t walk = (size_t)(n < 32 ? n : 32) * 64 * jtab_chunks(npairs);
+    const size_t rows = n > 32 ? (size_t)n * npairs : 0;
+    return walk > rows ? walk : rows;
+}
 __device__ __host__ inline size_t lds_table_bytes(int n, int m, int npairs, bool lb2)
 {
     const int mp = (m + 3) & ~3;
     size_t off = ((size_t)2 * m * PM_STRIDE + 3 * (size_t)mp) * 4;
     off = (off + 15) & ~(size_t)15;
-    if (lb2) off += ((size_t)npairs * n * 4 + 15) & ~(size_t)15;
+    if (lb2) off += (jtab_lds_words(n, npairs) * 4 + 15) & ~(size_t)15;
     return off;
 }
 // offset of IVM row l (rows 0..l-1 hold n, n-1, ..., n-l+1 cells)
@@ -204,7 +213,7 @@ __device__ __host__ inline size_t lds_wave_bytes(int n, int m, bool scratch)
 // then stay within a third (engine) and half (20-machine pool) of the CU's LDS,
 // as their registers allow.  Larger ones, and tables of large processing
 // times, are read from global memory (consecutive words per step).
-__device__ __host__ inline bool jtab_in_lds(int n, int npairs) { return (size_t)npairs * n * 4 <= 24 * 1024; }
+__device__ __host__ inline bool jtab_in_lds(int n, int npairs) { return jtab_lds_words(n, npairs) * 4 <= 24 * 1024; }
 __device__ __host__ inline bool jtab_staged(const DevInst &I) { return I.jpacked && jtab_in_lds(I.n, I.npairs); }
 // Explorers (wavefronts) per workgroup of the one-instance engine; they share
 // the workgroup's tables.
