@@ -61,7 +61,8 @@ __device__ __forceinline__ int mail_path_cell(int i, int p, int j) { return i ==
 #ifndef PBB_POLL_EVERY
 #define PBB_POLL_EVERY 8
 #endif
-// The pool's explorers poll every PBB_POOL_POLL_EVERY nodes.
+// The pool's explorers poll every PBB_POOL_POLL_EVERY nodes (512-instance batch:
+// every 8 / 16 / 32 / 64 nodes 49 / 49 / 51 / 53 ms).
 #ifndef PBB_POOL_POLL_EVERY
 #define PBB_POOL_POLL_EVERY 16
 #endif
@@ -290,8 +291,7 @@ struct PoolSlot {                 // device header of one instance slot
     Ctl c;
     unsigned long long best;      // cost << 32 | explorer
     unsigned long long t_admit;
-    int occ;                      // POOL_RUNNING | POOL_DONE | member explorers
-    int n, m, ub, tag, npairs, root_dir, best_cost, improved, status, jpacked, pad[1];
+    int n, m, ub, tag, npairs, root_dir, best_cost, improved, status, jpacked;
     int root_row[PBB_POOL_ROW];
     int perm[PBB_POOL_ROW];
 };
@@ -322,6 +322,7 @@ __device__ __host__ inline PoolLayout pool_layout(int nmax, int M, int pmax, int
 
 struct PoolArgs {
     char *arena;                  // nslots x layout.stride
+    int *occ;                     // [nslots] POOL_RUNNING | POOL_DONE | member explorers
     PoolLayout lay;
     int nslots;
     int W;                        // explorers (wavefronts) per workgroup

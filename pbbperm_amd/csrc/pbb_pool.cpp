@@ -120,6 +120,7 @@ static PoolArgs pool_pargs(const pbb_pool *p, bool serve)
 {
     PoolArgs q{};
     q.arena = p->arena;
+    q.occ = (int *)(p->arena + (size_t)p->prm.slots * p->lay.stride);
     q.lay = p->lay;
     q.nslots = p->prm.slots;
     q.W = p->W;
@@ -267,7 +268,8 @@ extern "C" int pbb_pool_create(const pbb_config *cfg, const pbb_pool_params *prm
     p->epi_max = next_pow2(std::max(32, p->epi));
     p->lay = pool_layout(p->nmax, p->M, p->pmax, p->epi_max);
     const size_t S = (size_t)prm->slots, E = (size_t)p->E;
-    HTRY(hipMalloc(&p->arena, S * p->lay.stride));
+    const size_t arena_bytes = S * (p->lay.stride + sizeof(int));
+    HTRY(hipMalloc(&p->arena, arena_bytes));
     HTRY(hipMalloc(&p->mat, E * p->nmax * 64));
     HTRY(hipMalloc(&p->pos, E * 64));
     HTRY(hipMalloc(&p->end, E * 64));
@@ -281,7 +283,7 @@ extern "C" int pbb_pool_create(const pbb_config *cfg, const pbb_pool_params *prm
     HTRY(hipMalloc(&p->req_d, S * sizeof(PoolReq)));
     HTRY(hipMalloc(&p->res_d, S * sizeof(PoolRes)));
     HTRY(hipMalloc(&p->q_d, queue_bytes(p->qcap)));
-    HTRY(hipMemset(p->arena, 0, S * p->lay.stride));
+    HTRY(hipMemset(p->arena, 0, arena_bytes));
     HTRY(hipMemset(p->state, 0, E * 4));
     HTRY(hipMemset(p->mbox, 0, E * 64 * 8));
     HTRY(hipMemset(p->run, 0, sizeof(Ctl)));

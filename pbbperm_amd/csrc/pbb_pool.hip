@@ -87,7 +87,7 @@ __device__ __forceinline__ InstRef slot_ref(const PoolArgs &p, int s, PoolSlot *
     r.idle = (unsigned long long *)(b + p.lay.idle);
     r.idle_words = p.idle_words;
     r.member = (const int *)(b + p.lay.member);
-    r.occ = &S->occ;
+    r.occ = p.occ + s;
     r.ub0 = ub;
     r.best = &S->best;
     r.root_row = S->root_row;
@@ -223,11 +223,34 @@ static __device__ __forceinline__ bool pool_admit(const PoolArgs &p, int s, bool
 }
 
 // -------------------------------------------------------- slot selection
-// Wave 0 of a free workgroup: a new instance from the queue first, else the
-// running slot with the largest surplus of busy over idle explorers (below
-// the per-instance cap), else wait.  Returns the role; *slot receives the slot id
+// Wave 0 of a free workgroup: a new instance from the queue first, else a
+// running slot below the per-instance cap, drawn with its surplus of busy over
+// idle explorers as weight, else wait.  Returns the role; *slot receives the slot id
 // and *base the member index of the group's first wave (members stay until the
 // slot is done, so the indices are dense).
+//
+// Hundreds of groups choose at once (a batch's tail, an idle server).  When all
+// went for the largest surplus they raced for one word, one join per pass over
+// the slots, and the occupancy words lay a slot's arena apart, a cache line
+// each: 60 % of the explorers' time passed here (512-instance batch 86 ms, 49
+// with the draw and the words side by side; weights of the surplus squared or
+// cubed 48-51, capped at 16 52).
+__device__ __forceinline__ unsigned pool_draw(unsigned &x, unsigned k)
+{
+    x ^= x << 13;
+    x ^= x >> 17;
+    x ^= x << 5;
+    return (unsigned)(((unsigned long long)x * k) >> 32);
+}
+// compare-and-swap by lane 0; the word found, to all lanes
+__device__ __forceinline__ int w_cas_old(int *p, int expect, int desired)
+{
+    int e = expect;
+    if (lane_id() == 0)
+        __hip_atomic_compare_exchange_strong(p, &e, desired, __ATOMIC_ACQ_REL, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+    return rdlane(e, 0);
+}
 static __device__ __forceinline__ int pool_pick(const PoolArgs &p, int W, unsigned long long t_end, const int *host_flag, int *slot,
                                                  int *base)
 {
@@ -238,6 +261,8 @@ static __device__ __forceinline__ int pool_pick(const PoolArgs &p, int W, unsign
     // relaxed, with the acquire (an L2 invalidate) taken only by the group
     // that claims a request (512-instance batch: 0.92-1.0 s before, 0.48-0.50
     // s with both and the relaxed idle polls).
+    unsigned rng = (blockIdx.x + 1u) * 0x9E3779B9u ^ (unsigned)uni((int)(unsigned)wall_clock64());
+    int nap = 1;
     for (unsigned it = 0;; it++) {
         if (uni(ld_rlx(&p.run->stop))) return ROLE_EXIT;
         if (t_end && uni64(wall_clock64()) >= t_end) return ROLE_EXIT;
@@ -255,46 +280,63 @@ static __device__ __forceinline__ int pool_pick(const PoolArgs &p, int W, unsign
                 // the queue closed and drained waits while a request is
                 // still being admitted, instead of leaving the launch
                 if (lane == 0)
-                    __hip_atomic_store(&slot_hdr(p, *slot)->occ, W, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(p.occ + *slot, W, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 *base = 0;
                 return ROLE_OWNER;
             }
             continue;
         }
-        int best_score = -1, best_slot = -1, best_occ = 0;
+        int total = 0, take = -1, occ = 0, surplus = 0;
         bool running = false;
         for (int base = 0; base < p.nslots; base += PBB_WAVE) {
             const int s = base + lane;
-            int o = 0, wc = 0;
-            if (s < p.nslots) o = ld_rlx(&slot_hdr(p, s)->occ);
-            const bool live = (o & POOL_RUNNING) && !(o & POOL_DONE);
-            if (live) wc = ld_rlx(&slot_hdr(p, s)->c.work_count);
-            const int mem = o & POOL_MEMBERS;
-            // a slot whose request ran out of time is draining: do not join it
-            const bool stopping = live && ld_rlx(&slot_hdr(p, s)->c.stop) != 0;
-            // more busy than idle members: work is there to be split
-            const bool cand = live && !stopping && mem + W <= p.epi && 2 * wc > mem;
+            const int o = s < p.nslots ? ld_rlx(p.occ + s) : 0;
             running = running || ballot(o != 0) != 0ull;
-            const int sc = cand ? 2 * wc - mem : -1;
-            const int mx = wave_max(sc);
-            if (mx > best_score) {
-                const int l = __ffsll((unsigned long long)ballot(sc == mx)) - 1;
-                best_score = mx;
-                best_slot = base + l;
-                best_occ = rdlane(o, l);
+            const int mem = o & POOL_MEMBERS;
+            const bool room = (o & POOL_RUNNING) && !(o & POOL_DONE) && mem + W <= p.epi;
+            if (!ballot(room)) continue;
+            int more = 0;
+            if (room) {
+                // more busy than idle members: work is there to be split; a slot
+                // whose request ran out of time is draining: do not join it
+                const PoolSlot *S = slot_hdr(p, s);
+                const int wc = ld_rlx(&S->c.work_count), stop = ld_rlx(&S->c.stop);
+                more = stop ? 0 : max(0, 2 * wc - mem);
+            }
+            const int upto = scan_add64(more), sum = rdlane(upto, 63);
+            if (!sum) continue;
+            // one pass: this block of slots replaces the choice so far with
+            // probability sum / (total + sum)
+            total += sum;
+            const int r = (int)pool_draw(rng, (unsigned)total);
+            if (r < sum) {
+                const int l = __ffsll((unsigned long long)ballot(upto > r)) - 1;
+                take = base + l;
+                occ = rdlane(o, l);
+                surplus = rdlane(more, l);
             }
         }
-        if (best_slot >= 0) {
-            if (w_cas((unsigned *)&slot_hdr(p, best_slot)->occ, (unsigned)best_occ, (unsigned)(best_occ + W))) {
-                *slot = best_slot;
-                *base = best_occ & POOL_MEMBERS;
-                return ROLE_HELPER;
+        if (take >= 0) {
+            // another group's join changes the word: try again while there is
+            // work and room beside it
+            for (;;) {
+                const int seen = w_cas_old(p.occ + take, occ, occ + W);
+                if (seen == occ) {
+                    *slot = take;
+                    *base = occ & POOL_MEMBERS;
+                    return ROLE_HELPER;
+                }
+                surplus -= (seen & POOL_MEMBERS) - (occ & POOL_MEMBERS);
+                occ = seen;
+                if (!(occ & POOL_RUNNING) || (occ & POOL_DONE) || (occ & POOL_MEMBERS) + W > p.epi || surplus <= 0) break;
             }
+            nap = 1;
             continue;
         }
         const int closed = uni(sys_ld_rlx(&p.q->closed));
         if (closed && (int)head >= tail && !running) return ROLE_EXIT;
-        __builtin_amdgcn_s_sleep(32);
+        for (int i = 0; i < nap; i++) __builtin_amdgcn_s_sleep(32);
+        if (nap < 4) nap <<= 1;
     }
 }
 
@@ -304,7 +346,7 @@ static __device__ __forceinline__ int pool_pick(const PoolArgs &p, int W, unsign
 // solved, or aborted when its stop word was raised (the request's time
 // budget ran out and its explorers gave their intervals up)
 template <int M, int REF>
-__device__ __forceinline__ void pool_finish(Explorer<M, REF> &X, const KArgs &a, PoolSlot *S)
+__device__ __forceinline__ void pool_finish(Explorer<M, REF> &X, const KArgs &a, PoolSlot *S, int *occ)
 {
     const unsigned long long b =
         __hip_atomic_load(&S->best, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
@@ -321,7 +363,7 @@ __device__ __forceinline__ void pool_finish(Explorer<M, REF> &X, const KArgs &a,
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     if (X.lane == 0) {
         st_rel(&S->c.done, 1);
-        __hip_atomic_fetch_or(&S->occ, (int)POOL_DONE, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_fetch_or(occ, (int)POOL_DONE, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
@@ -330,7 +372,7 @@ static __device__ __forceinline__ void pool_leave(const PoolArgs &p, int s, int 
 {
     const int lane = lane_id();
     PoolSlot *S = slot_hdr(p, s);
-    const int old = w_add(&S->occ, -W);
+    const int old = w_add(p.occ + s, -W);
     if ((old & POOL_MEMBERS) != W) return;
     PoolRes *R = p.res + s;
     const int status = (old & POOL_DONE) ? uni(ld_rlx(&S->status)) : (int)RES_ABORTED;
@@ -348,7 +390,7 @@ static __device__ __forceinline__ void pool_leave(const PoolArgs &p, int s, int 
         sys_st64(&R->t_done, wall_clock64());
     }
     const int tag = uni(ld_rlx(&S->tag));
-    if (lane == 0) __hip_atomic_exchange(&S->occ, 0, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    if (lane == 0) __hip_atomic_exchange(p.occ + s, 0, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
     if (lane == 0) sys_st_rel(&R->tag, tag);
 }
 
@@ -453,7 +495,7 @@ __global__ __launch_bounds__(256, PBB_POOL_MIN_WAVES(M)) void k_pool(KArgs a, Po
         if (!ok) {
             // a malformed request retires at once with RES_INVALID
             if (threadIdx.x == 0)
-                __hip_atomic_exchange(&S->occ, (int)(POOL_RUNNING | POOL_DONE) + W, __ATOMIC_RELEASE,
+                __hip_atomic_exchange(p.occ + slot, (int)(POOL_RUNNING | POOL_DONE) + W, __ATOMIC_RELEASE,
                                       __HIP_MEMORY_SCOPE_AGENT);
         } else {
             const int n = uni(ld_rlx(&S->n)), m = uni(ld_rlx(&S->m)), npairs = uni(ld_rlx(&S->npairs));
@@ -501,7 +543,7 @@ __global__ __launch_bounds__(256, PBB_POOL_MIN_WAVES(M)) void k_pool(KArgs a, Po
             X.join(base + wave);
             int st = ST_IDLE;
             if (igw) {
-                if (X.go_idle()) pool_finish(X, a, S);
+                if (X.go_idle()) pool_finish(X, a, S, p.occ + slot);
             } else if (role == ROLE_OWNER) {
                 if (wave == 0) {
                     // boundRoot: the identity order bounded with LB1 and pruned
@@ -513,12 +555,12 @@ __global__ __launch_bounds__(256, PBB_POOL_MIN_WAVES(M)) void k_pool(KArgs a, Po
                 }
                 __syncthreads();
                 if (threadIdx.x == 0)
-                    __hip_atomic_exchange(&S->occ, (int)POOL_RUNNING + W, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_exchange(p.occ + slot, (int)POOL_RUNNING + W, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
                 if (wave == 0) {
                     if (X.start_root()) {
                         st = ST_ACTIVE;
                     } else if (X.go_idle()) {
-                        pool_finish(X, a, S);
+                        pool_finish(X, a, S, p.occ + slot);
                     }
                 } else {
                     X.register_idle();
@@ -555,7 +597,7 @@ __global__ __launch_bounds__(256, PBB_POOL_MIN_WAVES(M)) void k_pool(KArgs a, Po
                 unsigned long long bw = ~0ull;
                 if (refresh) bw = ld_rlx(&S->best);
                 if (!X.step()) {
-                    if (X.go_idle()) pool_finish(X, a, S);
+                    if (X.go_idle()) pool_finish(X, a, S, p.occ + slot);
                     st = ST_IDLE;
                     continue;
                 }
@@ -564,7 +606,7 @@ __global__ __launch_bounds__(256, PBB_POOL_MIN_WAVES(M)) void k_pool(KArgs a, Po
                     const int sc = X.check_stop_slot(&S->c.stop);
                     if (sc == 1) break;  // the launch stops
                     if (sc == 2) {       // this request stops: release the interval
-                        if (X.go_idle()) pool_finish(X, a, S);
+                        if (X.go_idle()) pool_finish(X, a, S, p.occ + slot);
                         st = ST_IDLE;
                         continue;
                     }
@@ -588,7 +630,7 @@ __global__ void k_pool_init(PoolArgs p, int count)
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int nt = gridDim.x * blockDim.x;
     for (int s = t; s < p.nslots; s += nt) {
-        slot_hdr(p, s)->occ = 0;
+        p.occ[s] = 0;
         if (count > 0) {
             p.res[s].tag = -1;
             p.res[s].status = RES_PENDING;
