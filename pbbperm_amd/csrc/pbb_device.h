@@ -103,61 +103,6 @@ struct DevInst {
     int jpacked;
 };
 
-// ---------------------------------------------------------------------------
-// LB1 of one child per lane (bound_fsp_weak.cpp:133-191).
-// fv/bv/rv: uniform front/back/remain vectors.  pj: the lane's job's
-// processing times.  Writes the front-direction bound to lbF and, when both,
-// the back-direction bound to lbB; chF/chB receive the child's own front
-// (resp. back) completion chain (the values scheduleFront/scheduleBack would
-// compute with the child job appended), which the refinement bounds reuse.
-template <int M>
-__device__ __forceinline__ void lb1_child(const int (&fv)[M], const int (&bv)[M], const int (&rv)[M],
-                                          const int (&pj)[M], bool both, int &lbF, int &lbB,
-                                          int (&chF)[M], int (&chB)[M])
-{
-    int t0 = fv[0] + pj[0];
-    int lb = fv[0] + rv[0] + bv[0];
-    chF[0] = t0;
-#pragma unroll
-    for (int k = 1; k < M; k++) {
-        int t1 = max(fv[k], t0);
-        lb = max(lb, t1 + rv[k] + bv[k]);
-        t0 = t1 + pj[k];
-        chF[k] = t0;
-    }
-    lbF = lb;
-    if (both) {
-        t0 = bv[M - 1] + pj[M - 1];
-        lb = fv[M - 1] + rv[M - 1] + bv[M - 1];
-        chB[M - 1] = t0;
-#pragma unroll
-        for (int k = M - 2; k >= 0; k--) {
-            int t1 = max(t0, bv[k]);
-            lb = max(lb, fv[k] + rv[k] + t1);
-            t0 = t1 + pj[k];
-            chB[k] = t0;
-        }
-        lbB = lb;
-    } else {
-        lbB = 0;
-    }
-}
-
-// LB1' node bound (bound_fsp_weak.cpp:288-311) from explicit vectors.
-template <int M>
-__device__ __forceinline__ int lb1_node_vec(const int (&f)[M], const int (&r)[M], const int (&b)[M])
-{
-    int t0 = f[0] + r[0];
-    int lb = t0 + b[0];
-#pragma unroll
-    for (int k = 1; k < M; k++) {
-        int t1 = max(f[k] + r[k], t0);
-        lb = max(lb, t1 + b[k]);
-        t0 = t1;
-    }
-    return lb;
-}
-
 // Machine pairs of the Johnson bound, one per lane and chunk: chunk c of
 // lane l holds pair c*64 + l of the list as a | b << 8, or -1 when there is
 // no such pair or the JohnsonMode drops it (pairs_mode 1: pairs ending on the

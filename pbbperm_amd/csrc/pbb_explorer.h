@@ -344,10 +344,6 @@ struct Explorer {
 
     __device__ __forceinline__ int *frow(int s) const { return lds.stk + s * M; }
     __device__ __forceinline__ int *brow(int s) const { return lds.stk + (n - s) * M; }
-    // uniform stack values (LDS broadcast reads)
-    __device__ __forceinline__ int fval(int q) const { return frow(nf)[q]; }
-    __device__ __forceinline__ int bval(int q) const { return brow(nb)[q]; }
-    __device__ __forceinline__ int rval(int q) const { return rdlane(remv, q); }
 
     // lane q: p[q][job].  Lanes past the machines read machine M-1 and drop
     // it: an unconditional load, no exec-mask branch around it (as for the
@@ -612,17 +608,18 @@ struct Explorer {
             lb1_children(k, cb, ce);
             if (mode == 1) {
                 int csF = 0, csB = 0;
-                refine_both(valid, job, csF, csB);
+                refine_both(valid, cb, ce, csF, csB);
                 dir = choose(valid, csF, csB);
                 c1 = c2 = dir ? csB : csF;
                 refined = true;
             } else {
+                const int back = ce;
                 if (!both) ce = 0;
                 sb += (unsigned)(both ? 2 * k : k);
                 dir = choose(valid, cb, ce);
                 c1 = dir ? ce : cb;
                 if (mode == 2) {
-                    c2 = refine_dir(dir, valid, job, c1);
+                    c2 = refine_dir(dir, valid, c1, dir ? back : cb);
                     refined = true;
                 }
             }
@@ -636,53 +633,16 @@ struct Explorer {
     }
 
     // ---------------------------------------------------------- refinement
-    // The refinement bounds below work on one child per lane (lane = row
-    // cell), both directions, with the child's chains computed per lane
-    // (the refinement modes serve instances of up to 30 jobs; LB1 above is
-    // the fused hot loop).
-    // d = 0: front' = front + job; d = 1: back' = job + back.
-    __device__ __forceinline__ void child_chains(int job, int (&chF)[M], int (&chB)[M]) const
-    {
-        const int *pj = lds.pm + job;  // machine q at pj[q * PM_STRIDE]
-        constexpr int ps = PM_STRIDE;
-        int t = 0;
-#pragma unroll
-        for (int q = 0; q < M; q++) {
-            int f = fval(q);
-            t = (q == 0 ? f : max(f, t)) + pj[q * ps];
-            chF[q] = t;
-        }
-#pragma unroll
-        for (int q = M - 1; q >= 0; q--) {
-            int b = bval(q);
-            t = (q == M - 1 ? b : max(b, t)) + pj[q * ps];
-            chB[q] = t;
-        }
-    }
-
-    // LB1' of this lane's child (bound_fsp_weak::bornes_calculer with the
-    // child's front or back)
-    __device__ __forceinline__ int lb1p_child(int d, int job, const int (&chF)[M], const int (&chB)[M]) const
-    {
-        const int *pj = lds.pm + job;  // machine q at pj[q * PM_STRIDE]
-        constexpr int ps = PM_STRIDE;
-        int t0 = 0, lb = 0;
-#pragma unroll
-        for (int q = 0; q < M; q++) {
-            int f = d == 0 ? chF[q] : fval(q);
-            int b = d == 1 ? chB[q] : bval(q);
-            int r = rval(q) - pj[q * ps];
-            if (q == 0) {
-                t0 = f + r;
-                lb = t0 + b;
-            } else {
-                int t1 = max(f + r, t0);
-                lb = max(lb, t1 + b);
-                t0 = t1;
-            }
-        }
-        return lb;
-    }
+    // LB1' of a child (bound_fsp_weak::bornes_calculer with the child's front or
+    // back, bound_fsp_weak.cpp:288-311) is its LB1 bound, so the refinement of REF
+    // 1 takes that value and only counts.  With front times f, remaining work r and
+    // back times b, LB1' is the maximum over machines i <= q of f_i + r_i + b_q.
+    // Back times never grow with the machine: a back chain has b_q >= b_(q+1) +
+    // p_q, min_dep sums fewer times, and no time is negative.  So the maximum is at
+    // q = i, and f_i + r_i + b_i of the child is the LB1 term of machine i: front,
+    // max(f_i, f'_(i-1)) + p_i + (r_i - p_i) + b_i; back, the same from the other
+    // end.  A pass of its own with both of the child's chains per lane took half of
+    // a node's time (30x17, 6.3 M nodes: 8.1 ms, 6.2 without it).
 
     // Johnson LB2 of children c0 and c1 (uniform; K = 1: of c0 alone), direction d
     // (bound_fsp_strong::bornes_calculer with the child's partial schedule), to v0
@@ -779,20 +739,16 @@ struct Explorer {
     }
 
     // mixed mode (computeStrongBounds, ivm_bound.cpp:141-195): refine the
-    // children not pruned by LB1 in the chosen direction; 0 for the others
-    __device__ __forceinline__ int refine_dir(int d, bool valid, int job, int cw)
+    // children not pruned by LB1 in the chosen direction (cost cw, zero where only
+    // front costs are computed; lb1 is the bound itself); 0 for the others
+    __device__ __forceinline__ int refine_dir(int d, bool valid, int cw, int lb1)
     {
         const int k = n - L;
         bool todo = valid && !gt_best(cw);
         uint64_t tmask = ballot(todo);
         jb += (unsigned)__popcll(tmask);
         jhist += lane == L ? __popcll(tmask) : 0;
-        if constexpr (REF == 1) {
-            int chF[M], chB[M];
-            child_chains(job, chF, chB);
-            int v = lb1p_child(d, job, chF, chB);
-            return todo ? v : 0;
-        }
+        if constexpr (REF == 1) return todo ? lb1 : 0;
         int cs = 0;
         uint64_t m = tmask;
         while (m) {
@@ -813,16 +769,14 @@ struct Explorer {
     }
 
     // strong-only mode (strongBoundPrune, ivm_bound.cpp:668-676)
-    __device__ __forceinline__ void refine_both(bool valid, int job, int &csF, int &csB)
+    __device__ __forceinline__ void refine_both(bool valid, int cb, int ce, int &csF, int &csB)
     {
         const int k = n - L;
         jb += 2u * (unsigned)k;
         jhist += lane == L ? 2 * k : 0;
         if constexpr (REF == 1) {
-            int chF[M], chB[M];
-            child_chains(job, chF, chB);
-            csF = valid ? lb1p_child(0, job, chF, chB) : 0;
-            csB = valid ? lb1p_child(1, job, chF, chB) : 0;
+            csF = valid ? cb : 0;
+            csB = valid ? ce : 0;
             return;
         }
         csF = csB = 0;

@@ -26,8 +26,7 @@ namespace pbb {
 
 // ------------------------------------------------------------ kernels
 // Minimum resident waves per SIMD the compiler must allow (register
-// budget): 4 for the LB1 explorer (128 VGPRs), free for the refinement
-// variants.
+// budget): 4 for the LB1 and LB1' explorers (128 VGPRs), 3 with LB2.
 #ifndef PBB_EXPLORE_MIN_WAVES
 #define PBB_EXPLORE_MIN_WAVES 4
 #endif
@@ -123,7 +122,7 @@ __device__ __forceinline__ void explore_loop(const KArgs &a, const Lds &lds, int
 }
 
 template <int M, int REF>
-__global__ __launch_bounds__(64 * PBB_EXPLORE_WAVES, REF == 0 ? PBB_EXPLORE_MIN_WAVES : 3) void k_explore(KArgs a)
+__global__ __launch_bounds__(64 * PBB_EXPLORE_WAVES, REF == 2 ? 3 : PBB_EXPLORE_MIN_WAVES) void k_explore(KArgs a)
 {
     extern __shared__ __align__(16) char smem[];
     Lds lds = lds_setup(a.I, smem, REF == 2, REF == 2);

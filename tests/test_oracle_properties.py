@@ -195,3 +195,26 @@ def test_share_work_keeps_counts(oracle_mod, mode):
         total[1] += st.leaves
         total[2] += st.johnson_bounds
     assert total == [ref.decomposed, ref.leaves, ref.johnson_bounds]
+
+
+@pytest.mark.parametrize("n,m,top", [(5, 2, 99), (9, 7, 99), (20, 10, 3), (30, 17, 99), (63, 20, 1000000)])
+def test_lb1_of_a_child_is_its_lb1_prime(oracle_mod, n, m, top):
+    """The refinement bound LB1' of a child is its LB1 bound in either direction (the back times of a schedule do not
+    grow with the machine), which the engine's LB1' refinement relies on; empty fronts and backs and zero times among
+    the instances."""
+    rng = np.random.default_rng(n * m)
+    for t in range(12):
+        ptm = rng.integers(0, top + 1, (m, n)).astype(np.int32)
+        if t % 3 == 0:
+            ptm[rng.integers(0, m)] = 0
+        inst = oracle_mod.Instance(ptm)
+        perm = rng.permutation(n).astype(np.intc)
+        l1 = -1 if t % 2 else int(rng.integers(-1, n - 3))
+        l2 = n if t % 4 < 2 else int(rng.integers(l1 + 3, n + 1))
+        cb, ce, _, _ = inst.lb1_children(perm, l1, l2, True)
+        for i in range(l1 + 1, l2):
+            front, back = perm.copy(), perm.copy()
+            front[[l1 + 1, i]] = front[[i, l1 + 1]]
+            back[[l2 - 1, i]] = back[[i, l2 - 1]]
+            assert inst.lb1_node(front, l1 + 1, l2) == cb[perm[i]]
+            assert inst.lb1_node(back, l1, l2 - 1) == ce[perm[i]]
