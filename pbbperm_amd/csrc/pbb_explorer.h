@@ -309,6 +309,7 @@ struct Explorer {
     unsigned nchk;                    // periodic checks so far (host-word phase)
     unsigned since;                   // nodes decomposed in this launch's own interval (ramp)
     bool end_dirty;                   // end moved since pos was last compared with it
+    bool deep;                        // the last try_donate handed over a part of a large interval
     int hist;                         // lane d: nodes decomposed at depth d since the flush
     int jhist;                        // lane d: refinement bounds at depth d (REF != 0)
     unsigned long long t_end;
@@ -332,6 +333,7 @@ struct Explorer {
         pollw = seen = 0;
         nchk = (unsigned)eid;  // staggers the host-word reads across explorers
         end_dirty = true;
+        deep = false;
         hist = jhist = 0;
         local_best = PBB_INF;
         t_end = args.deadline ? wall_clock64() + args.deadline : 0ull;
@@ -1116,6 +1118,7 @@ struct Explorer {
     // whether idle explorers were waiting in it.
     __device__ __forceinline__ bool try_donate(unsigned long long idle)
     {
+        deep = false;
         idle = uni64(idle);
         const int word = pollw;
         next_word();
@@ -1145,6 +1148,7 @@ struct Explorer {
             else if (lane >= l && lane < n) endE = n - 1 - lane;
         }
         int nexp = __popcll(expl);
+        if (L - l < SHARE_NEAR && nexp < SHARE_CELLS) return true;
         // Claim one explorer of the word by clearing its bit; each donor starts
         // its choice at another bit.  Relaxed: the claim orders nothing, the
         // donor has published nothing yet.
@@ -1189,6 +1193,7 @@ struct Explorer {
         if (lane == l) endv = cut - 1;
         if (lane > l && lane < n) endv = n - 1 - lane;
         end_dirty = true;
+        deep = L - l >= SHARE_DEEP;
         return true;
     }
 

@@ -61,6 +61,14 @@ __device__ __forceinline__ int mail_path_cell(int i, int p, int j) { return i ==
 #ifndef PBB_POLL_EVERY
 #define PBB_POLL_EVERY 8
 #endif
+// What a donor gives: a split fewer than SHARE_NEAR lines above its own row hands
+// over a few nodes, less than the hand-over costs the two of them, unless that
+// line has SHARE_CELLS cells left (a wide, shallow tree).  A donor whose split
+// was SHARE_DEEP lines up or more holds a large interval and polls again at the
+// next node.  20x20 LB1 (0.83 M nodes) 2.9 -> 2.5 ms, 30x17 LB1' 6.2 -> 5.4, 47x17
+// LB1 (3.4 M) 5.6 -> 4.7, 19x10 LB2 7.6 -> 6.8; 2 lines and 4 cells 2.5, 5.7, 5.0,
+// 7.3; SHARE_DEEP 2, 3, 5 without the lower limit 2.8, 2.65, 2.66 at 20x20.
+enum { SHARE_NEAR = 3, SHARE_CELLS = 6, SHARE_DEEP = 4 };
 // The pool's explorers poll every PBB_POOL_POLL_EVERY nodes (512-instance batch:
 // every 8 / 16 / 32 / 64 nodes 49 / 49 / 51 / 53 ms).
 #ifndef PBB_POOL_POLL_EVERY

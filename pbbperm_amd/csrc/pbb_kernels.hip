@@ -98,9 +98,10 @@ __device__ __forceinline__ void explore_loop(const KArgs &a, const Lds &lds, int
         // hidden; none while the ramp holds this explorer's work back.  In
         // the workgroup team (at most 16 explorers, workgroup-scope atomics)
         // and with LB2 a donor that saw explorers waiting polls again at the
-        // next node (PBB_POLL_EVERY).
+        // next node, otherwise one that gave from a large interval
+        // (PBB_POLL_EVERY, SHARE_DEEP).
         constexpr bool eager = SC == __HIP_MEMORY_SCOPE_WORKGROUP || REF == 2;
-        const bool poll = X.since >= a.ramp && ((eager && hungry) || (iter & (PBB_POLL_EVERY - 1)) == 0u);
+        const bool poll = X.since >= a.ramp && (hungry || (iter & (PBB_POLL_EVERY - 1)) == 0u);
         unsigned long long idle = 0ull;
         if (poll) idle = X.peek_idle();
         const bool refresh = (iter & (PBB_BEST_EVERY - 1)) == 0u;
@@ -117,7 +118,7 @@ __device__ __forceinline__ void explore_loop(const KArgs &a, const Lds &lds, int
             X.flush_counters();
             return;
         }
-        if (poll) hungry = X.try_donate(idle);
+        if (poll) hungry = X.try_donate(idle) && (eager || X.deep);
     }
 }
 

@@ -569,6 +569,7 @@ __global__ __launch_bounds__(256, PBB_POOL_MIN_WAVES(M)) void k_pool(KArgs a, Po
                 X.register_idle();
             }
             unsigned iter = 0;
+            bool hungry = false;
             for (;;) {
                 if (st == ST_IDLE) {
                     bool leave = false;
@@ -590,7 +591,7 @@ __global__ __launch_bounds__(256, PBB_POOL_MIN_WAVES(M)) void k_pool(KArgs a, Po
                     }
                     if (leave) break;
                 }
-                const bool poll = (iter & (PBB_POOL_POLL_EVERY - 1)) == 0u;
+                const bool poll = hungry || (iter & (PBB_POOL_POLL_EVERY - 1)) == 0u;
                 unsigned long long idle = 0ull;
                 if (poll) idle = X.peek_idle();
                 const bool refresh = (iter & (PBB_BEST_EVERY - 1)) == 0u;
@@ -611,7 +612,7 @@ __global__ __launch_bounds__(256, PBB_POOL_MIN_WAVES(M)) void k_pool(KArgs a, Po
                         continue;
                     }
                 }
-                if (poll) X.try_donate(idle);
+                if (poll) hungry = X.try_donate(idle) && (REF == 2 || X.deep);
             }
             X.flush_counters();
         }
