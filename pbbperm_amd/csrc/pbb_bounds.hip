@@ -70,7 +70,7 @@ __device__ __host__ inline size_t bound_table_bytes(const DevInst &I, bool jtab)
 {
     size_t b = ((size_t)2 * M * PM_STRIDE + 3 * M) * 4;
     b = (b + 15) & ~(size_t)15;
-    if (jtab) b += ((size_t)I.npairs * I.n * 4 + 15) & ~(size_t)15;
+    if (jtab) b += (size_t)I.n * 64 * jtab_chunks(I.npairs) * 5;  // words, then a byte of place each
     return b;
 }
 
@@ -132,8 +132,16 @@ __global__ __launch_bounds__(B_THREADS) void k_bounds(DevInst I, int count, int 
         minA[tid] = I.min_arr[tid];
         minD[tid] = I.min_dep[tid];
     }
-    if (jtab)
-        for (int i = tid; i < I.npairs * n; i += B_THREADS) jtabL[i] = ((const unsigned *)I.jtab)[i];
+    uint8_t *place = (uint8_t *)(jtabL + (size_t)n * 64 * jtab_chunks(I.npairs));
+    if (jtab) {
+        const int W = 64 * jtab_chunks(I.npairs);
+        for (int i = wave; i < n; i += B_THREADS / 64)
+            for (int c = lane; c < W; c += 64) {
+                const unsigned e = ((const unsigned *)I.jtab)[i * I.npairs + min(c, I.npairs - 1)];
+                jtabL[i * W + c] = e;
+                place[(e & 63u) * W + c] = (uint8_t)i;
+            }
+    }
     constexpr int PCH = (M * (M - 1) / 2 + PBB_WAVE - 1) / PBB_WAVE;
     int pinfo[PCH];
     if constexpr (WHICH == B_LB2) pair_lanes<PCH>(I.pair_ab, I.npairs, I.m, arg, pinfo);
@@ -344,7 +352,15 @@ __global__ __launch_bounds__(B_THREADS) void k_bounds(DevInst I, int count, int 
                     const uint64_t mid = uni64(S.mid[s]);
                     if (__popcll(mid) <= 1) continue;
                     const int *fs = (const int *)(S.U + (size_t)s * US);
-                    const int v = lb2_pairs_any<PCH, 2>(pinfo, jtab, jtabL, I.jtab, false, n, I.npairs, fs, fs + 1, mid);
+                    const int k = __popcll(mid);
+                    int v;
+                    if (!jtab) v = lb2_pairs<PCH, false, false, 2>(pinfo, I.jtab, n, I.npairs, fs, fs + 1, mid);
+                    else if (n <= 32)
+                        v = 12 * k < 7 * n ? lb2_few<PCH, true, 2>(pinfo, jtabL, place, fs, fs + 1, mid)
+                                           : lb2_pairs<PCH, true, true, 2>(pinfo, jtabL, n, 64 * PCH, fs, fs + 1, mid);
+                    else
+                        v = 19 * k < 9 * n ? lb2_few<PCH, false, 2>(pinfo, jtabL, place, fs, fs + 1, mid)
+                                           : lb2_pairs<PCH, false, true, 2>(pinfo, jtabL, n, 64 * PCH, fs, fs + 1, mid);
                     if (lane == 0) o1[s0 + s] = v;
                 }
             }
@@ -365,9 +381,10 @@ static hipError_t launch(const DevInst &I, int count, const int *perms, const in
     while (T > 16 && tab + bound_tile_bytes<M>(T) > room) T -= 16;
     while (T > 16 && (count + T - 1) / T < 512) T -= 16;
     const size_t lds = tab + bound_tile_bytes<M>(T);
-    if (const hipError_t err = hipFuncSetAttribute((const void *)k_bounds<M, WHICH>,
-                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
-        return err;
+    if (lds > 64 * 1024)
+        if (const hipError_t err = hipFuncSetAttribute((const void *)k_bounds<M, WHICH>,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
+            return err;
     const int tiles = (count + T - 1) / T;
     const int resident = 256 * (int)(160 * 1024 / lds < 8 ? 160 * 1024 / lds : 8);
     const int grid = tiles < resident ? tiles : resident;

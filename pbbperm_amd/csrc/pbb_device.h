@@ -17,6 +17,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #define PBB_WAVE 64
 #define PBB_INF 0x7fffffff
 
@@ -151,6 +153,23 @@ __device__ __forceinline__ int job_mask(int e, uint64_t unsched)
     else return __builtin_amdgcn_sbfe((int)(unsigned)(unsched >> (e & 63)), 0u, 1u);
 }
 
+// The bound from every pair's best (lb2_pairs): the greatest over this lane's
+// pairs and the wavefront.
+template <int PCH, int ST>
+__device__ __forceinline__ int lb2_finish(const int (&pinfo)[PCH], const int (&best)[PCH], const int *fs, const int *gs)
+{
+    int r = 0;
+#pragma unroll
+    for (int c = 0; c < PCH; c++) {
+        const int info = pinfo[c];
+        if (info >= 0) {
+            const int a = info & 0xff, b = info >> 8;
+            r = max(r, max(best[c] + gs[b * ST], fs[a * ST] + gs[a * ST]));
+        }
+    }
+    return wave_max(r);
+}
+
 // Johnson LB2 of one partial schedule over the machine pairs of pinfo
 // (bound_fsp_strong.cpp:50-100, :102-162 without early exit, as
 // bornes_calculer calls them, :540-560).  fs: its front completion times;
@@ -205,16 +224,7 @@ __device__ __forceinline__ int lb2_pairs(const int (&pinfo)[PCH], const void *jt
             }
         }
     }
-    int r = 0;
-#pragma unroll
-    for (int c = 0; c < PCH; c++) {
-        const int info = pinfo[c];
-        if (info >= 0) {
-            const int a = info & 0xff, b = info >> 8;
-            r = max(r, max(best[c] + gs[b * ST], fs[a * ST] + gs[a * ST]));
-        }
-    }
-    return wave_max(r);
+    return lb2_finish<PCH, ST>(pinfo, best, fs, gs);
 }
 
 // Word of the staged table of up to 32 jobs, row i of a pair's column: w of the
@@ -253,18 +263,59 @@ __device__ __forceinline__ void lb2_walk(const unsigned *tab, int cnt, unsigned 
     }
 }
 
-// lb2_pairs with the packed table staged in LDS, or the packed or the wide one
-// in global memory
-template <int PCH, int ST = 1>
+// lb2_pairs of one schedule with few unscheduled jobs, of a table staged with rows
+// of W = 64 PCH words (the columns past the last pair repeat it): place[j * W + c]
+// is job j's place in the order of column c.  The lane's mask of places is built
+// for the schedule, 3 instructions (4 above 32 jobs) per unscheduled job and
+// chunk, and walked as in lb2_walk, 9 (15); lb2_pairs takes 7 (9) for every job.
+// 100 k schedules at 50x20, a quarter of the jobs unscheduled on average: 382 -> 276 us.
+template <int PCH, bool N32, int ST>
+__device__ __forceinline__ int lb2_few(const int (&pinfo)[PCH], const unsigned *tab, const uint8_t *place, const int *fs,
+                                       const int *gs, uint64_t unsched)
+{
+    typedef std::conditional_t<N32, unsigned, uint64_t> Mask;
+    constexpr int W = 64 * PCH;
+    const int lane = lane_id();
+    Mask places[PCH];
+    int D[PCH], best[PCH];
+#pragma unroll
+    for (int c = 0; c < PCH; c++) {
+        const int ab = pinfo[c] < 0 ? 0 : pinfo[c];
+        D[c] = fs[(ab & 0xff) * ST];
+        best[c] = fs[(ab >> 8) * ST];
+        places[c] = 0;
+    }
+    for (uint64_t u = unsched; u; u &= u - 1) {
+        const uint8_t *pl = place + (__ffsll((unsigned long long)u) - 1) * W + lane;
+#pragma unroll
+        for (int c = 0; c < PCH; c++) places[c] |= (Mask)1 << pl[c * 64];
+    }
+    const int cnt = __popcll(unsched);
+#pragma unroll 2
+    for (int i = 0; i < cnt; i++) {
+#pragma unroll
+        for (int c = 0; c < PCH; c++) {
+            const int p = N32 ? __builtin_ctz((unsigned)places[c]) : __builtin_ctzll(places[c]);
+            places[c] &= places[c] - 1;
+            const int e = (int)tab[p * W + c * 64 + lane];
+            best[c] = max(best[c], D[c] + (int)__builtin_amdgcn_ubfe((unsigned)e, 6u, 15u));
+            D[c] += e >> 21;
+        }
+    }
+    return lb2_finish<PCH, ST>(pinfo, best, fs, gs);
+}
+
+// lb2_pairs of an explorer's child where lb2_walk's table does not apply: the
+// packed table of more than 32 jobs in LDS, the packed or the wide one in global
+// memory
+template <int PCH>
 __device__ __forceinline__ int lb2_pairs_any(const int (&pinfo)[PCH], bool staged, const unsigned *jtabL,
                                              const void *jtabG, bool packed, int n, int npairs, const int *fs,
                                              const int *gs, uint64_t unsched)
 {
-    if (staged)
-        return n <= 32 ? lb2_pairs<PCH, true, true, ST>(pinfo, jtabL, n, npairs, fs, gs, unsched)
-                       : lb2_pairs<PCH, false, true, ST>(pinfo, jtabL, n, npairs, fs, gs, unsched);
-    return packed ? lb2_pairs<PCH, false, true, ST>(pinfo, jtabG, n, npairs, fs, gs, unsched)
-                  : lb2_pairs<PCH, false, false, ST>(pinfo, jtabG, n, npairs, fs, gs, unsched);
+    if (staged) return lb2_pairs<PCH, false, true, 1>(pinfo, jtabL, n, npairs, fs, gs, unsched);
+    return packed ? lb2_pairs<PCH, false, true, 1>(pinfo, jtabG, n, npairs, fs, gs, unsched)
+                  : lb2_pairs<PCH, false, false, 1>(pinfo, jtabG, n, npairs, fs, gs, unsched);
 }
 
 }  // namespace pbb
