@@ -309,7 +309,6 @@ struct Explorer {
     unsigned nchk;                    // periodic checks so far (host-word phase)
     unsigned since;                   // nodes decomposed in this launch's own interval (ramp)
     bool end_dirty;                   // end moved since pos was last compared with it
-    bool deep;                        // the last try_donate handed over a part of a large interval
     int hist;                         // lane d: nodes decomposed at depth d since the flush
     int jhist;                        // lane d: refinement bounds at depth d (REF != 0)
     unsigned long long t_end;
@@ -333,7 +332,6 @@ struct Explorer {
         pollw = seen = 0;
         nchk = (unsigned)eid;  // staggers the host-word reads across explorers
         end_dirty = true;
-        deep = false;
         hist = jhist = 0;
         local_best = PBB_INF;
         t_end = args.deadline ? wall_clock64() + args.deadline : 0ull;
@@ -1114,17 +1112,17 @@ struct Explorer {
     // work on: a small tree then runs depth-first in one explorer, finding
     // the incumbents the reference's order finds, and a large one fans out
     // after that many nodes (woken and resumed explorers share at once).
-    // idle: the mask word loaded before the node's work (peek_idle).  Returns
-    // whether idle explorers were waiting in it.
-    __device__ __forceinline__ bool try_donate(unsigned long long idle)
+    // idle: the mask word loaded before the node's work (peek_idle).  Returns 0
+    // when no explorer waits in it, 2 after a hand-over from a large interval
+    // (SHARE_DEEP), else 1.
+    __device__ __forceinline__ int try_donate(unsigned long long idle)
     {
-        deep = false;
         idle = uni64(idle);
         const int word = pollw;
         next_word();
-        if (!idle) return false;
+        if (!idle) return 0;
         const int lim = min(L, n - 1 - a.steal_margin);  // last line a split may use
-        if (lim < 0) return true;                         // margin >= n: never split
+        if (lim < 0) return 1;                         // margin >= n: never split
         uint64_t ne = lanes_below(n) & ballot(posv != endv);
         uint64_t limmask = lim >= 64 ? ~0ull : ((1ull << lim) - 1ull);
         uint64_t cand = ne & limmask;
@@ -1132,7 +1130,7 @@ struct Explorer {
         int l = first, pl = 0, el = 0, rowl = -1;
         uint64_t expl = 0ull;
         for (;; l++) {
-            if (l > lim) return true;
+            if (l > lim) return 1;
             pl = rdlane(posv, l);
             el = (l == first) ? rdlane(endv, l) : n - 1 - l;
             if (pl < el) {
@@ -1148,7 +1146,7 @@ struct Explorer {
             else if (lane >= l && lane < n) endE = n - 1 - lane;
         }
         int nexp = __popcll(expl);
-        if (L - l < SHARE_NEAR && nexp < SHARE_CELLS) return true;
+        if (L - l < SHARE_NEAR && nexp < SHARE_CELLS) return 1;
         // Claim one explorer of the word by clearing its bit; each donor starts
         // its choice at another bit.  Relaxed: the claim orders nothing, the
         // donor has published nothing yet.
@@ -1162,7 +1160,7 @@ struct Explorer {
             if (ir.member) thief = ld_rlx<SC>(ir.member + idx);
             got = (int)((old >> bit) & 1ull);
         }
-        if (!rdlane(got, 0)) return true;
+        if (!rdlane(got, 0)) return 1;
         thief = rdlane(thief, 0);
         // The thief is idle and this donor's alone now, so its mailbox holds the
         // last message it consumed: the next one's tag follows from it.  The
@@ -1193,8 +1191,7 @@ struct Explorer {
         if (lane == l) endv = cut - 1;
         if (lane > l && lane < n) endv = n - 1 - lane;
         end_dirty = true;
-        deep = L - l >= SHARE_DEEP;
-        return true;
+        return L - l >= SHARE_DEEP ? 2 : 1;
     }
 
     // member index of this explorer in its instance (the engine's explorers

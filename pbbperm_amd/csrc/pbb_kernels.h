@@ -259,7 +259,7 @@ inline size_t root_lds_bytes(const DevInst &I)
 // ------------------------------------------------------------------ pool
 // Many instances in one resident launch.  Workgroups of W explorers take one
 // instance slot at a time: the first group to pop a slot from the request
-// queue admits it (tables, idle ring, root), later groups join running slots
+// queue admits it (tables, idle mask, root), later groups join running slots
 // whose explorers are all busy, up to a per-instance explorer cap; work moves
 // between the members of a slot through its idle mask exactly as in the
 // one-instance engine.  The last member to leave a solved slot writes its

@@ -612,7 +612,7 @@ __global__ __launch_bounds__(256, PBB_POOL_MIN_WAVES(M)) void k_pool(KArgs a, Po
                         continue;
                     }
                 }
-                if (poll) hungry = X.try_donate(idle) && (REF == 2 || X.deep);
+                if (poll) hungry = X.try_donate(idle) >= (REF == 2 ? 1 : 2);
             }
             X.flush_counters();
         }
