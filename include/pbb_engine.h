@@ -68,9 +68,10 @@ typedef struct pbb_config {
                                reference counterpart */
     int team_nodes;         /* a search from pbb_init_full first runs on one
                                workgroup of explorers (16 with LB1 only, 8 with
-                               a refinement bound) for up to this many nodes,
-                               then on the whole device (0: whole device at
-                               once); engine-specific, no reference counterpart */
+                               a refinement bound) for up to this many nodes
+                               (LB1: half of it until the incumbent moves;
+                               a refinement bound: an eighth), then on the
+                               whole device (0: whole device at once); engine-specific, no reference counterpart */
     int team_waves;         /* explorers of that workgroup (0: the largest the
                                kernel allows, 16 or 8; larger values are
                                clamped to it); engine-specific, no reference
