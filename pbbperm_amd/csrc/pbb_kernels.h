@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "pbb_device.h"
+#include "pbb_slot.h"
 
 namespace pbb {
 
@@ -265,7 +266,6 @@ inline size_t root_lds_bytes(const DevInst &I)
 // one-instance engine.  The last member to leave a solved slot writes its
 // result record.  Instances with fewer machines than the pool's M are padded
 // with zero-time machines, which changes none of the bounds or makespans.
-enum { POOL_RUNNING = 1 << 30, POOL_DONE = 1 << 29, POOL_MEMBERS = (1 << 29) - 1 };
 enum { RES_PENDING = 0, RES_SOLVED = 1, RES_ABORTED = 2, RES_INVALID = 3 };
 enum { ROLE_EXIT = 0, ROLE_OWNER = 1, ROLE_HELPER = 2 };
 
@@ -330,7 +330,7 @@ __device__ __host__ inline PoolLayout pool_layout(int nmax, int M, int pmax, int
 
 struct PoolArgs {
     char *arena;                  // nslots x layout.stride
-    int *occ;                     // [nslots] POOL_RUNNING | POOL_DONE | member explorers
+    int *occ;                     // [nslots] occupancy words (pbb_slot.h)
     PoolLayout lay;
     int nslots;
     int W;                        // explorers (wavefronts) per workgroup

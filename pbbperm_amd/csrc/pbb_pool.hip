@@ -12,11 +12,10 @@
 //                      bounds the root (ivm_bound::boundRoot,
 //                      ivm_bound.cpp:273-330) and explores the full interval
 //                      from explorer 0 of the group;
-//                    * helper: joins the running slot with the most busy
-//                      explorers net of idle ones (up to the per-instance
-//                      cap) and receives work
-//                      through the slot's idle mask, as explorers of the
-//                      one-instance engine do.
+//                    * helper: joins a running slot below the per-instance
+//                      cap, drawn by its surplus of busy over idle explorers,
+//                      and receives work through the slot's idle mask, as
+//                      explorers of the one-instance engine do.
 //                  The explorer whose release empties a slot records the
 //                  optimum; the last member to leave writes the result
 //                  record (host-visible when serving).  The launch ends when
@@ -226,8 +225,8 @@ static __device__ __forceinline__ bool pool_admit(const PoolArgs &p, int s, bool
 // Wave 0 of a free workgroup: a new instance from the queue first, else a
 // running slot below the per-instance cap, drawn with its surplus of busy over
 // idle explorers as weight, else wait.  Returns the role; *slot receives the slot id
-// and *base the member index of the group's first wave (members stay until the
-// slot is done, so the indices are dense).
+// and *base the member index of the group's first wave (slot_open: no index is
+// given twice).
 //
 // Hundreds of groups choose at once (a batch's tail, an idle server).  When all
 // went for the largest surplus they raced for one word, one join per pass over
@@ -293,7 +292,7 @@ static __device__ __forceinline__ int pool_pick(const PoolArgs &p, int W, unsign
             const int o = s < p.nslots ? ld_rlx(p.occ + s) : 0;
             running = running || ballot(o != 0) != 0ull;
             const int mem = o & POOL_MEMBERS;
-            const bool room = (o & POOL_RUNNING) && !(o & POOL_DONE) && mem + W <= p.epi;
+            const bool room = slot_open(o, W, p.epi);
             if (!ballot(room)) continue;
             int more = 0;
             if (room) {
@@ -328,7 +327,7 @@ static __device__ __forceinline__ int pool_pick(const PoolArgs &p, int W, unsign
                 }
                 surplus -= (seen & POOL_MEMBERS) - (occ & POOL_MEMBERS);
                 occ = seen;
-                if (!(occ & POOL_RUNNING) || (occ & POOL_DONE) || (occ & POOL_MEMBERS) + W > p.epi || surplus <= 0) break;
+                if (!slot_open(occ, W, p.epi) || surplus <= 0) break;
             }
             nap = 1;
             continue;
@@ -372,7 +371,8 @@ static __device__ __forceinline__ void pool_leave(const PoolArgs &p, int s, int 
 {
     const int lane = lane_id();
     PoolSlot *S = slot_hdr(p, s);
-    const int old = w_add(p.occ + s, -W);
+    if (lane == 0) __hip_atomic_fetch_or(p.occ + s, (int)POOL_CLOSING, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int old = w_add(p.occ + s, -W);  // the same word: after the or
     if ((old & POOL_MEMBERS) != W) return;
     PoolRes *R = p.res + s;
     const int status = (old & POOL_DONE) ? uni(ld_rlx(&S->status)) : (int)RES_ABORTED;
