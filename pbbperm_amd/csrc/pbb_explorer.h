@@ -1194,17 +1194,18 @@ struct Explorer {
         return L - l >= SHARE_DEEP ? 2 : 1;
     }
 
-    // member index of this explorer in its instance (the engine's explorers
-    // are their own members).  The member word is complete before the first
-    // registration names it: the wait for the store is explicit, as a fence at
-    // agent scope would write the L2 back.
+    // member index of this explorer in its instance (the engine's explorers are
+    // their own members).  The member word is complete, and the old tag of the
+    // mailbox has been read (open_mail, before), when the first registration
+    // names this explorer: a donor that claims it at once would otherwise find
+    // another explorer's number, or send a message that is taken for the old one.
+    // Relaxed accesses to different words have no order, so the wait is explicit (a
+    // fence at agent scope would write the L2 back).
     __device__ __forceinline__ void join(int idx)
     {
         self = idx;
-        if (ir.member) {
-            if (lane == 0) st_rlx<SC>(const_cast<int *>(ir.member) + idx, e);
-            asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-        }
+        if (ir.member && lane == 0) st_rlx<SC>(const_cast<int *>(ir.member) + idx, e);
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(mtag) : : "memory");
         pollw = ir.occ ? 0 : idx % ir.idle_words;
     }
 
