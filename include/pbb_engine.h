@@ -38,6 +38,8 @@ extern "C" {
 
 /* ------------------------------------------------------------------ config */
 
+#define PBB_TEAM_NODES_DEFAULT 8192
+
 /* Mirrors the [bb]/[gpu]/[initial] keys read by arguments::readIniFile. */
 typedef struct pbb_config {
     int bound_mode;         /* [bb] boundingMode: 0 LB1, 1 strong only, 2 LB1 + refinement */
@@ -68,10 +70,13 @@ typedef struct pbb_config {
                                reference counterpart */
     int team_nodes;         /* a search from pbb_init_full first runs on one
                                workgroup of explorers (16 with LB1 only, 8 with
-                               a refinement bound) for up to this many nodes
-                               (LB1: half of it until the incumbent moves;
-                               a refinement bound: an eighth), then on the
-                               whole device (0: whole device at once); engine-specific, no reference counterpart */
+                               a refinement bound) for up to this many nodes,
+                               then on the whole device (0: whole device at
+                               once).  At PBB_TEAM_NODES_DEFAULT the engine
+                               gives the team its share of them: LB1 half until
+                               the incumbent moves, a refinement bound an
+                               eighth.  Engine-specific, no reference
+                               counterpart */
     int team_waves;         /* explorers of that workgroup (0: the largest the
                                kernel allows, 16 or 8; larger values are
                                clamped to it); engine-specific, no reference

@@ -613,25 +613,37 @@ static int launch_once(pbb_engine *e, bool team, uint64_t node_budget, uint64_t 
     return take_incumbent(e, *e->best_h);
 }
 
-// Nodes of the team phase, at most cfg.team_nodes.  The team pays on trees that
-// end within it; on a larger one it holds the device back, so it gets about
-// the time that a device-wide launch needs to fan out, half a millisecond: half
-// of team_nodes with LB1 (16 explorers, 0.14-0.17 us a node), an eighth with a
-// refinement bound (8 explorers, 0.33 us a node with LB1' at 17 machines, 0.42
-// and 0.78 us with LB2 at 10 and 20).  At the default 8192, all of it against
-// this share: 30x20 LB2 9.0 -> 3.9 ms, 20x20 LB1 3.5 -> 3.0, 30x17 LB1' 10.5 ->
-// 8.3, 20x10 LB2 (3636 nodes, all in the team before) 1.67 -> 1.45; at none, a
-// 2457-node LB1 tree 1.1 against 0.55 ms.  With LB1 the team keeps all of
+// Nodes of the team phase while the incumbent has not moved, and once it has.
+// team_nodes as the caller set it, unless it is the default: then the engine
+// chooses.  The team pays on trees that end within it; on a larger one it holds
+// the device back, so it gets about the time that a device-wide launch needs to
+// fan out, half a millisecond: half of team_nodes with LB1 (16 explorers,
+// 0.14-0.17 us a node), an eighth with a refinement bound (8 explorers, 0.33 us a
+// node with LB1' at 17 machines, 0.42 and 0.78 us with LB2 at 10 and 20).  All of
+// it against this share: 30x20 LB2 9.0 -> 3.9 ms, 20x20 LB1 3.5 -> 3.0, 30x17 LB1'
+// 10.5 -> 8.3, 20x10 LB2 (3636 nodes, all in the team before) 1.67 -> 1.45; at
+// none, a 2457-node LB1 tree 1.1 against 0.55 ms.  With LB1 the team keeps all of
 // team_nodes once it has found a better schedule: more explorers would search
-// more of what the next one prunes (20x5 from NEH: 1.05 against 0.9 ms).
-static uint64_t team_budget(const pbb_config &c)
+// more of what the next one prunes (20x5 from NEH: 1.05 against 0.9 ms).  An engine
+// of no more explorers than the team has nothing to gain from the second launch,
+// and a run for fewer nodes than team_nodes stays with the team, which stops
+// within a few hundred nodes of its budget; thousands of explorers, each of which
+// looks every 64 nodes, overrun it by as many.
+struct TeamBudget {
+    uint64_t quiet, moved;
+};
+static TeamBudget team_budget(const pbb_engine *e, uint64_t node_budget)
 {
-    return std::max<uint64_t>(1, (uint64_t)c.team_nodes / (c.bound_mode == 0 ? 2 : 8));
+    const uint64_t most = (uint64_t)e->cfg.team_nodes;
+    if (node_budget && node_budget <= most) return {node_budget, node_budget};
+    if (e->cfg.team_nodes != PBB_TEAM_NODES_DEFAULT || e->E <= e->team_E) return {most, most};
+    if (e->cfg.bound_mode == 0) return {most / 2, most};
+    return {most / 8, most / 8};
 }
 
 // A search started by pbb_init_full runs first on the team (one workgroup)
-// for team_budget() decomposed nodes (LB1: team_nodes once the incumbent has
-// moved); what is left then continues on the device-wide grid from the team's saved intervals.
+// for team_budget() decomposed nodes; what is left then continues on the
+// device-wide grid from the team's saved intervals.
 extern "C" int pbb_run(pbb_engine *e, uint64_t node_budget, double time_budget_s, int *all_done)
 {
     if (!e) return fail(PBB_E_ARG, "null engine");
@@ -645,11 +657,10 @@ extern "C" int pbb_run(pbb_engine *e, uint64_t node_budget, double time_budget_s
     float ms = 0.f;
     if (e->team_pending) {
         e->team_pending = false;
-        const uint64_t share = team_budget(e->cfg), full = e->cfg.bound_mode == 0 ? (uint64_t)e->cfg.team_nodes : share;
-        const uint64_t tb = node_budget ? std::min(node_budget, full) : full;
+        const TeamBudget tb = team_budget(e, node_budget);
         const uint64_t before = e->dec_dev;
         const auto t0 = std::chrono::steady_clock::now();
-        int rc = launch_once(e, true, tb, std::min(tb, share), time_budget_s, &ms);
+        int rc = launch_once(e, true, tb.moved, tb.quiet, time_budget_s, &ms);
         if (rc) return rc;
         e->last_ms += ms;
         if (e->done_host) {

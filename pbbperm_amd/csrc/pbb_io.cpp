@@ -57,7 +57,7 @@ extern "C" int pbb_config_default(pbb_config *c)
     c->checkpoint_s = 1;
     c->balance_s = 1;
     c->ramp_nodes = 0;
-    c->team_nodes = 8192;
+    c->team_nodes = PBB_TEAM_NODES_DEFAULT;
     c->team_waves = 0;
     return PBB_OK;
 }
@@ -185,7 +185,7 @@ extern "C" int pbb_config_load_ini(const char *path, pbb_config *c, char *proble
     c->refine = (int)ini_int(kv, "bb.refinementbound", 0);
     c->steal_margin = (int)ini_int(kv, "gpu.stealmargin", 6);
     c->ramp_nodes = (int)ini_int(kv, "gpu.rampnodes", 0);
-    c->team_nodes = (int)ini_int(kv, "gpu.teamnodes", 8192);
+    c->team_nodes = (int)ini_int(kv, "gpu.teamnodes", PBB_TEAM_NODES_DEFAULT);
     c->team_waves = (int)ini_int(kv, "gpu.teamwaves", 0);
     return validate(c);
 }

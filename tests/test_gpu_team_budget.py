@@ -1,0 +1,29 @@
+"""team_nodes holds a search in the team (explorers 0-15 with LB1, 0-7 with a
+refinement bound) for as many nodes as the caller set, and a run for fewer nodes
+stops in the team near its budget: it has saved intervals of those explorers only.
+Incumbent frozen, so the whole search's count is exact."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+LB2 = dict(bound_mode=2, branching=1, refine=1, johnson_pairs=0, early_stop_johnson=0)
+LB1 = dict(bound_mode=0, branching=1)
+
+# mode, team size, seed, jobs, machines, incumbent, nodes of the tree, node budget of the first run
+SEARCHES = [(LB2, 8, 1, 20, 10, 1548, 3636, 2500), (LB1, 16, 2, 30, 10, 2117, 5394, 4700)]
+
+
+@pytest.mark.parametrize("mode,team,seed,n,m,ub,nodes,budget", SEARCHES)
+@pytest.mark.parametrize("team_nodes", [5000, 100000, 8192])
+def test_team_keeps_a_search_for_team_nodes(mode, team, seed, n, m, ub, nodes, budget, team_nodes):
+    import pbbperm_amd as P
+    cfg = P.default_config(nb_ivms=4096, team_nodes=team_nodes, **mode)
+    with P.GpuBB(P.synth(seed, n, m), cfg, ub=ub) as eng:
+        eng.init_full_interval()
+        assert not eng.next(node_budget=budget)
+        ids = eng.get_intervals()[0]
+        assert len(ids) and max(ids) < team
+        # an explorer looks at the budget every 64 nodes
+        assert budget <= eng.stats().decomposed < budget + 64 * team
+        assert eng.next()
+        assert eng.stats().decomposed == nodes
