@@ -138,7 +138,8 @@ struct Lds {
                     // (2066 against 2100-2104 M nodes/s at 50x20)
 };
 
-__device__ __forceinline__ Lds lds_setup(const DevInst &I, char *smem, bool load_jtab, bool scratch)
+// jt: bytes set aside for a Johnson table; an instance's is staged if it fits
+__device__ __forceinline__ Lds lds_setup(const DevInst &I, char *smem, int jt, bool scratch)
 {
     Lds L;
     const int n = I.n, mp = I.mp, m = I.m;
@@ -148,16 +149,14 @@ __device__ __forceinline__ Lds lds_setup(const DevInst &I, char *smem, bool load
     L.minA = L.pmR + m * PM_STRIDE;
     L.minD = L.minA + mp;
     L.tot = L.minD + mp;
-    size_t off = ((size_t)2 * m * PM_STRIDE + 3 * (size_t)mp) * 4;
-    off = (off + 15) & ~(size_t)15;
-    load_jtab = load_jtab && jtab_staged(I);
-    L.jtabL = (unsigned *)(smem + off);
+    const bool load_jtab = jt > 0 && I.jpacked && jtab_lds_bytes(n, I.npairs) <= jt;
+    L.jtabL = (unsigned *)(smem + lds_table_bytes(m, 0));
     L.jpacked = I.jpacked != 0;
     L.jtabG = I.jtab;
     L.jtl = load_jtab;
     L.nch = jtab_chunks(I.npairs);
     L.jtwalk = load_jtab && n <= 32;
-    char *wbase = smem + lds_table_bytes(n, m, I.npairs, load_jtab) +
+    char *wbase = smem + lds_table_bytes(m, jt) +
                   (size_t)(threadIdx.x >> 6) * lds_wave_bytes(n, m, scratch);
     L.mat = (int8_t *)wbase;
     L.stk = (int *)(wbase + lds_mat_bytes(n));

@@ -300,6 +300,7 @@ static KArgs make_args(pbb_engine *e)
     a.mbox = e->mbox;
     a.idle = e->idle;
     a.idle_words = idle_words_for(e->E);
+    a.jt_lds = e->D.I.jpacked ? explore_jtab_bytes(e->D.I) : 0;
     a.ctl = e->ctl;
     a.best = e->best;
     a.best_perm = e->best_perm;
@@ -332,7 +333,7 @@ static hipError_t copy_sync(pbb_engine *e, void *dst, const void *src, size_t by
 static int capacity(pbb_engine *e, int *explorers)
 {
     KArgs a = make_args(e);
-    a.I.jpacked = 1;  // the larger footprint: a retargeted engine keeps its explorers
+    a.jt_lds = explore_jtab_bytes(a.I);  // staged or not: a retargeted engine keeps its explorers
     int bpc = 0;
     HIPCHK(explore_occupancy(a, &bpc));
     if (bpc < 1) return fail(PBB_E_CAPACITY, "explorer kernel does not fit one workgroup per CU (LDS)");
@@ -404,9 +405,7 @@ extern "C" int pbb_create(const int32_t *ptm, int n, int m, const pbb_config *cf
         const int ref = cfg->bound_mode == 0 ? 0 : (cfg->refine == 1 ? 2 : 1);
         int w = std::min(e->E, team_waves_max(ref));
         if (cfg->team_waves > 0) w = std::min(w, cfg->team_waves);
-        DevInst I = e->D.I;
-        I.jpacked = 1;
-        while (w > 0 && team_lds_bytes(I, lb2, w) > 160 * 1024) w--;
+        while (w > 0 && team_lds_bytes(e->D.I, lb2, lb2 ? explore_jtab_bytes(e->D.I) : 0, w) > 160 * 1024) w--;
         e->team_E = w;
     }
     size_t E = (size_t)e->E;

@@ -168,6 +168,7 @@ struct KArgs {
     int bound_mode, branching, refine, pairs_mode, find_all, single_node, initial_ub;
     int steal_margin;
     unsigned ramp;      // nodes an explorer decomposes in a fresh interval before it donates
+    int jt_lds;         // bytes of LDS for the staged Johnson table (0: read from global memory)
 };
 
 // The root order of k_bound_root, passed by value (no upload before the launch).
@@ -187,23 +188,22 @@ struct RootPerm {
 // lanes past a row in stores that would otherwise need an exec mask.
 #define PM_STRIDE 65
 __device__ __host__ inline int lds_pm_stride(int) { return PM_STRIDE; }
-// Words of the staged Johnson table: up to 32 jobs rows of a multiple of 64
+// Bytes of the staged Johnson table: up to 32 jobs rows of a multiple of 64
 // pairs (lb2_walk), above that rows of npairs; not less for a smaller instance
 // in a pool's larger layout.
 __device__ __host__ inline int jtab_chunks(int npairs) { return (npairs + 63) / 64; }
-__device__ __host__ inline size_t jtab_lds_words(int n, int npairs)
+__device__ __host__ inline int jtab_lds_bytes(int n, int npairs)
 {
-    const size_t walk = (size_t)(n < 32 ? n : 32) * 64 * jtab_chunks(npairs);
-    const size_t rows = n > 32 ? (size_t)n * npairs : 0;
-    return walk > rows ? walk : rows;
+    const int walk = (n < 32 ? n : 32) * 64 * jtab_chunks(npairs);
+    const int rows = n > 32 ? n * npairs : 0;
+    return ((walk > rows ? walk : rows) * 4 + 15) & ~15;
 }
-__device__ __host__ inline size_t lds_table_bytes(int n, int m, int npairs, bool lb2)
+// jt: bytes set aside for a Johnson table, a multiple of 16
+__device__ __host__ inline size_t lds_table_bytes(int m, int jt)
 {
     const int mp = (m + 3) & ~3;
-    size_t off = ((size_t)2 * m * PM_STRIDE + 3 * (size_t)mp) * 4;
-    off = (off + 15) & ~(size_t)15;
-    if (lb2) off += (jtab_lds_words(n, npairs) * 4 + 15) & ~(size_t)15;
-    return off;
+    const size_t off = ((size_t)2 * m * PM_STRIDE + 3 * (size_t)mp) * 4;
+    return ((off + 15) & ~(size_t)15) + jt;
 }
 // offset of IVM row l (rows 0..l-1 hold n, n-1, ..., n-l+1 cells)
 __device__ __host__ inline int lds_mat_row(int l, int n) { return l * n - (l * (l - 1)) / 2; }
@@ -218,32 +218,11 @@ __device__ __host__ inline size_t lds_wave_bytes(int n, int m, bool scratch)
 {
     return lds_mat_bytes(n) + lds_stack_bytes(n, m) + (size_t)m * 16 + (scratch ? 64 * 4 : 0) + 64 * 8;
 }
-// The packed Johnson table is staged in LDS when it is at most 24 KB (20
-// machines up to 32 jobs, 13 at any n): the workgroups of the LB2 explorers
-// then stay within a third (engine) and half (20-machine pool) of the CU's LDS,
-// as their registers allow.  Larger ones, and tables of large processing
-// times, are read from global memory (consecutive words per step).
-__device__ __host__ inline bool jtab_in_lds(int n, int npairs) { return jtab_lds_words(n, npairs) * 4 <= 24 * 1024; }
-__device__ __host__ inline bool jtab_staged(const DevInst &I) { return I.jpacked && jtab_in_lds(I.n, I.npairs); }
 // Explorers (wavefronts) per workgroup of the one-instance engine; they share
 // the workgroup's tables.
 #ifndef PBB_EXPLORE_WAVES
 #define PBB_EXPLORE_WAVES 4
 #endif
-inline size_t explore_lds_bytes(const DevInst &I, bool lb2)
-{
-    return lds_table_bytes(I.n, I.m, I.npairs, lb2 && jtab_staged(I)) +
-           PBB_EXPLORE_WAVES * lds_wave_bytes(I.n, I.m, lb2);
-}
-// The team launch (one workgroup) holds at most 16 explorers with LB1 only
-// (4 per SIMD, the register budget of the LB1 explorer) and 8 with a
-// refinement bound (whose explorer needs more than 128 registers).
-__device__ __host__ constexpr int team_waves_max(int ref) { return ref == 0 ? 16 : 8; }
-inline size_t team_lds_bytes(const DevInst &I, bool lb2, int waves)
-{
-    return lds_table_bytes(I.n, I.m, I.npairs, lb2 && jtab_staged(I)) +
-           (size_t)waves * lds_wave_bytes(I.n, I.m, lb2);
-}
 // LDS size handed to the occupancy query of the persistent kernels.  Their
 // explorers wait on one another (hand-overs, the work count), so every
 // workgroup of the grid must be resident at once.  The query's count can be
@@ -252,10 +231,31 @@ inline size_t team_lds_bytes(const DevInst &I, bool lb2, int waves)
 // queried as 3, held 2); rounding each workgroup up to 2 KB keeps the grid
 // inside what the hardware actually co-schedules.
 inline size_t residency_lds_bytes(size_t lds) { return (lds + 2047) & ~(size_t)2047; }
-inline size_t root_lds_bytes(const DevInst &I)
+inline size_t explore_lds_bytes(const DevInst &I, bool lb2, int jt)
 {
-    return lds_table_bytes(I.n, I.m, I.npairs, false) + lds_wave_bytes(I.n, I.m, false);
+    return lds_table_bytes(I.m, jt) + PBB_EXPLORE_WAVES * lds_wave_bytes(I.n, I.m, lb2);
 }
+// The packed Johnson table is staged in LDS when it is at most 24 KB and three of
+// the engine's workgroups still share a CU, as their registers allow (the
+// 20-machine pool's two do then as well): a wider table costs explorers, and an
+// engine holds as many intervals as it has explorers.  That leaves out 59-63 jobs
+// at 14 machines, 54-58 at 15, 49-51 at 16, 43-45 at 17 and 40 at 18 (2048
+// explorers with the table, 3072 without).  What is not staged, and tables of
+// large processing times, are read from global memory (consecutive words per step).
+inline int explore_jtab_bytes(const DevInst &I)
+{
+    const int b = jtab_lds_bytes(I.n, I.npairs);
+    return b <= 24 * 1024 && 3 * residency_lds_bytes(explore_lds_bytes(I, true, b)) <= 160 * 1024 ? b : 0;
+}
+// The team launch (one workgroup) holds at most 16 explorers with LB1 only
+// (4 per SIMD, the register budget of the LB1 explorer) and 8 with a
+// refinement bound (whose explorer needs more than 128 registers).
+__device__ __host__ constexpr int team_waves_max(int ref) { return ref == 0 ? 16 : 8; }
+inline size_t team_lds_bytes(const DevInst &I, bool lb2, int jt, int waves)
+{
+    return lds_table_bytes(I.m, jt) + (size_t)waves * lds_wave_bytes(I.n, I.m, lb2);
+}
+inline size_t root_lds_bytes(const DevInst &I) { return lds_table_bytes(I.m, 0) + lds_wave_bytes(I.n, I.m, false); }
 
 // ------------------------------------------------------------------ pool
 // Many instances in one resident launch.  Workgroups of W explorers take one
@@ -338,7 +338,7 @@ struct PoolArgs {
     int nmax;                     // largest n served
     int pmax;                     // pair-table capacity
     int idle_words;               // idle mask words per slot (64 members each)
-    int jt_lds;                   // packed Johnson tables staged in LDS
+    int jt_lds;                   // bytes of LDS for a staged Johnson table
     int pairs_mode;               // JohnsonMode: pair list built at admission
     int qcap;                     // queue capacity (power of two)
     int sys;                      // req/res/q live in host-mapped memory
@@ -351,9 +351,9 @@ struct PoolArgs {
     int ig_iters;                 // IG helper rounds per instance (0 = no helper wave)
 };
 
-__device__ __host__ inline size_t pool_lds_bytes(int nmax, int M, int pmax, bool jt_lds, int W)
+__device__ __host__ inline size_t pool_lds_bytes(int nmax, int M, int pmax, int jt_lds, int W)
 {
-    return lds_table_bytes(nmax, M, pmax, jt_lds) + (size_t)W * lds_wave_bytes(nmax, M, pmax > 0);
+    return lds_table_bytes(M, jt_lds) + (size_t)W * lds_wave_bytes(nmax, M, pmax > 0);
 }
 
 // per-M kernels (pbb_kernels.hip, one translation unit per M)
@@ -384,7 +384,7 @@ hipError_t launch_neh_m(const int *ptms, const long long *off, const int *ns, co
 __device__ __host__ inline size_t pool_ig_bytes(int M) { return (size_t)IG_THR * 8 + ((size_t)2 * M * 64 + 128) * 4; }
 __device__ __host__ inline size_t pool_lds_total(const PoolArgs &p, int M)
 {
-    return pool_lds_bytes(p.nmax, M, p.pmax, p.jt_lds != 0, p.W) + (p.ig_iters > 0 ? pool_ig_bytes(M) : 0);
+    return pool_lds_bytes(p.nmax, M, p.pmax, p.jt_lds, p.W) + (p.ig_iters > 0 ? pool_ig_bytes(M) : 0);
 }
 template <int M>
 hipError_t launch_ig_m(const int *ptms, const long long *off, const int *ns, const int *ms, int count, int chains,

@@ -128,7 +128,7 @@ template <int M, int REF>
 __global__ __launch_bounds__(64 * PBB_EXPLORE_WAVES, REF == 2 ? 3 : PBB_EXPLORE_MIN_WAVES) void k_explore(KArgs a)
 {
     extern __shared__ __align__(16) char smem[];
-    Lds lds = lds_setup(a.I, smem, REF == 2, REF == 2);
+    Lds lds = lds_setup(a.I, smem, REF == 2 ? a.jt_lds : 0, REF == 2);
     const int e = blockIdx.x * PBB_EXPLORE_WAVES + (threadIdx.x >> 6);
     if (e >= a.E) return;
     explore_loop<M, REF, __HIP_MEMORY_SCOPE_AGENT>(a, lds, e);
@@ -144,7 +144,7 @@ template <int M, int REF>
 __global__ __launch_bounds__(64 * team_waves_max(REF)) void k_team(KArgs a)
 {
     extern __shared__ __align__(16) char smem[];
-    Lds lds = lds_setup(a.I, smem, REF == 2, REF == 2);
+    Lds lds = lds_setup(a.I, smem, REF == 2 ? a.jt_lds : 0, REF == 2);
     const int e = threadIdx.x >> 6;
     if (e >= a.E) return;
     explore_loop<M, REF, __HIP_MEMORY_SCOPE_WORKGROUP>(a, lds, e);
@@ -154,7 +154,7 @@ template <int M>
 __global__ __launch_bounds__(64) void k_bound_root(KArgs a, RootPerm root_perm)
 {
     extern __shared__ __align__(16) char smem[];
-    Lds lds = lds_setup(a.I, smem, false, false);
+    Lds lds = lds_setup(a.I, smem, 0, false);
     Explorer<M, 0> X(a, lds, 0, engine_inst(a), a.ctl, a.I.n, a.I.mp);
     X.local_best = a.initial_ub;
     X.rowv = X.lane < X.n ? root_perm.p[X.lane] : 0;
@@ -177,7 +177,7 @@ template <int M>
 hipError_t launch_explore_m(const KArgs &a, int blocks, hipStream_t s)
 {
     const bool lb2 = a.bound_mode != 0 && a.refine == 1;
-    const size_t lds = explore_lds_bytes(a.I, lb2);
+    const size_t lds = explore_lds_bytes(a.I, lb2, lb2 ? a.jt_lds : 0);
     if (const hipError_t err =
             hipFuncSetAttribute(explore_kernel<M>(a), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
         return err;
@@ -194,7 +194,7 @@ template <int M>
 hipError_t launch_team_m(const KArgs &a, hipStream_t s)
 {
     const bool lb2 = a.bound_mode != 0 && a.refine == 1;
-    const size_t lds = team_lds_bytes(a.I, lb2, a.E);
+    const size_t lds = team_lds_bytes(a.I, lb2, lb2 ? a.jt_lds : 0, a.E);
     const void *k = a.bound_mode == 0 ? (const void *)k_team<M, 0>
                     : a.refine == 1   ? (const void *)k_team<M, 2>
                                       : (const void *)k_team<M, 1>;
@@ -213,7 +213,7 @@ template <int M>
 hipError_t occupancy_m(const KArgs &a, int *blocks_per_cu)
 {
     const bool lb2 = a.bound_mode != 0 && a.refine == 1;
-    const size_t lds = explore_lds_bytes(a.I, lb2);
+    const size_t lds = explore_lds_bytes(a.I, lb2, lb2 ? a.jt_lds : 0);
     if (lds > 160 * 1024) {
         *blocks_per_cu = 0;
         return hipSuccess;

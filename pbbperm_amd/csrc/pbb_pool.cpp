@@ -226,9 +226,10 @@ extern "C" int pbb_pool_create(const pbb_config *cfg, const pbb_pool_params *prm
     p->margin = prm->steal_margin ? prm->steal_margin : cfg->steal_margin;
     const bool lb2 = cfg->bound_mode != 0 && cfg->refine == 1;
     p->pmax = lb2 ? (cfg->johnson_pairs == 0 ? p->M * (p->M - 1) / 2 : p->M - 1) : 0;
-    p->jt_lds = (lb2 && jtab_in_lds(p->nmax, p->pmax)) ? 1 : 0;
+    p->jt_lds = lb2 ? jtab_lds_bytes(p->nmax, p->pmax) : 0;
+    if (p->jt_lds > 24 * 1024) p->jt_lds = 0;
     p->ig = p->W >= 2 ? prm->ig_iterations : 0;
-    p->lds = pool_lds_bytes(p->nmax, p->M, p->pmax, p->jt_lds != 0, p->W) + (p->ig ? pool_ig_bytes(p->M) : 0);
+    p->lds = pool_lds_bytes(p->nmax, p->M, p->pmax, p->jt_lds, p->W) + (p->ig ? pool_ig_bytes(p->M) : 0);
     p->qcap = next_pow2(std::max(64, prm->slots));
 #define TRY(x)              \
     do {                    \

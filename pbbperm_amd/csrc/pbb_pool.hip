@@ -415,7 +415,7 @@ __device__ __forceinline__ void pool_ig_helper(const Lds &lds, int n, int e, con
 {
     const int lane = lane_id();
     unsigned long long *thr =
-        (unsigned long long *)(smem + pool_lds_bytes(p.nmax, M, p.pmax, p.jt_lds != 0, p.W));
+        (unsigned long long *)(smem + pool_lds_bytes(p.nmax, M, p.pmax, p.jt_lds, p.W));
     int *spt = (int *)(thr + IG_THR);
     int *hd = spt + 64, *tl = hd + M * 64, *scr = tl + M * 64;
     int tot = 0;
@@ -500,7 +500,7 @@ __global__ __launch_bounds__(256, PBB_POOL_MIN_WAVES(M)) void k_pool(KArgs a, Po
         } else {
             const int n = uni(ld_rlx(&S->n)), m = uni(ld_rlx(&S->m)), npairs = uni(ld_rlx(&S->npairs));
             const DevInst I = slot_inst<M>(p, slot, n, npairs, uni(ld_rlx(&S->jpacked)));
-            const Lds lds = lds_setup(I, smem, p.jt_lds != 0, REF == 2);
+            const Lds lds = lds_setup(I, smem, p.jt_lds, REF == 2);
             if (role == ROLE_OWNER) {
                 // a request without an incumbent gets NEH's (ub < 0)
                 if (wave == 0 && uni(ld_rlx(&S->ub)) < 0) {
