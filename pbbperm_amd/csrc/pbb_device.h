@@ -227,26 +227,47 @@ __device__ __forceinline__ int lb2_pairs(const int (&pinfo)[PCH], const void *jt
     return lb2_finish<PCH, ST>(pinfo, best, fs, gs);
 }
 
-// Word of the staged table of up to 32 jobs, row i of a pair's column: w of the
-// i-th job of the pair's order in bits 0-15, the place of job i in that order in
-// 16-20, p_a - p_b of the i-th job in 21-31.
-__device__ __forceinline__ unsigned jwalk_word(unsigned e) { return ((e >> 6) & 0x7fffu) | (e & 0xffe00000u); }
-__device__ __forceinline__ unsigned jwalk_place(unsigned w) { return (w >> 16) & 31u; }
+// Entry of the staged table of up to 32 jobs, row i of a pair's column: w of the
+// i-th job of the pair's order, the place of job i in that order and p_a - p_b of
+// the i-th job.  Packed in one word: w in bits 0-15, the place in 16-20, the
+// difference in 21-31; wide in two: w (at most 19 x 10^6) in bits 0-24 and the place
+// in 25-29, the difference.
+template <bool WIDE>
+struct JWalk {
+    typedef unsigned Entry;
+    static constexpr int PLACE = 16;
+    __device__ __forceinline__ static Entry make(unsigned e)
+    {
+        return ((e >> 6) & 0x7fffu) | (e & 0xffe00000u);
+    }
+    __device__ __forceinline__ static int w(Entry e) { return (int)(e & 0xffffu); }
+    __device__ __forceinline__ static int diff(Entry e) { return (int)e >> 21; }
+};
+template <>
+struct JWalk<true> {
+    typedef int2 Entry;
+    static constexpr int PLACE = 25;
+    __device__ __forceinline__ static Entry make(int2 e) { return make_int2(e.x, e.y >> 6); }
+    __device__ __forceinline__ static int w(Entry e) { return e.x & 0x1ffffff; }
+    __device__ __forceinline__ static int diff(Entry e) { return e.y; }
+};
 
 // The recurrence of lb2_pairs for K children over NCH chunks of 64 pairs, cnt
 // steps: places[k][c] has a bit per unscheduled job, at its place in the order
 // of this lane's pair, so a step takes the next unscheduled job and the
 // scheduled ones cost nothing (7 instructions for each of the n jobs there, 9
 // for each unscheduled one here, and those are a third to two thirds of n).
-// Rows are a multiple of 64 words apart, so the lanes of a wavefront read
+// Rows are a multiple of 64 entries apart, so the lanes of a wavefront read
 // distinct banks whatever their places.  512-instance batch 101 -> 86 ms, burst of
 // 256 requests 64 -> 46, 30x20 LB2 proof 4.26 -> 4.04.  D and best enter as the children's front
 // times on the pair's machines; best leaves without the remaining work.
-template <int K, int NCH>
+template <int K, int NCH, bool WIDE>
 __device__ __forceinline__ void lb2_walk(const unsigned *tab, int cnt, unsigned (&places)[K][NCH], int (&D)[K][NCH],
                                          int (&best)[K][NCH])
 {
-    const char *col = (const char *)(tab + lane_id());
+    typedef typename JWalk<WIDE>::Entry Entry;
+    constexpr unsigned row = 64u * sizeof(Entry);
+    const char *col = (const char *)((const Entry *)tab + lane_id());
 #pragma unroll 2
     for (int i = 0; i < cnt; i++) {
 #pragma unroll
@@ -255,9 +276,9 @@ __device__ __forceinline__ void lb2_walk(const unsigned *tab, int cnt, unsigned 
             for (int k = 0; k < K; k++) {
                 const unsigned p = (unsigned)__builtin_ctz(places[k][c]);
                 places[k][c] &= places[k][c] - 1u;
-                const unsigned e = *(const unsigned *)(col + p * (256u * NCH) + c * 256);
-                best[k][c] = max(best[k][c], D[k][c] + (int)(e & 0xffffu));
-                D[k][c] += (int)e >> 21;
+                const Entry e = *(const Entry *)(col + p * (row * NCH) + c * row);
+                best[k][c] = max(best[k][c], D[k][c] + JWalk<WIDE>::w(e));
+                D[k][c] += JWalk<WIDE>::diff(e);
             }
         }
     }
@@ -305,16 +326,22 @@ __device__ __forceinline__ int lb2_few(const int (&pinfo)[PCH], const unsigned *
     return lb2_finish<PCH, ST>(pinfo, best, fs, gs);
 }
 
+// Forms of the Johnson table that an explorer is built for.  The engine has a
+// kernel for each (its node loop's registers and code are then one form's); the
+// pool's launch meets both, and walks the packed one only.
+enum { TAB_ANY = 0, TAB_PACKED = 1, TAB_WIDE = 2 };
+
 // lb2_pairs of an explorer's child where lb2_walk's table does not apply: the
-// packed table of more than 32 jobs in LDS, the packed or the wide one in global
-// memory
-template <int PCH>
+// table of more than 32 jobs in LDS, any in global memory
+template <int PCH, int TAB>
 __device__ __forceinline__ int lb2_pairs_any(const int (&pinfo)[PCH], bool staged, const unsigned *jtabL,
                                              const void *jtabG, bool packed, int n, int npairs, const int *fs,
                                              const int *gs, uint64_t unsched)
 {
-    if (staged) return lb2_pairs<PCH, false, true, 1>(pinfo, jtabL, n, npairs, fs, gs, unsched);
-    return packed ? lb2_pairs<PCH, false, true, 1>(pinfo, jtabG, n, npairs, fs, gs, unsched)
+    if (TAB == TAB_PACKED || (TAB == TAB_ANY && packed))
+        return staged ? lb2_pairs<PCH, false, true, 1>(pinfo, jtabL, n, npairs, fs, gs, unsched)
+                      : lb2_pairs<PCH, false, true, 1>(pinfo, jtabG, n, npairs, fs, gs, unsched);
+    return staged ? lb2_pairs<PCH, false, false, 1>(pinfo, jtabL, n, npairs, fs, gs, unsched)
                   : lb2_pairs<PCH, false, false, 1>(pinfo, jtabG, n, npairs, fs, gs, unsched);
 }
 

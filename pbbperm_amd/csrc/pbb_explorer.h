@@ -124,7 +124,7 @@ struct Lds {
     int *pmR;       // the same rows, machines reversed: pmR[q] = pm[m-1-q]
     int ps;         // row stride of pm (PM_STRIDE)
     int *minA, *minD, *tot;
-    unsigned *jtabL;    // packed Johnson table staged in LDS (valid when jtl)
+    unsigned *jtabL;    // Johnson table staged in LDS (valid when jtl)
     const void *jtabG;  // the table in global memory
     bool jtl, jpacked;
     int nch;        // chunks of 64 pairs (jtwalk)
@@ -138,7 +138,29 @@ struct Lds {
                     // (2066 against 2100-2104 M nodes/s at 50x20)
 };
 
+// lb2_walk's table from the one in global memory, by the whole workgroup: a thread
+// per column (the columns past the last pair repeat it), a second pass for the
+// places.
+template <bool WIDE, class Src, class Entry>
+__device__ __forceinline__ void stage_walk(const Src *src, Entry *tab, int n, int npairs, int nch)
+{
+    const int width = 64 * nch;
+    for (int c = threadIdx.x; c < width; c += blockDim.x) {
+        const Src *s = src + min(c, npairs - 1);
+#pragma unroll 4
+        for (int i = 0; i < n; i++) tab[i * width + c] = JWalk<WIDE>::make(s[i * npairs]);
+#pragma unroll 4
+        for (int i = 0; i < n; i++) {
+            unsigned job;
+            if constexpr (WIDE) job = (unsigned)s[i * npairs].y & 63u;
+            else job = s[i * npairs] & 63u;
+            atomicOr((unsigned *)(tab + (int)job * width + c), (unsigned)i << JWalk<WIDE>::PLACE);
+        }
+    }
+}
+
 // jt: bytes set aside for a Johnson table; an instance's is staged if it fits
+template <int TAB>
 __device__ __forceinline__ Lds lds_setup(const DevInst &I, char *smem, int jt, bool scratch)
 {
     Lds L;
@@ -149,13 +171,16 @@ __device__ __forceinline__ Lds lds_setup(const DevInst &I, char *smem, int jt, b
     L.minA = L.pmR + m * PM_STRIDE;
     L.minD = L.minA + mp;
     L.tot = L.minD + mp;
-    const bool load_jtab = jt > 0 && I.jpacked && jtab_lds_bytes(n, I.npairs) <= jt;
+    const bool packed = TAB == TAB_PACKED || (TAB == TAB_ANY && I.jpacked);
+    const bool walk = n <= 32 && (TAB != TAB_ANY || packed);
+    const int bytes = TAB != TAB_ANY || packed ? jtab_lds_bytes(n, I.npairs, packed) : n * I.npairs * 8;
+    const bool load_jtab = jt > 0 && bytes <= jt;
     L.jtabL = (unsigned *)(smem + lds_table_bytes(m, 0));
-    L.jpacked = I.jpacked != 0;
+    L.jpacked = packed;
     L.jtabG = I.jtab;
     L.jtl = load_jtab;
     L.nch = jtab_chunks(I.npairs);
-    L.jtwalk = load_jtab && n <= 32;
+    L.jtwalk = load_jtab && walk;
     char *wbase = smem + lds_table_bytes(m, jt) +
                   (size_t)(threadIdx.x >> 6) * lds_wave_bytes(n, m, scratch);
     L.mat = (int8_t *)wbase;
@@ -177,19 +202,12 @@ __device__ __forceinline__ Lds lds_setup(const DevInst &I, char *smem, int jt, b
         L.tot[i] = s;
     }
     if (L.jtwalk) {
-        // a thread per column; the columns past the last pair repeat it
-        const unsigned *src = (const unsigned *)I.jtab;
-        const int width = 64 * L.nch;
-        for (int c = threadIdx.x; c < width; c += blockDim.x) {
-            const int p = min(c, I.npairs - 1);
-#pragma unroll 4
-            for (int i = 0; i < n; i++) L.jtabL[i * width + c] = jwalk_word(src[i * I.npairs + p]);
-#pragma unroll 4
-            for (int i = 0; i < n; i++)
-                atomicOr(&L.jtabL[(int)(src[i * I.npairs + p] & 63u) * width + c], (unsigned)i << 16);
-        }
+        if constexpr (TAB == TAB_WIDE) stage_walk<true>((const int2 *)I.jtab, (int2 *)L.jtabL, n, I.npairs, L.nch);
+        else stage_walk<false>((const unsigned *)I.jtab, L.jtabL, n, I.npairs, L.nch);
     } else if (load_jtab) {
-        for (int i = threadIdx.x; i < I.npairs * n; i += blockDim.x) L.jtabL[i] = ((const unsigned *)I.jtab)[i];
+        const int words = I.npairs * n * (packed ? 1 : 2);
+#pragma unroll 4
+        for (int i = threadIdx.x; i < words; i += blockDim.x) L.jtabL[i] = ((const unsigned *)I.jtab)[i];
     }
     __syncthreads();
     return L;
@@ -283,8 +301,9 @@ __device__ __forceinline__ InstRef engine_inst(const KArgs &a)
 // its tail).
 // REF: 0 LB1 only (boundingMode 0); 1 LB1 + LB1' refinement (boundingMode
 // 1/2 as shipped); 2 LB1 + Johnson LB2 refinement.
-template <int M, int REF, int SC = __HIP_MEMORY_SCOPE_AGENT>
+template <int M, int REF, int SC = __HIP_MEMORY_SCOPE_AGENT, int TAB = TAB_ANY>
 struct Explorer {
+    static constexpr bool WIDE = TAB == TAB_WIDE;  // form of lb2_walk's table
     const KArgs &a;
     Lds lds;
     InstRef ir;   // the instance this explorer works on
@@ -354,11 +373,15 @@ struct Explorer {
         return lane < M ? v : 0;
     }
 
+    __device__ __forceinline__ int walk_place(int at) const
+    {
+        return (int)((lds.jtabL[WIDE ? 2 * at : at] >> JWalk<WIDE>::PLACE) & 31u);
+    }
     // job j's bit in the place masks: one LDS word per chunk, kept up along the
     // path (rebuilt for every node, it costs what the shorter walk saves)
     __device__ __forceinline__ unsigned place_bit(int c, int j) const
     {
-        return 1u << jwalk_place(lds.jtabL[(j * lds.nch + c) * 64 + lane]);
+        return 1u << walk_place((j * lds.nch + c) * 64 + lane);
     }
     template <bool ADD>
     __device__ __forceinline__ void mark_places(int j)
@@ -696,8 +719,8 @@ struct Explorer {
         } else {
 #pragma unroll
             for (int i = 0; i < K; i++)
-                r[i] = lb2_pairs_any<PCH>(pinfo, lds.jtl, lds.jtabL, lds.jtabG, lds.jpacked, n, ir.npairs, fs + 32 * i,
-                                          gs + 32 * i, free_jobs & ~(1ull << (i ? j1 : j0)));
+                r[i] = lb2_pairs_any<PCH, TAB>(pinfo, lds.jtl, lds.jtabL, lds.jtabG, lds.jpacked, n, ir.npairs,
+                                               fs + 32 * i, gs + 32 * i, free_jobs & ~(1ull << (i ? j1 : j0)));
         }
         if (K == 1) r[1] = r[0];
         const auto h = __builtin_amdgcn_permlane32_swap(r[0], r[1], false, false);
@@ -718,13 +741,13 @@ struct Explorer {
             const int info = pinfo[c] < 0 ? 0 : pinfo[c], a = info & 0xff, b = info >> 8;
 #pragma unroll
             for (int i = 0; i < K; i++) {
-                pl[i][c] = places[c] & ~(1u << jwalk_place(lds.jtabL[((i ? j1 : j0) * NCH + c) * 64 + lane]));
+                pl[i][c] = places[c] & ~(1u << walk_place(((i ? j1 : j0) * NCH + c) * 64 + lane));
                 D[i][c] = fs[32 * i + a];
                 best[i][c] = fs[32 * i + b];
                 end[i][c] = D[i][c] + gs[32 * i + a];
             }
         }
-        lb2_walk<K, NCH>(lds.jtabL, cnt, pl, D, best);
+        lb2_walk<K, NCH, WIDE>(lds.jtabL, cnt, pl, D, best);
 #pragma unroll
         for (int i = 0; i < K; i++) {
             r[i] = 0;

@@ -239,11 +239,25 @@ extern "C" int pbb_makespan_batch(pbb_bounds *b, int count, const int *perms, in
 }
 
 // ------------------------------------------------------------------ engine
+// Launches with one form of the Johnson table: the bytes of LDS it is staged in (0:
+// read from global memory), the explorers that are resident with them and the
+// explorers of the team launch (0: none fits).  The resident ones can be fewer than
+// the engine's (a wide table of 30 jobs and 20 machines, 46 KB, leaves one or two
+// workgroups per CU); a launch then uses the table with so many as long as they
+// hold all intervals, else all explorers without it.  A wide table is staged whatever
+// it costs: read from global memory beside thousands of polling explorers, a step
+// of the recurrence takes a memory round trip (times of 11 to 1089, global / staged:
+// 18x20, 3065 nodes 11.5 / 1.7 ms; 30x20, 268 k nodes 35 / 3.7 ms; 45x17, 28 k nodes
+// 23 / 3.8 ms).
+struct JForm {
+    int bytes, explorers, team;
+};
+
 struct pbb_engine {
     pbb_config cfg;
     HostTables T;
     DevTables D;
-    int n, m, E, blocks;
+    int n, m, E;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // device buffers, in one allocation
@@ -261,6 +275,8 @@ struct pbb_engine {
     // the incumbent word after a launch
     Ctl *ctl_h = nullptr;
     unsigned long long *best_h = nullptr;
+    JForm form[2]{};  // wide, packed (DevInst::jpacked)
+    int top = 0;      // all intervals are held by explorers below this
     // host state
     std::vector<int> root_perm;
     int inc_cost;
@@ -276,9 +292,7 @@ struct pbb_engine {
     // set-up or launch (nothing else writes them between launches)
     bool done_host = false;
     unsigned long long dec_dev = 0;
-    // the team launch: its explorer count (0: none fits) and whether the
-    // next pbb_run starts with it (set by pbb_init_full)
-    int team_E = 0;
+    // whether the next pbb_run starts with the team launch (set by pbb_init_full)
     bool team_pending = false;
     double last_ms = 0.0;
     int wall_khz = 100000;
@@ -300,7 +314,6 @@ static KArgs make_args(pbb_engine *e)
     a.mbox = e->mbox;
     a.idle = e->idle;
     a.idle_words = idle_words_for(e->E);
-    a.jt_lds = e->D.I.jpacked ? explore_jtab_bytes(e->D.I) : 0;
     a.ctl = e->ctl;
     a.best = e->best;
     a.best_perm = e->best_perm;
@@ -330,10 +343,12 @@ static hipError_t copy_sync(pbb_engine *e, void *dst, const void *src, size_t by
     return r;
 }
 
-static int capacity(pbb_engine *e, int *explorers)
+// resident explorers of a device-wide launch of the given form with jt bytes of LDS for its table
+static int capacity(pbb_engine *e, int packed, int jt, int *explorers)
 {
     KArgs a = make_args(e);
-    a.jt_lds = explore_jtab_bytes(a.I);  // staged or not: a retargeted engine keeps its explorers
+    a.I.jpacked = packed;
+    a.jt_lds = jt;
     int bpc = 0;
     HIPCHK(explore_occupancy(a, &bpc));
     if (bpc < 1) return fail(PBB_E_CAPACITY, "explorer kernel does not fit one workgroup per CU (LDS)");
@@ -344,6 +359,47 @@ static int capacity(pbb_engine *e, int *explorers)
     *explorers = bpc * cus * PBB_EXPLORE_WAVES;
     return PBB_OK;
 }
+
+static bool with_lb2(const pbb_engine *e) { return e->cfg.bound_mode != 0 && e->cfg.refine == 1; }
+
+// The engine's explorers: what is resident of either form, so that a retargeted
+// engine keeps them.
+static int engine_explorers(pbb_engine *e)
+{
+    int cap = 0, wide = 0;
+    const bool lb2 = with_lb2(e);
+    if (const int rc = capacity(e, 1, lb2 ? explore_jtab_bytes(e->D.I) : 0, &cap)) return rc;
+    if (lb2) {
+        if (const int rc = capacity(e, 0, 0, &wide)) return rc;
+        cap = std::min(cap, wide);
+    }
+    e->E = std::max(1, std::min(e->cfg.nb_ivms, cap));
+    return PBB_OK;
+}
+
+// The present form's launches (JForm), found once per form.
+static int plan_form(pbb_engine *e)
+{
+    const int packed = e->D.I.jpacked;
+    JForm &f = e->form[packed];
+    if (f.explorers) return PBB_OK;
+    const bool lb2 = with_lb2(e);
+    JForm g{0, e->E, 0};
+    if (lb2) g.bytes = jtab_lds_bytes(e->n, e->D.I.npairs, packed);
+    if (packed ? g.bytes > JTAB_PACKED_MOST : explore_lds_bytes(e->D.I, lb2, g.bytes) > 160 * 1024) g.bytes = 0;
+    if (g.bytes && !(packed && g.bytes == explore_jtab_bytes(e->D.I))) {
+        int cap = 0;
+        if (const int rc = capacity(e, packed, g.bytes, &cap)) return rc;
+        g.explorers = std::min(e->E, cap);
+    }
+    // the team: up to team_waves_max explorers whose LDS fits one workgroup
+    g.team = std::min(e->E, team_waves_max(e->cfg.bound_mode == 0 ? 0 : (lb2 ? 2 : 1)));
+    if (e->cfg.team_waves > 0) g.team = std::min(g.team, e->cfg.team_waves);
+    while (g.team > 0 && team_lds_bytes(e->D.I, lb2, g.bytes, g.team) > 160 * 1024) g.team--;
+    f = g;
+    return PBB_OK;
+}
+static const JForm &form_of(const pbb_engine *e) { return e->form[e->D.I.jpacked]; }
 
 extern "C" int pbb_destroy(pbb_engine *e)
 {
@@ -395,19 +451,8 @@ extern "C" int pbb_create(const int32_t *ptm, int n, int m, const pbb_config *cf
     HTRY(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
     HTRY(hipEventCreate(&e->ev0));
     HTRY(hipEventCreate(&e->ev1));
-    int cap = 0;
-    TRY(capacity(e, &cap));
-    e->E = std::max(1, std::min(cfg->nb_ivms, cap));
-    e->blocks = (e->E + PBB_EXPLORE_WAVES - 1) / PBB_EXPLORE_WAVES;
-    {
-        // the team: up to team_waves_max explorers whose LDS fits one workgroup
-        const bool lb2 = cfg->bound_mode != 0 && cfg->refine == 1;
-        const int ref = cfg->bound_mode == 0 ? 0 : (cfg->refine == 1 ? 2 : 1);
-        int w = std::min(e->E, team_waves_max(ref));
-        if (cfg->team_waves > 0) w = std::min(w, cfg->team_waves);
-        while (w > 0 && team_lds_bytes(e->D.I, lb2, lb2 ? explore_jtab_bytes(e->D.I) : 0, w) > 160 * 1024) w--;
-        e->team_E = w;
-    }
+    TRY(engine_explorers(e));
+    TRY(plan_form(e));
     size_t E = (size_t)e->E;
     // cleared once: mailboxes, idle mask, state words, tags
     const size_t idle_bytes = (size_t)idle_words_for(e->E) * IDLE_STRIDE * 8;
@@ -534,6 +579,7 @@ static int setup_pool(pbb_engine *e, const std::vector<int> &ids, const int *pos
     e->done_host = c.done != 0;
     e->dec_dev = 0;
     e->team_pending = false;
+    e->top = ids.empty() ? 0 : *std::max_element(ids.begin(), ids.end()) + 1;
     e->initialized = true;
     return PBB_OK;
 }
@@ -552,8 +598,9 @@ extern "C" int pbb_init_full(pbb_engine *e)
     e->dec_base = e->sb_base = 0;
     e->done_host = false;
     e->dec_dev = 0;
+    e->top = 1;
     e->initialized = true;
-    e->team_pending = e->team_E > 0 && e->cfg.team_nodes > 0;
+    e->team_pending = form_of(e).team > 0 && e->cfg.team_nodes > 0;
     return PBB_OK;
 }
 
@@ -589,17 +636,23 @@ static int launch_once(pbb_engine *e, bool team, uint64_t node_budget, uint64_t 
 {
     *e->host_flag = 0;
     KArgs a = make_args(e);
+    const JForm &f = form_of(e);
     if (team) {
-        a.E = e->team_E;
-        a.idle_words = idle_words_for(a.E);
+        a.E = f.team;
+        a.jt_lds = f.bytes;
+    } else if (f.bytes && e->top <= f.explorers) {
+        a.E = f.explorers;
+        a.jt_lds = f.bytes;
     }
+    a.idle_words = idle_words_for(a.E);
+    e->top = std::max(e->top, a.E);
     a.node_budget = node_budget ? e->dec_dev + node_budget : 0;
     a.quiet_budget = e->dec_dev + quiet_budget;
     a.deadline = time_budget_s > 0 ? (unsigned long long)(time_budget_s * e->wall_khz * 1000.0) : 0;
     HIPCHK(launch_prelaunch(a, e->stream));
     HIPCHK(hipEventRecord(e->ev0, e->stream));
     if (team) HIPCHK(launch_team(a, e->stream));
-    else HIPCHK(launch_explore(a, e->blocks, e->stream));
+    else HIPCHK(launch_explore(a, (a.E + PBB_EXPLORE_WAVES - 1) / PBB_EXPLORE_WAVES, e->stream));
     HIPCHK(hipEventRecord(e->ev1, e->stream));
     HIPCHK(hipMemcpyAsync(e->ctl_h, e->ctl, sizeof(Ctl), hipMemcpyDeviceToHost, e->stream));
     HIPCHK(hipMemcpyAsync(e->best_h, e->best, 8, hipMemcpyDeviceToHost, e->stream));
@@ -635,7 +688,7 @@ static TeamBudget team_budget(const pbb_engine *e, uint64_t node_budget)
 {
     const uint64_t most = (uint64_t)e->cfg.team_nodes;
     if (node_budget && node_budget <= most) return {node_budget, node_budget};
-    if (e->cfg.team_nodes != PBB_TEAM_NODES_DEFAULT || e->E <= e->team_E) return {most, most};
+    if (e->cfg.team_nodes != PBB_TEAM_NODES_DEFAULT || e->E <= form_of(e).team) return {most, most};
     if (e->cfg.bound_mode == 0) return {most / 2, most};
     return {most / 8, most / 8};
 }
@@ -848,6 +901,7 @@ static int engine_retarget(pbb_engine *e, const int32_t *ptm, int ub, const int 
     const std::vector<char> v = pack_tables(T);
     HIPCHK(copy_sync(e, e->D.mem, v.data(), v.size(), hipMemcpyHostToDevice));
     e->D.I.jpacked = T.jpacked ? 1 : 0;
+    if (const int rc = plan_form(e)) return rc;
     e->inc_cost = ub;
     e->initial_ub = ub;
     for (int i = 0; i < e->n; i++) {

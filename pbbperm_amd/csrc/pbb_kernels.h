@@ -188,15 +188,15 @@ struct RootPerm {
 // lanes past a row in stores that would otherwise need an exec mask.
 #define PM_STRIDE 65
 __device__ __host__ inline int lds_pm_stride(int) { return PM_STRIDE; }
-// Bytes of the staged Johnson table: up to 32 jobs rows of a multiple of 64
-// pairs (lb2_walk), above that rows of npairs; not less for a smaller instance
-// in a pool's larger layout.
+// Bytes of the staged Johnson table, packed or wide: up to 32 jobs rows of a
+// multiple of 64 pairs (lb2_walk), above that rows of npairs; not less for a
+// smaller instance in a pool's larger layout.
 __device__ __host__ inline int jtab_chunks(int npairs) { return (npairs + 63) / 64; }
-__device__ __host__ inline int jtab_lds_bytes(int n, int npairs)
+__device__ __host__ inline int jtab_lds_bytes(int n, int npairs, bool packed)
 {
     const int walk = (n < 32 ? n : 32) * 64 * jtab_chunks(npairs);
     const int rows = n > 32 ? n * npairs : 0;
-    return ((walk > rows ? walk : rows) * 4 + 15) & ~15;
+    return ((walk > rows ? walk : rows) * (packed ? 4 : 8) + 15) & ~15;
 }
 // jt: bytes set aside for a Johnson table, a multiple of 16
 __device__ __host__ inline size_t lds_table_bytes(int m, int jt)
@@ -235,17 +235,20 @@ inline size_t explore_lds_bytes(const DevInst &I, bool lb2, int jt)
 {
     return lds_table_bytes(I.m, jt) + PBB_EXPLORE_WAVES * lds_wave_bytes(I.n, I.m, lb2);
 }
-// The packed Johnson table is staged in LDS when it is at most 24 KB and three of
-// the engine's workgroups still share a CU, as their registers allow (the
-// 20-machine pool's two do then as well): a wider table costs explorers, and an
-// engine holds as many intervals as it has explorers.  That leaves out 59-63 jobs
-// at 14 machines, 54-58 at 15, 49-51 at 16, 43-45 at 17 and 40 at 18 (2048
-// explorers with the table, 3072 without).  What is not staged, and tables of
-// large processing times, are read from global memory (consecutive words per step).
+// The packed Johnson table is staged in LDS when it is at most 24 KB: 20 machines up
+// to 32 jobs, 14 at any n.  What is not staged is read from global memory
+// (consecutive words per step).
+#define JTAB_PACKED_MOST (24 * 1024)
+// The bytes an engine's number of explorers is found with: those of the packed
+// table where three workgroups still share a CU, as their registers allow (the
+// 20-machine pool's two do then as well), else none.  An engine holds as many
+// intervals as it has explorers, whatever its times.  The shapes of "none": 59-63
+// jobs at 14 machines, 54-58 at 15, 49-51 at 16, 43-45 at 17, 40 at 18 (2048
+// explorers with the table, 3072 without), and tables above the limit.
 inline int explore_jtab_bytes(const DevInst &I)
 {
-    const int b = jtab_lds_bytes(I.n, I.npairs);
-    return b <= 24 * 1024 && 3 * residency_lds_bytes(explore_lds_bytes(I, true, b)) <= 160 * 1024 ? b : 0;
+    const int b = jtab_lds_bytes(I.n, I.npairs, true);
+    return b <= JTAB_PACKED_MOST && 3 * residency_lds_bytes(explore_lds_bytes(I, true, b)) <= 160 * 1024 ? b : 0;
 }
 // The team launch (one workgroup) holds at most 16 explorers with LB1 only
 // (4 per SIMD, the register budget of the LB1 explorer) and 8 with a

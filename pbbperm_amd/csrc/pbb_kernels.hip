@@ -1,6 +1,6 @@
 // pbb_kernels.hip -- gfx950 kernels of the IVM branch-and-bound engine.
 //
-//   k_explore<M,REF> persistent explorer kernel: one IVM per 64-lane
+//   k_explore<M,REF,TAB> persistent explorer kernel: one IVM per 64-lane
 //                  wavefront, 4 explorers per 256-thread workgroup.  The IVM
 //                  matrix (int8 rows) and the front/back completion-time
 //                  stacks of each explorer live in LDS; the interval vectors
@@ -15,7 +15,8 @@
 //                  trip until the run ends (all idle, node budget, deadline
 //                  or interrupt).  REF selects the bounding variant at
 //                  compile time: 0 LB1 only (boundingMode 0), 1 LB1 + LB1'
-//                  refinement (modes 1/2 as shipped), 2 LB1 + Johnson LB2.
+//                  refinement (modes 1/2 as shipped), 2 LB1 + Johnson LB2,
+//                  of the table form TAB.
 //   k_bound_root<M> LB1 root bounding, ivm_bound::boundRoot (ivm_bound.cpp:273-330).
 //
 // Translation units: this file is compiled once per machine count M
@@ -33,10 +34,10 @@ namespace pbb {
 
 // The explorer loop of one wavefront (explorer e); SC is the memory scope of
 // the explorers it shares work with.
-template <int M, int REF, int SC>
+template <int M, int REF, int TAB, int SC>
 __device__ __forceinline__ void explore_loop(const KArgs &a, const Lds &lds, int e)
 {
-    Explorer<M, REF, SC> X(a, lds, e, engine_inst(a), a.ctl, a.I.n, a.I.mp);
+    Explorer<M, REF, SC, TAB> X(a, lds, e, engine_inst(a), a.ctl, a.I.n, a.I.mp);
     X.local_best = uni((int)(unsigned)(ld_rlx<SC>(a.best) >> 32));
     X.open_mail();
     X.join(e);
@@ -124,14 +125,14 @@ __device__ __forceinline__ void explore_loop(const KArgs &a, const Lds &lds, int
     }
 }
 
-template <int M, int REF>
+template <int M, int REF, int TAB>
 __global__ __launch_bounds__(64 * PBB_EXPLORE_WAVES, REF == 2 ? 3 : PBB_EXPLORE_MIN_WAVES) void k_explore(KArgs a)
 {
     extern __shared__ __align__(16) char smem[];
-    Lds lds = lds_setup(a.I, smem, REF == 2 ? a.jt_lds : 0, REF == 2);
+    Lds lds = lds_setup<TAB>(a.I, smem, REF == 2 ? a.jt_lds : 0, REF == 2);
     const int e = blockIdx.x * PBB_EXPLORE_WAVES + (threadIdx.x >> 6);
     if (e >= a.E) return;
-    explore_loop<M, REF, __HIP_MEMORY_SCOPE_AGENT>(a, lds, e);
+    explore_loop<M, REF, TAB, __HIP_MEMORY_SCOPE_AGENT>(a, lds, e);
 }
 
 // The team launch: explorers 0..a.E-1 as the wavefronts of one workgroup
@@ -140,21 +141,21 @@ __global__ __launch_bounds__(64 * PBB_EXPLORE_WAVES, REF == 2 ? 3 : PBB_EXPLORE_
 // by the team alone, without the cross-XCD writebacks and invalidates that
 // every hand-over costs in a device-wide launch; a larger one stops at the
 // node budget and the device-wide launch resumes from the saved intervals.
-template <int M, int REF>
+template <int M, int REF, int TAB>
 __global__ __launch_bounds__(64 * team_waves_max(REF)) void k_team(KArgs a)
 {
     extern __shared__ __align__(16) char smem[];
-    Lds lds = lds_setup(a.I, smem, REF == 2 ? a.jt_lds : 0, REF == 2);
+    Lds lds = lds_setup<TAB>(a.I, smem, REF == 2 ? a.jt_lds : 0, REF == 2);
     const int e = threadIdx.x >> 6;
     if (e >= a.E) return;
-    explore_loop<M, REF, __HIP_MEMORY_SCOPE_WORKGROUP>(a, lds, e);
+    explore_loop<M, REF, TAB, __HIP_MEMORY_SCOPE_WORKGROUP>(a, lds, e);
 }
 
 template <int M>
 __global__ __launch_bounds__(64) void k_bound_root(KArgs a, RootPerm root_perm)
 {
     extern __shared__ __align__(16) char smem[];
-    Lds lds = lds_setup(a.I, smem, 0, false);
+    Lds lds = lds_setup<TAB_PACKED>(a.I, smem, 0, false);
     Explorer<M, 0> X(a, lds, 0, engine_inst(a), a.ctl, a.I.n, a.I.mp);
     X.local_best = a.initial_ub;
     X.rowv = X.lane < X.n ? root_perm.p[X.lane] : 0;
@@ -166,11 +167,27 @@ __global__ __launch_bounds__(64) void k_bound_root(KArgs a, RootPerm root_perm)
 }
 
 // ---------------------------------------------------------- host launchers
+// the kernel of a bounding variant and, with LB2, of a table form
 template <int M>
 static const void *explore_kernel(const KArgs &a)
 {
-    if (a.bound_mode == 0) return (const void *)k_explore<M, 0>;
-    return a.refine == 1 ? (const void *)k_explore<M, 2> : (const void *)k_explore<M, 1>;
+    if (a.bound_mode == 0) return (const void *)k_explore<M, 0, TAB_PACKED>;
+    if (a.refine != 1) return (const void *)k_explore<M, 1, TAB_PACKED>;
+    return a.I.jpacked ? (const void *)k_explore<M, 2, TAB_PACKED> : (const void *)k_explore<M, 2, TAB_WIDE>;
+}
+template <int M>
+static const void *team_kernel(const KArgs &a)
+{
+    if (a.bound_mode == 0) return (const void *)k_team<M, 0, TAB_PACKED>;
+    if (a.refine != 1) return (const void *)k_team<M, 1, TAB_PACKED>;
+    return a.I.jpacked ? (const void *)k_team<M, 2, TAB_PACKED> : (const void *)k_team<M, 2, TAB_WIDE>;
+}
+
+static hipError_t launch_kernel(const void *k, int blocks, int threads, size_t lds, const KArgs &a, hipStream_t s)
+{
+    if (const hipError_t err = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)) return err;
+    void *args[] = {(void *)&a};
+    return hipLaunchKernel(k, dim3(blocks), dim3(threads), args, lds, s);
 }
 
 template <int M>
@@ -178,16 +195,7 @@ hipError_t launch_explore_m(const KArgs &a, int blocks, hipStream_t s)
 {
     const bool lb2 = a.bound_mode != 0 && a.refine == 1;
     const size_t lds = explore_lds_bytes(a.I, lb2, lb2 ? a.jt_lds : 0);
-    if (const hipError_t err =
-            hipFuncSetAttribute(explore_kernel<M>(a), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
-        return err;
-    if (a.bound_mode == 0)
-        hipLaunchKernelGGL((k_explore<M, 0>), dim3(blocks), dim3(64 * PBB_EXPLORE_WAVES), lds, s, a);
-    else if (a.refine == 1)
-        hipLaunchKernelGGL((k_explore<M, 2>), dim3(blocks), dim3(64 * PBB_EXPLORE_WAVES), lds, s, a);
-    else
-        hipLaunchKernelGGL((k_explore<M, 1>), dim3(blocks), dim3(64 * PBB_EXPLORE_WAVES), lds, s, a);
-    return hipGetLastError();
+    return launch_kernel(explore_kernel<M>(a), blocks, 64 * PBB_EXPLORE_WAVES, lds, a, s);
 }
 
 template <int M>
@@ -195,18 +203,7 @@ hipError_t launch_team_m(const KArgs &a, hipStream_t s)
 {
     const bool lb2 = a.bound_mode != 0 && a.refine == 1;
     const size_t lds = team_lds_bytes(a.I, lb2, lb2 ? a.jt_lds : 0, a.E);
-    const void *k = a.bound_mode == 0 ? (const void *)k_team<M, 0>
-                    : a.refine == 1   ? (const void *)k_team<M, 2>
-                                      : (const void *)k_team<M, 1>;
-    if (const hipError_t err = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
-        return err;
-    if (a.bound_mode == 0)
-        hipLaunchKernelGGL((k_team<M, 0>), dim3(1), dim3(64 * a.E), lds, s, a);
-    else if (a.refine == 1)
-        hipLaunchKernelGGL((k_team<M, 2>), dim3(1), dim3(64 * a.E), lds, s, a);
-    else
-        hipLaunchKernelGGL((k_team<M, 1>), dim3(1), dim3(64 * a.E), lds, s, a);
-    return hipGetLastError();
+    return launch_kernel(team_kernel<M>(a), 1, 64 * a.E, lds, a, s);
 }
 
 template <int M>
@@ -219,14 +216,9 @@ hipError_t occupancy_m(const KArgs &a, int *blocks_per_cu)
         return hipSuccess;
     }
     const size_t q = residency_lds_bytes(lds);
-    if (const hipError_t err =
-            hipFuncSetAttribute(explore_kernel<M>(a), hipFuncAttributeMaxDynamicSharedMemorySize, (int)q))
-        return err;
-    if (a.bound_mode == 0)
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, k_explore<M, 0>, 64 * PBB_EXPLORE_WAVES, q);
-    if (a.refine == 1)
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, k_explore<M, 2>, 64 * PBB_EXPLORE_WAVES, q);
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, k_explore<M, 1>, 64 * PBB_EXPLORE_WAVES, q);
+    const void *k = explore_kernel<M>(a);
+    if (const hipError_t err = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)q)) return err;
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, k, 64 * PBB_EXPLORE_WAVES, q);
 }
 
 template <int M>

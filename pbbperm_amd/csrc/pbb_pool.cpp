@@ -226,8 +226,8 @@ extern "C" int pbb_pool_create(const pbb_config *cfg, const pbb_pool_params *prm
     p->margin = prm->steal_margin ? prm->steal_margin : cfg->steal_margin;
     const bool lb2 = cfg->bound_mode != 0 && cfg->refine == 1;
     p->pmax = lb2 ? (cfg->johnson_pairs == 0 ? p->M * (p->M - 1) / 2 : p->M - 1) : 0;
-    p->jt_lds = lb2 ? jtab_lds_bytes(p->nmax, p->pmax) : 0;
-    if (p->jt_lds > 24 * 1024) p->jt_lds = 0;
+    p->jt_lds = lb2 ? jtab_lds_bytes(p->nmax, p->pmax, true) : 0;
+    if (p->jt_lds > JTAB_PACKED_MOST) p->jt_lds = 0;
     p->ig = p->W >= 2 ? prm->ig_iterations : 0;
     p->lds = pool_lds_bytes(p->nmax, p->M, p->pmax, p->jt_lds, p->W) + (p->ig ? pool_ig_bytes(p->M) : 0);
     p->qcap = next_pow2(std::max(64, prm->slots));
@@ -249,21 +249,33 @@ extern "C" int pbb_pool_create(const pbb_config *cfg, const pbb_pool_params *prm
     hipDeviceProp_t prop;
     HTRY(hipGetDeviceProperties(&prop, dev));
     // explorers: resident workgroups x W
-    {
+    const auto resident = [&](int jt, int *gpc) {
         PoolArgs q{};
         q.nmax = p->nmax;
         q.pmax = p->pmax;
-        q.jt_lds = p->jt_lds;
+        q.jt_lds = jt;
         q.W = p->W;
         KArgs a{};
         a.bound_mode = cfg->bound_mode;
         a.refine = cfg->refine;
-        int gpc = 0;
-        HTRY(pool_occupancy(p->M, a, q, &gpc));
-        if (gpc < 1) TRY(fail(PBB_E_CAPACITY, "pool workgroup does not fit a CU (LDS %zu bytes)", p->lds));
-        const int cap = gpc * prop.multiProcessorCount;
-        p->groups = prm->groups ? std::min(prm->groups, cap) : cap;
+        return pool_occupancy(p->M, a, q, gpc);
+    };
+    int gpc = 0;
+    HTRY(resident(p->jt_lds, &gpc));
+    if (gpc < 1) TRY(fail(PBB_E_CAPACITY, "pool workgroup does not fit a CU (LDS %zu bytes)", p->lds));
+    // room for the wide tables of large processing times, where it costs no workgroup
+    const int wide = lb2 ? (p->nmax * p->pmax * 8 + 15) & ~15 : 0;
+    if (wide > p->jt_lds && wide <= 32 * 1024) {
+        int g = 0;
+        const size_t more = p->lds + wide - p->jt_lds;
+        HTRY(resident(wide, &g));
+        if (g >= gpc && more * gpc <= 160 * 1024) {
+            p->jt_lds = wide;
+            p->lds = more;
+        }
     }
+    const int cap = gpc * prop.multiProcessorCount;
+    p->groups = prm->groups ? std::min(prm->groups, cap) : cap;
     p->E = p->groups * p->W;
     p->epi = std::min(p->epi, p->E);
     p->epi_max = next_pow2(std::max(32, p->epi));

@@ -500,7 +500,7 @@ __global__ __launch_bounds__(256, PBB_POOL_MIN_WAVES(M)) void k_pool(KArgs a, Po
         } else {
             const int n = uni(ld_rlx(&S->n)), m = uni(ld_rlx(&S->m)), npairs = uni(ld_rlx(&S->npairs));
             const DevInst I = slot_inst<M>(p, slot, n, npairs, uni(ld_rlx(&S->jpacked)));
-            const Lds lds = lds_setup(I, smem, p.jt_lds, REF == 2);
+            const Lds lds = lds_setup<TAB_ANY>(I, smem, p.jt_lds, REF == 2);
             if (role == ROLE_OWNER) {
                 // a request without an incumbent gets NEH's (ub < 0)
                 if (wave == 0 && uni(ld_rlx(&S->ub)) < 0) {
