@@ -69,14 +69,13 @@ typedef struct pbb_config {
                                interval (0: at once); engine-specific, no
                                reference counterpart */
     int team_nodes;         /* a search from pbb_init_full first runs on one
-                               workgroup of explorers (16 with LB1 only, 8 with
-                               a refinement bound) for up to this many nodes,
-                               then on the whole device (0: whole device at
-                               once).  At PBB_TEAM_NODES_DEFAULT the engine
-                               gives the team its share of them: LB1 half until
-                               the incumbent moves, a refinement bound an
-                               eighth.  Engine-specific, no reference
-                               counterpart */
+                               workgroup of explorers (16, with the Johnson
+                               bound 8) for up to this many nodes, then on the
+                               whole device (0: whole device at once).  At
+                               PBB_TEAM_NODES_DEFAULT the engine gives the team
+                               a share of them (LB1 a quarter, a refinement
+                               bound an eighth) until the incumbent moves.
+                               Engine-specific, no reference counterpart */
     int team_waves;         /* explorers of that workgroup (0: the largest the
                                kernel allows, 16 or 8; larger values are
                                clamped to it); engine-specific, no reference

@@ -669,18 +669,19 @@ static int launch_once(pbb_engine *e, bool team, uint64_t node_budget, uint64_t 
 // team_nodes as the caller set it, unless it is the default: then the engine
 // chooses.  The team pays on trees that end within it; on a larger one it holds
 // the device back, so it gets about the time that a device-wide launch needs to
-// fan out, half a millisecond: half of team_nodes with LB1 (16 explorers,
-// 0.14-0.17 us a node), an eighth with a refinement bound (8 explorers, 0.33 us a
-// node with LB1' at 17 machines, 0.42 and 0.78 us with LB2 at 10 and 20).  All of
-// it against this share: 30x20 LB2 9.0 -> 3.9 ms, 20x20 LB1 3.5 -> 3.0, 30x17 LB1'
-// 10.5 -> 8.3, 20x10 LB2 (3636 nodes, all in the team before) 1.67 -> 1.45; at
-// none, a 2457-node LB1 tree 1.1 against 0.55 ms.  With LB1 the team keeps all of
-// team_nodes once it has found a better schedule: more explorers would search
-// more of what the next one prunes (20x5 from NEH: 1.05 against 0.9 ms).  An engine
-// of no more explorers than the team has nothing to gain from the second launch,
-// and a run for fewer nodes than team_nodes stays with the team, which stops
-// within a few hundred nodes of its budget; thousands of explorers, each of which
-// looks every 64 nodes, overrun it by as many.
+// fan out: a quarter of team_nodes with LB1 (0.15-0.18 us a node), an eighth with a
+// refinement bound (0.42 and 0.78 us with LB2 at 10 and 20 machines).  A quarter / a
+// half / all of it with LB1: 2457 nodes 0.46 / 0.46 / 0.46 ms, 5394 nodes 1.0 / 1.07 /
+// 0.8, 31 k nodes 1.58 / 1.8 / 2.35; an eighth 1735 nodes 0.67 against 0.47.  An
+// eighth / all of it with LB2: 20x10 (3636 nodes) 1.13 / 1.34, 30x20 (14 k nodes) 2.5 /
+// 7.6; LB1' 20x10 (8 k nodes) 1.1 / 1.2, 30x17 (45 k) 1.47 / 2.4.  Once the team has
+// found a better schedule it keeps all of team_nodes: more explorers would search
+// more of what the next one prunes (20x5 from NEH, the share / all: LB1 1.08 / 0.8,
+// LB1' 1.3 / 0.87, LB2 1.9 / 1.1; 30x5 with LB2 253 k nodes in 2.8 ms against 5.7 k in
+// 2.05).  An engine of no more explorers than the team has nothing to gain from the
+// second launch, and a run for fewer nodes than team_nodes stays with the team,
+// which stops within a few hundred nodes of its budget; thousands of explorers, each
+// of which looks every 64 nodes, overrun it by as many.
 struct TeamBudget {
     uint64_t quiet, moved;
 };
@@ -689,8 +690,7 @@ static TeamBudget team_budget(const pbb_engine *e, uint64_t node_budget)
     const uint64_t most = (uint64_t)e->cfg.team_nodes;
     if (node_budget && node_budget <= most) return {node_budget, node_budget};
     if (e->cfg.team_nodes != PBB_TEAM_NODES_DEFAULT || e->E <= form_of(e).team) return {most, most};
-    if (e->cfg.bound_mode == 0) return {most / 2, most};
-    return {most / 8, most / 8};
+    return {most / (e->cfg.bound_mode == 0 ? 4 : 8), most};
 }
 
 // A search started by pbb_init_full runs first on the team (one workgroup)

@@ -250,10 +250,9 @@ inline int explore_jtab_bytes(const DevInst &I)
     const int b = jtab_lds_bytes(I.n, I.npairs, true);
     return b <= JTAB_PACKED_MOST && 3 * residency_lds_bytes(explore_lds_bytes(I, true, b)) <= 160 * 1024 ? b : 0;
 }
-// The team launch (one workgroup) holds at most 16 explorers with LB1 only
-// (4 per SIMD, the register budget of the LB1 explorer) and 8 with a
-// refinement bound (whose explorer needs more than 128 registers).
-__device__ __host__ constexpr int team_waves_max(int ref) { return ref == 0 ? 16 : 8; }
+// The team launch (one workgroup) holds at most 16 explorers with LB1 and LB1' (4 per
+// SIMD; their explorers take up to 102 registers of 128) and 8 with LB2 (up to 187).
+__device__ __host__ constexpr int team_waves_max(int ref) { return ref == 2 ? 8 : 16; }
 inline size_t team_lds_bytes(const DevInst &I, bool lb2, int jt, int waves)
 {
     return lds_table_bytes(I.m, jt) + (size_t)waves * lds_wave_bytes(I.n, I.m, lb2);
