@@ -74,7 +74,8 @@ typedef struct pbb_config {
                                whole device (0: whole device at once).  At
                                PBB_TEAM_NODES_DEFAULT the engine gives the team
                                a share of them (LB1 a quarter, a refinement
-                               bound an eighth) until the incumbent moves.
+                               bound an eighth), and all of them (the Johnson
+                               bound a quarter) once the incumbent has moved.
                                Engine-specific, no reference counterpart */
     int team_waves;         /* explorers of that workgroup (0: the largest the
                                kernel allows, 16 or 8; larger values are

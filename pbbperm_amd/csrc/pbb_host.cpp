@@ -675,10 +675,11 @@ static int launch_once(pbb_engine *e, bool team, uint64_t node_budget, uint64_t 
 // 0.8, 31 k nodes 1.58 / 1.8 / 2.35; an eighth 1735 nodes 0.67 against 0.47.  An
 // eighth / all of it with LB2: 20x10 (3636 nodes) 1.13 / 1.34, 30x20 (14 k nodes) 2.5 /
 // 7.6; LB1' 20x10 (8 k nodes) 1.1 / 1.2, 30x17 (45 k) 1.47 / 2.4.  Once the team has
-// found a better schedule it keeps all of team_nodes: more explorers would search
-// more of what the next one prunes (20x5 from NEH, the share / all: LB1 1.08 / 0.8,
-// LB1' 1.3 / 0.87, LB2 1.9 / 1.1; 30x5 with LB2 253 k nodes in 2.8 ms against 5.7 k in
-// 2.05).  An engine of no more explorers than the team has nothing to gain from the
+// found a better schedule it keeps all of team_nodes, a quarter with LB2: more
+// explorers would search more of what the next one prunes (20x5 from NEH, the share /
+// this: LB1 1.08 / 0.8, LB1' 1.3 / 0.87, LB2 1.9 / 1.1; with LB2 half of it brings no
+// more, and 256 instances of the batch one after the other take 0.376 s at the share,
+// 0.386 at a quarter, 0.408 at half, 0.458 at all).  An engine of no more explorers than the team has nothing to gain from the
 // second launch, and a run for fewer nodes than team_nodes stays with the team,
 // which stops within a few hundred nodes of its budget; thousands of explorers, each
 // of which looks every 64 nodes, overrun it by as many.
@@ -690,6 +691,7 @@ static TeamBudget team_budget(const pbb_engine *e, uint64_t node_budget)
     const uint64_t most = (uint64_t)e->cfg.team_nodes;
     if (node_budget && node_budget <= most) return {node_budget, node_budget};
     if (e->cfg.team_nodes != PBB_TEAM_NODES_DEFAULT || e->E <= form_of(e).team) return {most, most};
+    if (with_lb2(e)) return {most / 8, most / 4};
     return {most / (e->cfg.bound_mode == 0 ? 4 : 8), most};
 }
 
