@@ -325,7 +325,6 @@ struct Explorer {
     int pollw;                        // next idle word to poll
     int seen;                         // pool: the slot's member word as of the last poll
     unsigned nchk;                    // periodic checks so far (host-word phase)
-    unsigned since;                   // nodes decomposed in this launch's own interval (ramp)
     bool end_dirty;                   // end moved since pos was last compared with it
     int hist;                         // lane d: nodes decomposed at depth d since the flush
     int jhist;                        // lane d: refinement bounds at depth d (REF != 0)
@@ -344,7 +343,6 @@ struct Explorer {
         for (int c = 0; c < PCH; c++) places[c] = 0u;
         if constexpr (REF == 2) pair_lanes<PCH>(r.pair_ab, r.npairs, r.m, r.pairs_mode, pinfo);
         dec = leaves = sb = jb = 0;
-        since = 0;
         mtag = 0;
         self = eid;
         pollw = seen = 0;
@@ -941,7 +939,6 @@ struct Explorer {
                 continue;
             }
             dec++;
-            since += since < a.ramp ? 1u : 0u;  // saturates at the ramp
             go_down(c, true);
             hist += (lane == L);
             if (L == n - 1) {
@@ -975,7 +972,6 @@ struct Explorer {
         endv = lane < n ? (int)a.end[(size_t)e * 64 + lane] : 0;
         dirv = lane < n ? (int)a.dir[(size_t)e * 64 + lane] : 0;
         end_dirty = true;
-        since = a.ramp;  // a resumed interval is shared at once
         __builtin_amdgcn_wave_barrier();
         rebuild_stacks();
     }
@@ -1058,7 +1054,6 @@ struct Explorer {
             remv -= pmach(j);
         }
         end_dirty = true;
-        since = a.ramp;  // a donated interval is shared at once
         __builtin_amdgcn_wave_barrier();
     }
 
@@ -1086,7 +1081,6 @@ struct Explorer {
         endv = lane < n ? (int)a.end[(size_t)e * 64 + lane] : 0;
         dirv = lane == 0 ? ir.root_dir[0] : 0;
         end_dirty = true;
-        since = 0;
         reset_stacks();
         if (!before_end()) return false;
         unfold();
@@ -1103,7 +1097,6 @@ struct Explorer {
         endv = lane < n ? n - 1 - lane : 0;
         dirv = lane == 0 ? dirv : 0;
         end_dirty = true;
-        since = 0;
         reset_stacks();
         if (!before_end()) return false;
         unfold();

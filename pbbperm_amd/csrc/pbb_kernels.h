@@ -167,7 +167,7 @@ struct KArgs {
     // configuration
     int bound_mode, branching, refine, pairs_mode, find_all, single_node, initial_ub;
     int steal_margin;
-    unsigned ramp;      // nodes an explorer decomposes in a fresh interval before it donates
+    unsigned ramp;      // interior nodes an explorer decomposes in a fresh interval before it donates
     int jt_lds;         // bytes of LDS for the staged Johnson table (0: read from global memory)
 };
 

@@ -43,9 +43,12 @@ __device__ __forceinline__ void explore_loop(const KArgs &a, const Lds &lds, int
     X.join(e);
     // what the host or the previous launch left is visible at launch start
     int st = uni(ld_rlx<SC>(a.state + e));
+    unsigned iter = 0;
+    unsigned next = 0;  // node of the next poll
     if (st == ST_UNFOLD) {
         if (X.start_unfold()) {
             st = ST_ACTIVE;
+            next = a.ramp;  // none while the ramp holds this explorer's work back
         } else {
             if (X.go_idle() && X.lane == 0) st_rel<SC>(&a.ctl->done, 1);
             st = ST_IDLE;
@@ -61,8 +64,6 @@ __device__ __forceinline__ void explore_loop(const KArgs &a, const Lds &lds, int
         X.register_idle();
     }
 
-    unsigned iter = 0;
-    unsigned next = 0;  // node of the next poll
     while (true) {
         if (st == ST_IDLE) {
             // wait for a donation, global termination or a stop; the host
@@ -81,6 +82,7 @@ __device__ __forceinline__ void explore_loop(const KArgs &a, const Lds &lds, int
                     // a donated interval is explored under the current incumbent,
                     // not the one this explorer saw before it went idle
                     X.take_best(bw);
+                    if (a.ramp) next = iter;  // a donated interval is shared at once
                     break;
                 }
                 if (uni(done) || uni(stop) || (X.t_end && wall_clock64() >= X.t_end)) {
@@ -96,13 +98,12 @@ __device__ __forceinline__ void explore_loop(const KArgs &a, const Lds &lds, int
             }
         }
         // idle-mask poll issued before the node's work so its latency is
-        // hidden; none while the ramp holds this explorer's work back.  In
-        // the workgroup team (at most 16 explorers, workgroup-scope atomics)
+        // hidden.  In the workgroup team (at most 16 explorers, workgroup-scope atomics)
         // and with LB2 a donor that saw explorers waiting polls again at the
         // next node, otherwise one that gave from a large interval
         // (PBB_POLL_EVERY, SHARE_DEEP).
         constexpr bool eager = SC == __HIP_MEMORY_SCOPE_WORKGROUP || REF == 2;
-        const bool poll = X.since >= a.ramp && (int)(iter - next) >= 0;
+        const bool poll = (int)(iter - next) >= 0;
         unsigned long long idle = 0ull;
         if (poll) idle = X.peek_idle();
         const bool refresh = (iter & (PBB_BEST_EVERY - 1)) == 0u;
@@ -119,8 +120,9 @@ __device__ __forceinline__ void explore_loop(const KArgs &a, const Lds &lds, int
             X.flush_counters();
             return;
         }
-        // a count of nodes rather than a flag: 2078 against 2058 M nodes/s at 50x20
-        // (2104 with the flag left out)
+        // one count of nodes for the interval, the eager polls and the ramp: 2106 M
+        // nodes/s at 50x20 (2076 with a counter of the ramp's nodes beside it, 2058
+        // with that and a flag for the eager polls)
         if (poll) next = iter + (X.try_donate(idle) >= (eager ? 1 : 2) ? 0u : PBB_POLL_EVERY - 1u);
     }
 }
