@@ -8,9 +8,10 @@
 //   1. chains: one lane per schedule and side, its completion times in
 //      registers, so that a job costs 3 instructions per machine for 64 chains
 //      (a wavefront per schedule, lane = machine, pays a prefix scan of 25
-//      dependent instructions per job for one).  Lengths run over 0..n and a
-//      wavefront runs as long as its longest chain, so the tile's 2T chains are
-//      first sorted by length (a counting sort of 64 bins);
+//      dependent instructions per job for one; small batches take that, B_SMALL).
+//      Lengths run over 0..n and a wavefront runs as long as its longest chain,
+//      so the tile's 2T chains are first sorted by length (a counting sort of 64
+//      bins);
 //   2. operands: per schedule and machine the front and back times with the
 //      remaining work folded in, in LDS;
 //   3. the bound: children one lane per child, both directions, over the tile's
@@ -32,6 +33,16 @@ enum { B_CHILDREN = 0, B_LB1 = 1, B_LB2 = 2, B_MAKESPAN = 3 };
 // that read one position of different schedules on distinct banks
 #define BJ_STRIDE 68
 #define B_THREADS 256
+// Batches of up to B_SMALL_COUNT schedules go in tiles of B_SMALL, a schedule per
+// wavefront: what bounds them is the time of one chain, and a lane that takes
+// every machine of every job is slower for one schedule than a wavefront whose lanes
+// are the machines.  A kernel of its own: beside the lane-wise chains it costs LB2 a
+// third (50x10, 100 k schedules 102 -> 134 us).  One call, tiles of 16 / this: 256
+// schedules at 50x20, children 41.8 / 29.0 us, LB2 53.7 / 36.3; at 20x10 28.7 / 25.0
+// and 28.3 / 24.6; 4096 at 50x20, children 42.9 / 32.6, LB2 56.0 / 52.1, 8192 43.3 /
+// 40.5 and 61.9 / 75.5.
+#define B_SMALL (B_THREADS / 64)
+#define B_SMALL_COUNT 4096
 // most schedules per tile
 __host__ __device__ constexpr int b_tile(int which) { return which == B_LB2 ? 32 : 128; }
 
@@ -74,10 +85,11 @@ __device__ __host__ inline size_t bound_table_bytes(const DevInst &I, bool jtab)
     return b;
 }
 
-template <int M, int WHICH>
-__global__ __launch_bounds__(B_THREADS) void k_bounds(DevInst I, int count, int T, const int *perms, const int *l1s,
+template <int M, int WHICH, bool SMALL>
+__global__ __launch_bounds__(B_THREADS) void k_bounds(DevInst I, int count, int tile, const int *perms, const int *l1s,
                                                       const int *l2s, int arg, int *o1, int *o2)
 {
+    const int T = SMALL ? B_SMALL : tile;
     extern __shared__ __align__(16) char smem[];
     const int tid = threadIdx.x, lane = lane_id(), wave = uni(tid >> 6);
     const int n = I.n;
@@ -101,7 +113,7 @@ __global__ __launch_bounds__(B_THREADS) void k_bounds(DevInst I, int count, int 
     // per wavefront and register: a load per row and a wait for each took most
     // of the time (50x20: 700 us per million schedules, 473 this way).
     // Ids outside 0..n-1 become 63, which is none of them (n <= 63).
-    constexpr int ROWS = b_tile(WHICH) / (B_THREADS / 64);
+    constexpr int ROWS = (SMALL ? B_SMALL : b_tile(WHICH)) / (B_THREADS / 64);
     int rows[ROWS], pl1 = 0, pl2 = 0;
     const auto prefetch = [&](long long s0) {
         const int ns = (int)max(0ll, min((long long)T, count - s0));
@@ -146,7 +158,7 @@ __global__ __launch_bounds__(B_THREADS) void k_bounds(DevInst I, int count, int 
     int pinfo[PCH];
     if constexpr (WHICH == B_LB2) pair_lanes<PCH>(I.pair_ab, I.npairs, I.m, arg, pinfo);
     // the chains of a tile of up to 32 schedules are one wavefront's: no order
-    const bool sorted = WHICH != B_MAKESPAN && T > 32;
+    const bool sorted = !SMALL && WHICH != B_MAKESPAN && T > 32;
 
     for (long long s0 = (long long)blockIdx.x * T; s0 < count; s0 += (long long)gridDim.x * T) {
         const int ns = (int)min((long long)T, count - s0);
@@ -223,42 +235,67 @@ __global__ __launch_bounds__(B_THREADS) void k_bounds(DevInst I, int count, int 
         __syncthreads();
         // chains: front over machines 0..M-1 from min_arr, back over machines
         // M-1..0 from min_dep (as starting from zero, bound_fsp_weak.cpp:61-110)
-        for (int c = tid; c < 2 * ns; c += B_THREADS) {
-            const int s = S.order[c] >> 1, side = S.order[c] & 1;
-            const int len = side ? n - S.l2[s] : (S.l1[s] < -1 ? 0 : S.l1[s] + 1);
-            const uint8_t *js = S.jobs + s * BJ_STRIDE + (side ? n - 1 : 0);
-            const int *tab = side ? pmR : pm;
-            const int step = side ? -1 : 1;
-            int f[M], w[M], v[M];
-#pragma unroll
-            for (int q = 0; q < M; q++) {
-                f[q] = side ? minD[M - 1 - q] : minA[q];
-                w[q] = 0;
+        if constexpr (SMALL) {
+            // a wavefront per schedule, half of it per side, lane = machine: a job
+            // costs the wavefront a scan, but the chain is short
+            if (wave < ns) {
+                const int side = lane >> 5, q = lane & 31, qq = min(q, M - 1);
+                const int lf = uni(S.l1[wave] < -1 ? 0 : S.l1[wave] + 1), lb = uni(n - S.l2[wave]);
+                const int len = side ? lb : lf, step = side ? -1 : 1;
+                const uint8_t *js = S.jobs + wave * BJ_STRIDE + (side ? n - 1 : 0);
+                const int *tab = (side ? pmR : pm) + qq * PM_STRIDE;
+                int f = side ? minD[M - 1 - qq] : minA[qq], w = 0;
+                int v = tab[js[0]];
+                const int steps = max(lf, lb);
+                for (int i = 0; i < steps; i++) {
+                    js += step;
+                    const int next = tab[js[0] & 63];  // past the chain: unused
+                    const int p = i < len && q < M ? v : 0;
+                    const int c = chain_scan(q < M ? f : 0, p);
+                    f = i < len ? c : f;
+                    w += p;
+                    v = next;
+                }
+                if (q < M) S.U[(size_t)wave * US + side * M + q] = make_int2(f, w);
             }
-            // the next job's times are read before this one's are used (one
-            // past the chain: any byte, kept inside the table and unused)
-            int next = js[step] & 63;
-            {
-                const int *p = tab + js[0];
-#pragma unroll
-                for (int q = 0; q < M; q++) v[q] = p[q * PM_STRIDE];
-            }
-            for (int i = 0; i < len; i++) {
-                const int *p = tab + next;
-                js += step;
-                next = js[step] & 63;
-                int t = 0;
+        } else {
+            for (int c = tid; c < 2 * ns; c += B_THREADS) {
+                const int s = S.order[c] >> 1, side = S.order[c] & 1;
+                const int len = side ? n - S.l2[s] : (S.l1[s] < -1 ? 0 : S.l1[s] + 1);
+                const uint8_t *js = S.jobs + s * BJ_STRIDE + (side ? n - 1 : 0);
+                const int *tab = side ? pmR : pm;
+                const int step = side ? -1 : 1;
+                int f[M], w[M], v[M];
 #pragma unroll
                 for (int q = 0; q < M; q++) {
-                    t = max(t, f[q]) + v[q];  // times are not negative: t = 0 before the first machine
-                    f[q] = t;
-                    w[q] += v[q];
-                    v[q] = p[q * PM_STRIDE];
+                    f[q] = side ? minD[M - 1 - q] : minA[q];
+                    w[q] = 0;
                 }
-            }
-            int2 *u = S.U + (size_t)s * US + side * M;
+                // the next job's times are read before this one's are used (one
+                // past the chain: any byte, kept inside the table and unused)
+                int next = js[step] & 63;
+                {
+                    const int *p = tab + js[0];
 #pragma unroll
-            for (int q = 0; q < M; q++) u[q] = make_int2(f[q], w[q]);
+                    for (int q = 0; q < M; q++) v[q] = p[q * PM_STRIDE];
+                }
+                for (int i = 0; i < len; i++) {
+                    const int *p = tab + next;
+                    js += step;
+                    next = js[step] & 63;
+                    int t = 0;
+#pragma unroll
+                    for (int q = 0; q < M; q++) {
+                        t = max(t, f[q]) + v[q];  // times are not negative: t = 0 before the first machine
+                        f[q] = t;
+                        w[q] += v[q];
+                        v[q] = p[q * PM_STRIDE];
+                    }
+                }
+                int2 *u = S.U + (size_t)s * US + side * M;
+#pragma unroll
+                for (int q = 0; q < M; q++) u[q] = make_int2(f[q], w[q]);
+            }
         }
         __syncthreads();
         // (f, work in front), (b, work behind) -> (f, r + b), (b, f + r)
@@ -369,27 +406,29 @@ __global__ __launch_bounds__(B_THREADS) void k_bounds(DevInst I, int count, int 
 }
 
 // Tile size: up to 128 schedules, as many as leave room for three workgroups
-// per CU beside the tables (two with a Johnson table); a small batch is spread
-// over the CUs in smaller tiles, 16 schedules at least.
+// per CU beside the tables (two with a Johnson table); a smaller batch is spread
+// over the CUs in smaller tiles, 16 schedules at least, a small one in tiles of
+// B_SMALL.
 template <int M, int WHICH>
 static hipError_t launch(const DevInst &I, int count, const int *perms, const int *l1, const int *l2, int arg, int *o1,
                          int *o2, hipStream_t s)
 {
     const size_t tab = bound_table_bytes<M>(I, WHICH == B_LB2 && I.jpacked);
     const size_t room = 160 * 1024 / (WHICH == B_LB2 ? 2 : 3) - 2048;
-    int T = b_tile(WHICH);
+    const auto tiles = [&](int T) { return (int)(((long long)count + T - 1) / T); };
+    const bool small = count <= B_SMALL_COUNT;
+    int T = small ? B_SMALL : b_tile(WHICH);
     while (T > 16 && tab + bound_tile_bytes<M>(T) > room) T -= 16;
-    while (T > 16 && (count + T - 1) / T < 512) T -= 16;
+    while (T > 16 && tiles(T) < 512) T -= 16;
     const size_t lds = tab + bound_tile_bytes<M>(T);
+    const auto kernel = small ? k_bounds<M, WHICH, true> : k_bounds<M, WHICH, false>;
     if (lds > 64 * 1024)
-        if (const hipError_t err = hipFuncSetAttribute((const void *)k_bounds<M, WHICH>,
+        if (const hipError_t err = hipFuncSetAttribute((const void *)kernel,
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
             return err;
-    const int tiles = (count + T - 1) / T;
     const int resident = 256 * (int)(160 * 1024 / lds < 8 ? 160 * 1024 / lds : 8);
-    const int grid = tiles < resident ? tiles : resident;
-    hipLaunchKernelGGL((k_bounds<M, WHICH>), dim3(grid), dim3(B_THREADS), lds, s, I, count, T, perms, l1, l2, arg, o1,
-                       o2);
+    const int grid = tiles(T) < resident ? tiles(T) : resident;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(B_THREADS), lds, s, I, count, T, perms, l1, l2, arg, o1, o2);
     return hipGetLastError();
 }
 

@@ -75,6 +75,40 @@ PBB_DPP_REDUCE(wave_min, op_min, 0x7fffffff)
 PBB_DPP_REDUCE(wave_max, op_max, (int)0x80000000)
 #undef PBB_DPP_REDUCE
 
+// ------------------------------------------------------ lane scans (DPP)
+// Inclusive prefix scans over lanes 0..31, and over 32..63 by themselves (row_shr
+// 1,2,4,8 inside each 16-lane row, then row_bcast:15 into rows 1 and 3).  Lanes
+// only combine with lanes to their left, so values in lanes >= the vector length
+// are never read.
+__device__ __forceinline__ int scan_add32(int x)
+{
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);
+    return x;
+}
+__device__ __forceinline__ int scan_max32(int x)
+{
+    const int lo = (int)0x80000000;
+    x = max(x, __builtin_amdgcn_update_dpp(lo, x, 0x111, 0xF, 0xF, false));
+    x = max(x, __builtin_amdgcn_update_dpp(lo, x, 0x112, 0xF, 0xF, false));
+    x = max(x, __builtin_amdgcn_update_dpp(lo, x, 0x114, 0xF, 0xF, false));
+    x = max(x, __builtin_amdgcn_update_dpp(lo, x, 0x118, 0xF, 0xF, false));
+    x = max(x, __builtin_amdgcn_update_dpp(lo, x, 0x142, 0xA, 0xF, false));
+    return x;
+}
+
+// Max-plus chain of one job over the machines, lane q = machine q:
+// c_q = max(base_q, c_{q-1}) + p_q  ==  P_q + max_{i<=q}(base_i - P_{i-1})
+// with P the prefix sum of p (the recurrence of bound_fsp_weak.cpp:76-82).
+__device__ __forceinline__ int chain_scan(int base, int p)
+{
+    const int P = scan_add32(p);
+    return P + scan_max32(base - (P - p));
+}
+
 // lanes i and 32+i both receive x[i] (gfx950 v_permlane32_swap)
 __device__ __forceinline__ int bcast_low_half(int x)
 {

@@ -85,39 +85,6 @@ __device__ __forceinline__ void w_min64(unsigned long long *p, unsigned long lon
     if (lane_id() == 0) __hip_atomic_fetch_min(p, v, __ATOMIC_ACQ_REL, S);
 }
 
-// ------------------------------------------------------ lane scans (DPP)
-// Inclusive prefix scans over lanes 0..31 (row_shr 1,2,4,8 inside each
-// 16-lane row, then row_bcast:15 into row 1).  Lanes only combine with lanes
-// to their left, so values in lanes >= the vector length are never read.
-__device__ __forceinline__ int scan_add32(int x)
-{
-    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);
-    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);
-    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);
-    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);
-    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);
-    return x;
-}
-__device__ __forceinline__ int scan_max32(int x)
-{
-    const int lo = (int)0x80000000;
-    x = max(x, __builtin_amdgcn_update_dpp(lo, x, 0x111, 0xF, 0xF, false));
-    x = max(x, __builtin_amdgcn_update_dpp(lo, x, 0x112, 0xF, 0xF, false));
-    x = max(x, __builtin_amdgcn_update_dpp(lo, x, 0x114, 0xF, 0xF, false));
-    x = max(x, __builtin_amdgcn_update_dpp(lo, x, 0x118, 0xF, 0xF, false));
-    x = max(x, __builtin_amdgcn_update_dpp(lo, x, 0x142, 0xA, 0xF, false));
-    return x;
-}
-
-// Max-plus chain of one job over the machines, lane q = machine q:
-// c_q = max(base_q, c_{q-1}) + p_q  ==  P_q + max_{i<=q}(base_i - P_{i-1})
-// with P the prefix sum of p (the recurrence of bound_fsp_weak.cpp:76-82).
-__device__ __forceinline__ int chain_scan(int base, int p)
-{
-    const int P = scan_add32(p);
-    return P + scan_max32(base - (P - p));
-}
-
 // ------------------------------------------------------------ LDS layout
 struct Lds {
     int *pm;        // [m][PM_STRIDE] machine-major processing times
