@@ -126,9 +126,8 @@ __device__ __forceinline__ int flag_abs(int j) { return j >= 0 ? j : -j - 1; }  
 // Instance tables as seen by the device.
 struct DevInst {
     int n, m;
-    int mp;               // padded stride of ptmT (multiple of 4)
+    int mp;               // m, padded to a multiple of 4
     const int *ptm;       // [m][n] machine-major
-    const int *ptmT;      // [n][mp] job-major
     const int *min_arr;   // [m] bound_fsp_weak.cpp:270-283
     const int *min_dep;   // [m] bound_fsp_weak.cpp:253-267
     int npairs;

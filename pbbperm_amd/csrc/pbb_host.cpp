@@ -32,9 +32,6 @@ void pbb::build_tables(const int32_t *ptm, int n, int m, HostTables &T)
     T.m = m;
     T.mp = (m + 3) & ~3;
     T.ptm.assign(ptm, ptm + (size_t)n * m);
-    T.ptmT.assign((size_t)n * T.mp, 0);
-    for (int j = 0; j < n; j++)
-        for (int k = 0; k < m; k++) T.ptmT[(size_t)j * T.mp + k] = ptm[k * n + j];
     // bound_fsp_weak::fillMinTimeArrDep (bound_fsp_weak.cpp:248-286)
     T.min_arr.assign(m, INT_MAX);
     T.min_dep.assign(m, INT_MAX);
@@ -107,13 +104,12 @@ struct DevTables {
 
 static size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// Offsets of ptm, ptmT, min_arr, min_dep, pair_ab and jtab (in either form).
+// Offsets of ptm, min_arr, min_dep, pair_ab and jtab (in either form).
 struct TableLayout {
-    size_t ptmT, min_arr, min_dep, pair_ab, jtab, bytes;
+    size_t min_arr, min_dep, pair_ab, jtab, bytes;
     explicit TableLayout(const HostTables &T)
     {
-        ptmT = al256(T.ptm.size() * 4);
-        min_arr = ptmT + al256(T.ptmT.size() * 4);
+        min_arr = al256(T.ptm.size() * 4);
         min_dep = min_arr + al256((size_t)T.m * 4);
         pair_ab = min_dep + al256((size_t)T.m * 4);
         jtab = pair_ab + al256((size_t)T.npairs * 4);
@@ -127,7 +123,6 @@ static std::vector<char> pack_tables(const HostTables &T)
     const TableLayout L(T);
     std::vector<char> v(L.jtab + T.jdev.size() * 4);
     memcpy(v.data(), T.ptm.data(), T.ptm.size() * 4);
-    memcpy(v.data() + L.ptmT, T.ptmT.data(), T.ptmT.size() * 4);
     memcpy(v.data() + L.min_arr, T.min_arr.data(), (size_t)T.m * 4);
     memcpy(v.data() + L.min_dep, T.min_dep.data(), (size_t)T.m * 4);
     if (T.npairs) {
@@ -147,7 +142,6 @@ static int upload_tables(const HostTables &T, DevTables &D)
     D.I.m = T.m;
     D.I.mp = T.mp;
     D.I.ptm = (const int *)D.mem;
-    D.I.ptmT = (const int *)(D.mem + L.ptmT);
     D.I.min_arr = (const int *)(D.mem + L.min_arr);
     D.I.min_dep = (const int *)(D.mem + L.min_dep);
     D.I.npairs = T.npairs;

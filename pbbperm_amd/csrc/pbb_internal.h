@@ -18,7 +18,7 @@ namespace pbb {
 // Johnson order {job, p_a, p_b, lag}.
 struct HostTables {
     int n, m, mp, npairs;
-    std::vector<int> ptm, ptmT, min_arr, min_dep, pair_ab;
+    std::vector<int> ptm, min_arr, min_dep, pair_ab;
     std::vector<int4> jtab;
     // the device's form of it, job-major (pbb_device.h): packed words or pairs of words
     bool jpacked;

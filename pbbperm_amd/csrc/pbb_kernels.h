@@ -47,11 +47,8 @@ __device__ __forceinline__ unsigned mail_tag(unsigned w) { return w >> 26; }
 // the interval at once by the interval-end test, as on the donor's own row.
 __device__ __forceinline__ int mail_path_cell(int i, int p, int j) { return i == p ? j : (i > p ? 0 : -1); }
 
-#define PBB_SPIN_LIMIT (1 << 24)
-
 // A busy explorer of a device-wide launch reads a word of the idle mask every
-// PBB_POLL_EVERY decomposed nodes (power of two), whether or not explorers
-// wait in it; with Johnson LB2, whose node takes several times an LB1 node's
+// PBB_POLL_EVERY decomposed nodes, whether or not explorers wait in it; with Johnson LB2, whose node takes several times an LB1 node's
 // time, it reads the next word at the next node while it sees explorers
 // waiting.  A poll costs a busy device, a long interval between them a thin
 // tree, whose fan-out takes that long per doubling.  Every 16 / 8 / 4 / 1 nodes:
@@ -139,7 +136,7 @@ struct KArgs {
     DevInst I;
     int E;              // explorers (wavefronts)
     int rows;           // rows per explorer in mat (the largest n served)
-    // explorer state in HBM (row stride 64 bytes)
+    // explorer state in HBM between launches (row stride 64 bytes; the pool keeps none)
     int8_t *mat;        // [E][n][64]
     int8_t *pos;        // [E][64]
     int8_t *end;        // [E][64]
@@ -308,7 +305,7 @@ struct PoolSlot {                 // device header of one instance slot
 
 // byte offsets inside one slot's arena (all 256-byte aligned)
 struct PoolLayout {
-    size_t hdr, ptm, ptmT, minA, minD, pair, key, jtab, idle, member, stride;
+    size_t hdr, ptm, minA, minD, pair, key, jtab, idle, member, stride;
 };
 __device__ __host__ inline size_t pool_al(size_t x) { return (x + 255) & ~(size_t)255; }
 __device__ __host__ inline PoolLayout pool_layout(int nmax, int M, int pmax, int members)
@@ -318,7 +315,6 @@ __device__ __host__ inline PoolLayout pool_layout(int nmax, int M, int pmax, int
     size_t o = 0;
     L.hdr = o;      o += pool_al(sizeof(PoolSlot));
     L.ptm = o;      o += pool_al((size_t)M * nmax * 4);
-    L.ptmT = o;     o += pool_al((size_t)nmax * mp * 4);
     L.minA = o;     o += pool_al((size_t)mp * 4);
     L.minD = o;     o += pool_al((size_t)mp * 4);
     L.pair = o;     o += pool_al((size_t)(pmax > 0 ? pmax : 1) * 4);

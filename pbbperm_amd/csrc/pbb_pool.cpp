@@ -52,8 +52,7 @@ struct pbb_pool {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // device
     char *arena = nullptr;
-    int8_t *mat = nullptr, *pos = nullptr, *end = nullptr, *dir = nullptr;
-    int *line = nullptr, *state = nullptr, *best_perm = nullptr;
+    int *best_perm = nullptr;
     unsigned long long *mbox = nullptr;
     Ctl *run = nullptr;
     unsigned *q_head = nullptr;
@@ -94,12 +93,6 @@ static KArgs pool_kargs(const pbb_pool *p, double budget_s)
     a.I.mp = (p->M + 3) & ~3;
     a.E = p->E;
     a.rows = p->nmax;
-    a.mat = p->mat;
-    a.pos = p->pos;
-    a.end = p->end;
-    a.dir = p->dir;
-    a.line = p->line;
-    a.state = p->state;
     a.mbox = p->mbox;
     a.best_perm = p->best_perm;
     a.ctl = p->run;
@@ -168,12 +161,6 @@ extern "C" int pbb_pool_destroy(pbb_pool *p)
     }
     if (p->gexec) hipGraphExecDestroy(p->gexec);
     hipFree(p->arena);
-    hipFree(p->mat);
-    hipFree(p->pos);
-    hipFree(p->end);
-    hipFree(p->dir);
-    hipFree(p->line);
-    hipFree(p->state);
     hipFree(p->mbox);
     hipFree(p->best_perm);
     hipFree(p->run);
@@ -283,12 +270,6 @@ extern "C" int pbb_pool_create(const pbb_config *cfg, const pbb_pool_params *prm
     const size_t S = (size_t)prm->slots, E = (size_t)p->E;
     const size_t arena_bytes = S * (p->lay.stride + sizeof(int));
     HTRY(hipMalloc(&p->arena, arena_bytes));
-    HTRY(hipMalloc(&p->mat, E * p->nmax * 64));
-    HTRY(hipMalloc(&p->pos, E * 64));
-    HTRY(hipMalloc(&p->end, E * 64));
-    HTRY(hipMalloc(&p->dir, E * 64));
-    HTRY(hipMalloc(&p->line, E * 4));
-    HTRY(hipMalloc(&p->state, E * 4));
     HTRY(hipMalloc(&p->mbox, E * 64 * 8));
     HTRY(hipMalloc(&p->best_perm, E * 64 * 4));
     HTRY(hipMalloc(&p->run, sizeof(Ctl)));
@@ -297,7 +278,6 @@ extern "C" int pbb_pool_create(const pbb_config *cfg, const pbb_pool_params *prm
     HTRY(hipMalloc(&p->res_d, S * sizeof(PoolRes)));
     HTRY(hipMalloc(&p->q_d, queue_bytes(p->qcap)));
     HTRY(hipMemset(p->arena, 0, arena_bytes));
-    HTRY(hipMemset(p->state, 0, E * 4));
     HTRY(hipMemset(p->mbox, 0, E * 64 * 8));
     HTRY(hipMemset(p->run, 0, sizeof(Ctl)));
     HTRY(hipHostMalloc((void **)&p->req_h, S * sizeof(PoolReq), hipHostMallocDefault));

@@ -68,7 +68,6 @@ __device__ __forceinline__ DevInst slot_inst(const PoolArgs &p, int s, int n, in
     I.m = M;
     I.mp = (M + 3) & ~3;
     I.ptm = (const int *)(b + p.lay.ptm);
-    I.ptmT = (const int *)(b + p.lay.ptmT);
     I.min_arr = (const int *)(b + p.lay.minA);
     I.min_dep = (const int *)(b + p.lay.minD);
     I.npairs = npairs;
@@ -112,7 +111,6 @@ static __device__ __forceinline__ bool pool_admit(const PoolArgs &p, int s, bool
     const bool ok = n >= 3 && n <= p.nmax && m >= 2 && m <= M;
     const int mp = (M + 3) & ~3;
     int *ptm = (int *)(b + p.lay.ptm);
-    int *ptmT = (int *)(b + p.lay.ptmT);
     int *minA = (int *)(b + p.lay.minA);
     int *minD = (int *)(b + p.lay.minD);
     int *pair = (int *)(b + p.lay.pair);
@@ -131,10 +129,6 @@ static __device__ __forceinline__ bool pool_admit(const PoolArgs &p, int s, bool
     __threadfence_block();
     const bool jpacked = __syncthreads_or(big) == 0;
     if (ok) {
-        for (int i = tid; i < n * mp; i += nt) {
-            int j = i / mp, q = i - j * mp;
-            ptmT[i] = q < M ? ptm[q * n + j] : 0;
-        }
         // fillMinTimeArrDep: min over jobs of the head before / tail after machine q
         for (int q = tid; q < mp; q += nt) {
             int ha = 0, td = 0;
