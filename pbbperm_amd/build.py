@@ -44,6 +44,9 @@ def build(verbose: bool = False, jobs: int | None = None) -> str:
         for src in ("pbb_kernels", "pbb_pool", "pbb_ig", "pbb_bounds"):
             obj = os.path.join(BUILD, f"{src}_m{m}.o")
             units.append([HIPCC, *FLAGS, f"-DPBB_M={m}", "-c", os.path.join(CSRC, src + ".hip"), "-o", obj])
+        # the engine's kernels of the wide Johnson table, a code object of their own
+        units.append([HIPCC, *FLAGS, f"-DPBB_M={m}", "-DPBB_TAB=TAB_WIDE", "-c", os.path.join(CSRC, "pbb_kernels.hip"),
+                      "-o", os.path.join(BUILD, f"pbb_kernels_wide_m{m}.o")])
     for src in ("pbb_dispatch.cpp", "pbb_host.cpp", "pbb_io.cpp", "pbb_pool.cpp", "pbb_checkpoint.cpp", "pbb_cpu.cpp"):
         obj = os.path.join(BUILD, src.replace(".cpp", ".o"))
         units.append([HIPCC, *FLAGS, "-x", "hip", "-c", os.path.join(CSRC, src), "-o", obj])

@@ -28,23 +28,26 @@ namespace pbb {
     default: return hipErrorInvalidValue; \
     }
 
+// the Johnson table's form picks a kernel where there is one
+static bool wide(const KArgs &a) { return a.bound_mode != 0 && a.refine == 1 && !a.I.jpacked; }
+
 hipError_t launch_explore(const KArgs &a, int blocks, hipStream_t s)
 {
-#define C_(M) launch_explore_m<M>(a, blocks, s)
+#define C_(M) (wide(a) ? launch_explore_m<M, TAB_WIDE>(a, blocks, s) : launch_explore_m<M, TAB_PACKED>(a, blocks, s))
     PBB_FOR_M(C_, a.I.m)
 #undef C_
 }
 
 hipError_t launch_team(const KArgs &a, hipStream_t s)
 {
-#define C_(M) launch_team_m<M>(a, s)
+#define C_(M) (wide(a) ? launch_team_m<M, TAB_WIDE>(a, s) : launch_team_m<M, TAB_PACKED>(a, s))
     PBB_FOR_M(C_, a.I.m)
 #undef C_
 }
 
 hipError_t explore_occupancy(const KArgs &a, int *blocks_per_cu)
 {
-#define C_(M) occupancy_m<M>(a, blocks_per_cu)
+#define C_(M) (wide(a) ? occupancy_m<M, TAB_WIDE>(a, blocks_per_cu) : occupancy_m<M, TAB_PACKED>(a, blocks_per_cu))
     PBB_FOR_M(C_, a.I.m)
 #undef C_
 }

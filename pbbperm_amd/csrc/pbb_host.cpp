@@ -356,14 +356,17 @@ static int capacity(pbb_engine *e, int packed, int jt, int *explorers)
 
 static bool with_lb2(const pbb_engine *e) { return e->cfg.bound_mode != 0 && e->cfg.refine == 1; }
 
-// The engine's explorers: what is resident of either form, so that a retargeted
-// engine keeps them.
+// The engine's explorers: what is resident with the packed table's bytes, and
+// without a table where the instance is of the wide form (no fewer).  The query loads
+// the form's kernels, a tenth of a millisecond the first time, so the packed form asks
+// for its own only; a retargeted engine, which starts from explorer 0 alone, launches as many
+// of the other form as plan_form finds.
 static int engine_explorers(pbb_engine *e)
 {
     int cap = 0, wide = 0;
     const bool lb2 = with_lb2(e);
     if (const int rc = capacity(e, 1, lb2 ? explore_jtab_bytes(e->D.I) : 0, &cap)) return rc;
-    if (lb2) {
+    if (lb2 && !e->D.I.jpacked) {
         if (const int rc = capacity(e, 0, 0, &wide)) return rc;
         cap = std::min(cap, wide);
     }

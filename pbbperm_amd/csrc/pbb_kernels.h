@@ -354,10 +354,10 @@ __device__ __host__ inline size_t pool_lds_bytes(int nmax, int M, int pmax, int 
     return lds_table_bytes(M, jt_lds) + (size_t)W * lds_wave_bytes(nmax, M, pmax > 0);
 }
 
-// per-M kernels (pbb_kernels.hip, one translation unit per M)
-template <int M> hipError_t launch_explore_m(const KArgs &a, int blocks, hipStream_t s);
-template <int M> hipError_t launch_team_m(const KArgs &a, hipStream_t s);
-template <int M> hipError_t occupancy_m(const KArgs &a, int *blocks_per_cu);
+// per-M kernels (pbb_kernels.hip, one translation unit per M and table form)
+template <int M, int TAB> hipError_t launch_explore_m(const KArgs &a, int blocks, hipStream_t s);
+template <int M, int TAB> hipError_t launch_team_m(const KArgs &a, hipStream_t s);
+template <int M, int TAB> hipError_t occupancy_m(const KArgs &a, int *blocks_per_cu);
 template <int M> hipError_t launch_root_m(const KArgs &a, const RootPerm &root_perm, hipStream_t s);
 
 // batched bounds (pbb_bounds.hip, one translation unit per M)

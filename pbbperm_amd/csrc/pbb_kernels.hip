@@ -20,7 +20,9 @@
 //   k_bound_root<M> LB1 root bounding, ivm_bound::boundRoot (ivm_bound.cpp:273-330).
 //
 // Translation units: this file is compiled once per machine count M
-// (-DPBB_M=<m>) so the 19 instantiations build in parallel.
+// (-DPBB_M=<m>) so the 19 instantiations build in parallel, and once more for the
+// kernels of the wide Johnson table (-DPBB_TAB=TAB_WIDE): a process that meets no
+// large processing times then never loads them.
 #include "pbb_explorer.h"
 
 namespace pbb {
@@ -169,20 +171,24 @@ __global__ __launch_bounds__(64) void k_bound_root(KArgs a, RootPerm root_perm)
 }
 
 // ---------------------------------------------------------- host launchers
-// the kernel of a bounding variant and, with LB2, of a table form
-template <int M>
+// the kernel of a bounding variant (the wide form is LB2's)
+template <int M, int TAB>
 static const void *explore_kernel(const KArgs &a)
 {
-    if (a.bound_mode == 0) return (const void *)k_explore<M, 0, TAB_PACKED>;
-    if (a.refine != 1) return (const void *)k_explore<M, 1, TAB_PACKED>;
-    return a.I.jpacked ? (const void *)k_explore<M, 2, TAB_PACKED> : (const void *)k_explore<M, 2, TAB_WIDE>;
+    if constexpr (TAB == TAB_WIDE) return (const void *)k_explore<M, 2, TAB>;
+    else {
+        if (a.bound_mode == 0) return (const void *)k_explore<M, 0, TAB>;
+        return a.refine == 1 ? (const void *)k_explore<M, 2, TAB> : (const void *)k_explore<M, 1, TAB>;
+    }
 }
-template <int M>
+template <int M, int TAB>
 static const void *team_kernel(const KArgs &a)
 {
-    if (a.bound_mode == 0) return (const void *)k_team<M, 0, TAB_PACKED>;
-    if (a.refine != 1) return (const void *)k_team<M, 1, TAB_PACKED>;
-    return a.I.jpacked ? (const void *)k_team<M, 2, TAB_PACKED> : (const void *)k_team<M, 2, TAB_WIDE>;
+    if constexpr (TAB == TAB_WIDE) return (const void *)k_team<M, 2, TAB>;
+    else {
+        if (a.bound_mode == 0) return (const void *)k_team<M, 0, TAB>;
+        return a.refine == 1 ? (const void *)k_team<M, 2, TAB> : (const void *)k_team<M, 1, TAB>;
+    }
 }
 
 static hipError_t launch_kernel(const void *k, int blocks, int threads, size_t lds, const KArgs &a, hipStream_t s)
@@ -192,23 +198,23 @@ static hipError_t launch_kernel(const void *k, int blocks, int threads, size_t l
     return hipLaunchKernel(k, dim3(blocks), dim3(threads), args, lds, s);
 }
 
-template <int M>
+template <int M, int TAB>
 hipError_t launch_explore_m(const KArgs &a, int blocks, hipStream_t s)
 {
     const bool lb2 = a.bound_mode != 0 && a.refine == 1;
     const size_t lds = explore_lds_bytes(a.I, lb2, lb2 ? a.jt_lds : 0);
-    return launch_kernel(explore_kernel<M>(a), blocks, 64 * PBB_EXPLORE_WAVES, lds, a, s);
+    return launch_kernel(explore_kernel<M, TAB>(a), blocks, 64 * PBB_EXPLORE_WAVES, lds, a, s);
 }
 
-template <int M>
+template <int M, int TAB>
 hipError_t launch_team_m(const KArgs &a, hipStream_t s)
 {
     const bool lb2 = a.bound_mode != 0 && a.refine == 1;
     const size_t lds = team_lds_bytes(a.I, lb2, lb2 ? a.jt_lds : 0, a.E);
-    return launch_kernel(team_kernel<M>(a), 1, 64 * a.E, lds, a, s);
+    return launch_kernel(team_kernel<M, TAB>(a), 1, 64 * a.E, lds, a, s);
 }
 
-template <int M>
+template <int M, int TAB>
 hipError_t occupancy_m(const KArgs &a, int *blocks_per_cu)
 {
     const bool lb2 = a.bound_mode != 0 && a.refine == 1;
@@ -218,7 +224,7 @@ hipError_t occupancy_m(const KArgs &a, int *blocks_per_cu)
         return hipSuccess;
     }
     const size_t q = residency_lds_bytes(lds);
-    const void *k = explore_kernel<M>(a);
+    const void *k = explore_kernel<M, TAB>(a);
     if (const hipError_t err = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)q)) return err;
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, k, 64 * PBB_EXPLORE_WAVES, q);
 }
@@ -235,10 +241,13 @@ hipError_t launch_root_m(const KArgs &a, const RootPerm &root_perm, hipStream_t 
 }
 
 #ifdef PBB_M
-template hipError_t launch_explore_m<PBB_M>(const KArgs &, int, hipStream_t);
-template hipError_t launch_team_m<PBB_M>(const KArgs &, hipStream_t);
-template hipError_t occupancy_m<PBB_M>(const KArgs &, int *);
+#ifndef PBB_TAB
+#define PBB_TAB TAB_PACKED
 template hipError_t launch_root_m<PBB_M>(const KArgs &, const RootPerm &, hipStream_t);
+#endif
+template hipError_t launch_explore_m<PBB_M, PBB_TAB>(const KArgs &, int, hipStream_t);
+template hipError_t launch_team_m<PBB_M, PBB_TAB>(const KArgs &, hipStream_t);
+template hipError_t occupancy_m<PBB_M, PBB_TAB>(const KArgs &, int *);
 #endif
 
 }  // namespace pbb

@@ -17,6 +17,9 @@ def test_lb2_explorers_at_the_lds_limit(n, m):
     most = 3 * 4 * cus
     cfg = P.default_config(nb_ivms=1 << 16, bound_mode=2, branching=3, refine=1, johnson_pairs=0, early_stop_johnson=0)
     assert P.explorers_for(n, m, cfg) >= most
+    # whatever the times: 12-fold they are past the packed table's limit
+    with P.GpuBB(P.synth(n + m, n, m) * 12, cfg, ub=0) as eng:
+        assert eng.stats().explorers == P.explorers_for(n, m, cfg)
     # so many intervals are taken, the last explorers among their ids
     with P.GpuBB(P.synth(n + m, n, m), cfg, ub=0) as eng:
         E = eng.stats().explorers
