@@ -1,7 +1,8 @@
 """Build recipe for the in-tree gfx950 engine library ``libpbb_engine.so``.
 
-The kernel sources (one-instance engine, multi-instance pool) are compiled
-once per machine count M (2..20, -DPBB_M=M) in parallel, then linked with
+The kernel sources (one-instance engine, multi-instance pool, bounds, iterated
+greedy) are compiled once per machine count M (2..20, -DPBB_M=M) in parallel,
+two of them once more for a second form of their kernels, then linked with
 the runtime-M dispatch and the host C ABI.
 The library is built in-tree so it travels with the repository snapshot.
 """
@@ -44,9 +45,11 @@ def build(verbose: bool = False, jobs: int | None = None) -> str:
         for src in ("pbb_kernels", "pbb_pool", "pbb_ig", "pbb_bounds"):
             obj = os.path.join(BUILD, f"{src}_m{m}.o")
             units.append([HIPCC, *FLAGS, f"-DPBB_M={m}", "-c", os.path.join(CSRC, src + ".hip"), "-o", obj])
-        # the engine's kernels of the wide Johnson table, a code object of their own
-        units.append([HIPCC, *FLAGS, f"-DPBB_M={m}", "-DPBB_TAB=TAB_WIDE", "-c", os.path.join(CSRC, "pbb_kernels.hip"),
-                      "-o", os.path.join(BUILD, f"pbb_kernels_wide_m{m}.o")])
+        # kernels of the wide Johnson table and of small batches of bounds: code objects of
+        # their own, loaded by the processes that use them
+        for src, tag, flag in (("pbb_kernels", "wide", "-DPBB_TAB=TAB_WIDE"), ("pbb_bounds", "small", "-DPBB_SMALL=true")):
+            obj = os.path.join(BUILD, f"{src}_{tag}_m{m}.o")
+            units.append([HIPCC, *FLAGS, f"-DPBB_M={m}", flag, "-c", os.path.join(CSRC, src + ".hip"), "-o", obj])
     for src in ("pbb_dispatch.cpp", "pbb_host.cpp", "pbb_io.cpp", "pbb_pool.cpp", "pbb_checkpoint.cpp", "pbb_cpu.cpp"):
         obj = os.path.join(BUILD, src.replace(".cpp", ".o"))
         units.append([HIPCC, *FLAGS, "-x", "hip", "-c", os.path.join(CSRC, src), "-o", obj])

@@ -8,7 +8,7 @@
 //   1. chains: one lane per schedule and side, its completion times in
 //      registers, so that a job costs 3 instructions per machine for 64 chains
 //      (a wavefront per schedule, lane = machine, pays a prefix scan of 25
-//      dependent instructions per job for one; small batches take that, B_SMALL).
+//      dependent instructions per job for one; small batches take that, BOUNDS_SMALL).
 //      Lengths run over 0..n and a wavefront runs as long as its longest chain,
 //      so the tile's 2T chains are first sorted by length (a counting sort of 64
 //      bins);
@@ -21,7 +21,8 @@
 // What bounds it: the children are LDS reads (two 8-byte operands and a time per
 // child and machine) and VALU in about equal parts.
 //
-// Translation units: compiled once per machine count M (-DPBB_M=<m>).
+// Translation units: compiled once per machine count M (-DPBB_M=<m>), and once more
+// for the small batches' kernels (-DPBB_SMALL=true), a code object of their own.
 #include "pbb_device.h"
 #include "pbb_kernels.h"
 
@@ -33,16 +34,8 @@ enum { B_CHILDREN = 0, B_LB1 = 1, B_LB2 = 2, B_MAKESPAN = 3 };
 // that read one position of different schedules on distinct banks
 #define BJ_STRIDE 68
 #define B_THREADS 256
-// Batches of up to B_SMALL_COUNT schedules go in tiles of B_SMALL, a schedule per
-// wavefront: what bounds them is the time of one chain, and a lane that takes
-// every machine of every job is slower for one schedule than a wavefront whose lanes
-// are the machines.  A kernel of its own: beside the lane-wise chains it costs LB2 a
-// third (50x10, 100 k schedules 102 -> 134 us).  One call, tiles of 16 / this: 256
-// schedules at 50x20, children 41.8 / 29.0 us, LB2 53.7 / 36.3; at 20x10 28.7 / 25.0
-// and 28.3 / 24.6; 4096 at 50x20, children 42.9 / 32.6, LB2 56.0 / 52.1, 8192 43.3 /
-// 40.5 and 61.9 / 75.5.
+// schedules of a small batch's tile (BOUNDS_SMALL): one a wavefront
 #define B_SMALL (B_THREADS / 64)
-#define B_SMALL_COUNT 4096
 // most schedules per tile
 __host__ __device__ constexpr int b_tile(int which) { return which == B_LB2 ? 32 : 128; }
 
@@ -407,46 +400,47 @@ __global__ __launch_bounds__(B_THREADS) void k_bounds(DevInst I, int count, int 
 
 // Tile size: up to 128 schedules, as many as leave room for three workgroups
 // per CU beside the tables (two with a Johnson table); a smaller batch is spread
-// over the CUs in smaller tiles, 16 schedules at least, a small one in tiles of
-// B_SMALL.
-template <int M, int WHICH>
+// over the CUs in smaller tiles, 16 schedules at least.
+template <int M, int WHICH, bool SMALL>
 static hipError_t launch(const DevInst &I, int count, const int *perms, const int *l1, const int *l2, int arg, int *o1,
                          int *o2, hipStream_t s)
 {
     const size_t tab = bound_table_bytes<M>(I, WHICH == B_LB2 && I.jpacked);
     const size_t room = 160 * 1024 / (WHICH == B_LB2 ? 2 : 3) - 2048;
     const auto tiles = [&](int T) { return (int)(((long long)count + T - 1) / T); };
-    const bool small = count <= B_SMALL_COUNT;
-    int T = small ? B_SMALL : b_tile(WHICH);
+    int T = SMALL ? B_SMALL : b_tile(WHICH);
     while (T > 16 && tab + bound_tile_bytes<M>(T) > room) T -= 16;
     while (T > 16 && tiles(T) < 512) T -= 16;
     const size_t lds = tab + bound_tile_bytes<M>(T);
-    const auto kernel = small ? k_bounds<M, WHICH, true> : k_bounds<M, WHICH, false>;
     if (lds > 64 * 1024)
-        if (const hipError_t err = hipFuncSetAttribute((const void *)kernel,
+        if (const hipError_t err = hipFuncSetAttribute((const void *)k_bounds<M, WHICH, SMALL>,
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
             return err;
     const int resident = 256 * (int)(160 * 1024 / lds < 8 ? 160 * 1024 / lds : 8);
     const int grid = tiles(T) < resident ? tiles(T) : resident;
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(B_THREADS), lds, s, I, count, T, perms, l1, l2, arg, o1, o2);
+    hipLaunchKernelGGL((k_bounds<M, WHICH, SMALL>), dim3(grid), dim3(B_THREADS), lds, s, I, count, T, perms, l1, l2,
+                       arg, o1, o2);
     return hipGetLastError();
 }
 
-template <int M>
+template <int M, bool SMALL>
 hipError_t launch_bounds_m(int which, const DevInst &I, int count, const int *perms, const int *l1, const int *l2,
                            int arg, int *o1, int *o2, hipStream_t s)
 {
     switch (which) {
-    case B_CHILDREN: return launch<M, B_CHILDREN>(I, count, perms, l1, l2, arg, o1, o2, s);
-    case B_LB1: return launch<M, B_LB1>(I, count, perms, l1, l2, arg, o1, o2, s);
-    case B_LB2: return launch<M, B_LB2>(I, count, perms, l1, l2, arg, o1, o2, s);
-    default: return launch<M, B_MAKESPAN>(I, count, perms, l1, l2, arg, o1, o2, s);
+    case B_CHILDREN: return launch<M, B_CHILDREN, SMALL>(I, count, perms, l1, l2, arg, o1, o2, s);
+    case B_LB1: return launch<M, B_LB1, SMALL>(I, count, perms, l1, l2, arg, o1, o2, s);
+    case B_LB2: return launch<M, B_LB2, SMALL>(I, count, perms, l1, l2, arg, o1, o2, s);
+    default: return launch<M, B_MAKESPAN, SMALL>(I, count, perms, l1, l2, arg, o1, o2, s);
     }
 }
 
 #ifdef PBB_M
-template hipError_t launch_bounds_m<PBB_M>(int, const DevInst &, int, const int *, const int *, const int *, int, int *,
-                                          int *, hipStream_t);
+#ifndef PBB_SMALL
+#define PBB_SMALL false
+#endif
+template hipError_t launch_bounds_m<PBB_M, PBB_SMALL>(int, const DevInst &, int, const int *, const int *, const int *,
+                                                      int, int *, int *, hipStream_t);
 #endif
 
 }  // namespace pbb

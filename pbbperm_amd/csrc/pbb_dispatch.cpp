@@ -62,7 +62,9 @@ hipError_t launch_root(const KArgs &a, const RootPerm &root_perm, hipStream_t s)
 hipError_t launch_bounds(int which, const DevInst &I, int count, const int *perms, const int *l1,
                          const int *l2, int arg, int *o1, int *o2, hipStream_t s)
 {
-#define C_(M) launch_bounds_m<M>(which, I, count, perms, l1, l2, arg, o1, o2, s)
+#define C_(M)                                                                               \
+    (count <= BOUNDS_SMALL ? launch_bounds_m<M, true>(which, I, count, perms, l1, l2, arg, o1, o2, s) \
+                           : launch_bounds_m<M, false>(which, I, count, perms, l1, l2, arg, o1, o2, s))
     PBB_FOR_M(C_, I.m)
 #undef C_
 }

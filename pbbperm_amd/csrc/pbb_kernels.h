@@ -360,8 +360,17 @@ template <int M, int TAB> hipError_t launch_team_m(const KArgs &a, hipStream_t s
 template <int M, int TAB> hipError_t occupancy_m(const KArgs &a, int *blocks_per_cu);
 template <int M> hipError_t launch_root_m(const KArgs &a, const RootPerm &root_perm, hipStream_t s);
 
-// batched bounds (pbb_bounds.hip, one translation unit per M)
-template <int M>
+// batched bounds (pbb_bounds.hip, one translation unit per M and batch size).
+// Batches of up to BOUNDS_SMALL schedules go a schedule per wavefront, in tiles of
+// four: what bounds them is the time of one chain, and a lane that takes every
+// machine of every job is slower for one schedule than a wavefront whose lanes are
+// the machines.  A kernel of its own: beside the lane-wise chains it costs LB2 a
+// third (50x10, 100 k schedules 102 -> 134 us).  One call, tiles of 16 / this: 256
+// schedules at 50x20, children 41.8 / 29.0 us, LB2 53.7 / 36.3; at 20x10 28.7 / 25.0
+// and 28.3 / 24.6; 4096 at 50x20, children 42.9 / 32.6, LB2 56.0 / 52.1, 8192 43.3 /
+// 40.5 and 61.9 / 75.5.
+#define BOUNDS_SMALL 4096
+template <int M, bool SMALL>
 hipError_t launch_bounds_m(int which, const DevInst &I, int count, const int *perms, const int *l1,
                            const int *l2, int arg, int *o1, int *o2, hipStream_t s);
 
