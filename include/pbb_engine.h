@@ -359,7 +359,7 @@ int pbb_pool_destroy(pbb_pool *p);
 int pbb_pool_info(pbb_pool *p, int *explorers, int *groups, int *lds_bytes);
 
 /* Change the per-instance explorer cap and the steal margin of an idle pool
- * (the cap stays within the idle-ring capacity chosen at creation). */
+ * (the cap stays within the member capacity chosen at creation). */
 int pbb_pool_retune(pbb_pool *p, int explorers_per_instance, int steal_margin);
 
 /* Depth histograms of the last pbb_pool_solve batch, instance i at

@@ -29,7 +29,10 @@ namespace pbb {
 
 // ------------------------------------------------------------ kernels
 // Minimum resident waves per SIMD the compiler must allow (register
-// budget): 4 for the LB1 and LB1' explorers (128 VGPRs), 3 with LB2.
+// budget): 4 for the LB1 and LB1' explorers (128 VGPRs), 3 with LB2, where the
+// 20-machine one spills 21 registers for it (187 VGPRs without the bound, none
+// spilled, 2048 explorers).  3 / 2 waves at 18x20: 2.5 M nodes 6.7 / 8.4 ms, 3065
+// nodes 1.74 / 1.54; 30x20 3.59 / 3.55.
 #ifndef PBB_EXPLORE_MIN_WAVES
 #define PBB_EXPLORE_MIN_WAVES 4
 #endif
@@ -140,11 +143,11 @@ __global__ __launch_bounds__(64 * PBB_EXPLORE_WAVES, REF == 2 ? 3 : PBB_EXPLORE_
 }
 
 // The team launch: explorers 0..a.E-1 as the wavefronts of one workgroup
-// (up to team_waves_max(REF)), sharing work with workgroup-scope ordering only.
-// A fresh search starts here: a small tree (a few thousand nodes) is solved
-// by the team alone, without the cross-XCD writebacks and invalidates that
-// every hand-over costs in a device-wide launch; a larger one stops at the
-// node budget and the device-wide launch resumes from the saved intervals.
+// (up to team_waves_max(REF)), whose messages, mask word and counters stay in one
+// CU's L1 and XCD's L2.  A fresh search starts here: a small tree (a few thousand
+// nodes) is solved by the team alone, without a device-wide launch's fan-out; a
+// larger one stops at the node budget and the device-wide launch resumes from the
+// saved intervals.
 template <int M, int REF, int TAB>
 __global__ __launch_bounds__(64 * team_waves_max(REF)) void k_team(KArgs a)
 {

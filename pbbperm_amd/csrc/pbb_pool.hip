@@ -443,8 +443,10 @@ __device__ __forceinline__ void pool_ig_helper(const Lds &lds, int n, int e, con
 
 // ----------------------------------------------------------------- kernel
 // Minimum resident waves per SIMD the compiler must allow (register
-// budget): 3 up to 10 machines (168 VGPRs: the 10-machine LB2 pool would
-// otherwise take 169-176 and drop to 2 waves per SIMD), free above.
+// budget): 3 up to 10 machines (168 VGPRs; the 10-machine LB2 pool spills 34
+// for it), 2 above (256; 19 spilled at 20 machines).  512-instance batch at 3 / 2
+// waves 52 / 60 ms, burst of 256 requests in the 20-machine pool at 2 / without the
+// bound 44 / 62 ms.
 #ifndef PBB_POOL_MIN_WAVES
 #define PBB_POOL_MIN_WAVES(M) ((M) <= 10 ? 3 : 2)
 #endif
