@@ -61,10 +61,10 @@ PEAK_HBM_GBS = 8000.0
 # HBM bytes per decomposed node of k_explore on this workload, from two
 # rocprofv3 --pmc passes (FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0, factors from a
 # plain 256 MiB device copy): profiles/k_explore_50x20_lb1_pmc.md
-HBM_BYTES_PER_NODE = 0.80
+HBM_BYTES_PER_NODE = 0.82
 # HBM bytes of one k_pool<10,2> launch of the 512-instance batch, from the
 # same two counters and factors: profiles/k_pool_batch512_lb2_pmc.md
-BATCH_HBM_BYTES = 0.93e9
+BATCH_HBM_BYTES = 0.70e9
 # The serving stream of the default run: requests, Poisson rate and the
 # per-request time budget after admission.  Every path's replay ends at the
 # arrival span + 2 budgets + 15 s; what is not served by then counts late.
@@ -655,7 +655,8 @@ def leg_nodes(P, args):
                    "n": n, "m": m, "seed": seed, "explorers": st1.explorers,
                    "explorers_stated": "16384-65536",
                    "explorers_note": "one explorer per 64-lane wavefront; 4096 is the resident maximum of "
-                                     "k_explore<20,0> on gfx950 (128 VGPRs: 4 waves per SIMD x 4 SIMDs x 256 CUs), "
+                                     "k_explore<20,0> on gfx950 (95 VGPRs, launch-bounded to 4 waves per SIMD x 4 SIMDs x "
+                                     "256 CUs; 4 workgroups of 35.4 KB LDS per CU), "
                                      "and a persistent launch needs every explorer resident",
                    "ub": int(ub), "best": int(best), "node_budget_per_step": args.node_budget},
         "roofline": {"bound": "valu", "achieved": achieved, "peak": PEAK_INT32_TOPS, "unit": "TOP/s (int32)",
