@@ -359,8 +359,8 @@ static bool with_lb2(const pbb_engine *e) { return e->cfg.bound_mode != 0 && e->
 // The engine's explorers: what is resident with the packed table's bytes, and
 // without a table where the instance is of the wide form (no fewer).  The query loads
 // the form's kernels, a tenth of a millisecond the first time, so the packed form asks
-// for its own only; a retargeted engine, which starts from explorer 0 alone, launches as many
-// of the other form as plan_form finds.
+// for its own only; a retargeted engine, which starts from explorer 0 alone, launches
+// as many of the other form as plan_form finds.
 static int engine_explorers(pbb_engine *e)
 {
     int cap = 0, wide = 0;
@@ -676,10 +676,11 @@ static int launch_once(pbb_engine *e, bool team, uint64_t node_budget, uint64_t 
 // explorers would search more of what the next one prunes (20x5 from NEH, the share /
 // this: LB1 1.08 / 0.8, LB1' 1.3 / 0.87, LB2 1.9 / 1.1; with LB2 half of it brings no
 // more, and 256 instances of the batch one after the other take 0.376 s at the share,
-// 0.386 at a quarter, 0.408 at half, 0.458 at all).  An engine of no more explorers than the team has nothing to gain from the
-// second launch, and a run for fewer nodes than team_nodes stays with the team,
-// which stops within a few hundred nodes of its budget; thousands of explorers, each
-// of which looks every 64 nodes, overrun it by as many.
+// 0.386 at a quarter, 0.408 at half, 0.458 at all).  An engine of no more explorers
+// than the team has nothing to gain from the second launch, and a run for fewer
+// nodes than team_nodes stays with the team, which stops within a few hundred nodes of
+// its budget; thousands of explorers, each of which looks every 64 nodes, overrun it by
+// as many.
 struct TeamBudget {
     uint64_t quiet, moved;
 };

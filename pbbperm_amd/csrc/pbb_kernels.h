@@ -48,9 +48,9 @@ __device__ __forceinline__ unsigned mail_tag(unsigned w) { return w >> 26; }
 __device__ __forceinline__ int mail_path_cell(int i, int p, int j) { return i == p ? j : (i > p ? 0 : -1); }
 
 // A busy explorer of a device-wide launch reads a word of the idle mask every
-// PBB_POLL_EVERY decomposed nodes, whether or not explorers wait in it; with Johnson LB2, whose node takes several times an LB1 node's
-// time, it reads the next word at the next node while it sees explorers
-// waiting.  A poll costs a busy device, a long interval between them a thin
+// PBB_POLL_EVERY decomposed nodes, whether or not explorers wait in it; with
+// Johnson LB2, whose node takes several times an LB1 node's time, it reads the
+// next word at the next node while it sees explorers waiting.  A poll costs a busy device, a long interval between them a thin
 // tree, whose fan-out takes that long per doubling.  Every 16 / 8 / 4 / 1 nodes:
 // 50x20 LB1 (49.7 M nodes) 29.3 / 29.0 / 30.5 / 45.8 ms, 20x20 LB1 (0.83 M) 4.3 /
 // 3.5 / 3.7 / 4.6 ms; again while explorers wait, 20x20 4.1-4.5 ms.  30x20 LB2
